@@ -1,0 +1,131 @@
+"""GPU parity of the chunk-form Gated DeltaNet backward (triune_hip_gdn_bwd_chunked: 16-bit I/O, beta
+none or per head) against the fp64 oracle, at the edges of its 64-token chunks and 16-token tiles,
+through chunks too steep for the factored pair sums, and against the token-serial kernels.
+
+Tolerance: one ULP of the gradient's type at the oracle's value (its own rounding, 1/2 ULP, with the
+other half for values near a rounding boundary) plus 4e-5 of the largest gradient: the kernels work in
+fp32, and a pair factor e^(G - m) e^(m - G') with exponents up to 64 carries up to
+2 * 64 * 2^-24 * (1 + log2 e) = 2e-5 of relative error.
+"""
+
+import numpy as np
+import pytest
+import torch
+import torch.nn.functional as F
+
+import triune_amd.fast_gla as FG
+from oracle import oracle as O
+from triune_amd import _lib, fast_chunk_gated_deltanet
+
+pytestmark = pytest.mark.gpu
+
+
+def _ulp(r, dtype):
+    bits, emin = (7, -126) if dtype == torch.bfloat16 else (10, -14)
+    return torch.exp2(torch.floor(torch.log2(r.abs().clamp_min(2.0**emin))) - bits)
+
+
+def _check(got, ref, dtype, names):
+    for name, x, r in zip(names, got, ref):
+        if r is None:
+            assert x is None, name
+            continue
+        r = torch.as_tensor(np.asarray(r, dtype=np.float64))
+        assert x.dtype == dtype and tuple(x.shape) == tuple(r.shape), name
+        err = (x.detach().double().cpu() - r).abs()
+        slack = 4e-5 * max(1.0, float(r.abs().max()))
+        assert bool((err <= _ulp(r, dtype) + slack).all()), (name, float((err - _ulp(r, dtype)).max()), slack)
+
+
+def _inputs(B, T, H, D, gate, beta, dtype, seed, steep=None):
+    gen = torch.Generator().manual_seed(seed)
+    q, k = (F.normalize(torch.randn(B, T, H, D, generator=gen), dim=-1).to(dtype) for _ in range(2))
+    v, do = (torch.randn(B, T, H, D, generator=gen).to(dtype) for _ in range(2))
+    g = F.logsigmoid(torch.randn(*((B, T, H) if gate == "head" else (B, T, H, D)), generator=gen))
+    g = g * (1.0 if gate == "key" else 0.2)
+    g[:, 2::9] = 0.0  # on the clamp's edge: the gradient passes
+    g[:, 1::7] = 0.05  # clamped: no gradient
+    if steep is not None:
+        g[:, : T // 2] = g[:, : T // 2] * steep  # some chunks steep, some not
+        g[:, 5::31] = -float("inf")  # resets
+    b = torch.sigmoid(torch.randn(B, T, H, generator=gen)).to(dtype) if beta else None
+    ds = torch.randn(B, H, D, D, generator=gen)
+    return q, k, v, g.to(dtype), b, do, ds
+
+
+def _run(dev, q, k, v, g, b, do, ds):
+    kind = _lib.BETA_NONE if b is None else _lib.BETA_HEAD
+    args = [None if x is None else x.to(dev) for x in (q, k, v, g, b)]
+    got = FG._gdn_bwd(*args, None, kind, None if do is None else do.to(dev), None if ds is None else ds.to(dev))
+    torch.cuda.synchronize()
+    gf = g.unsqueeze(-1).expand(*g.shape, q.shape[-1]) if g.dim() == 3 else g
+    ref = list(O.gdn_bwd(q, k, v, gf, b, None, do, ds))
+    if g.dim() == 3:
+        ref[3] = ref[3].sum(-1)
+    return got, ref
+
+
+NAMES = ("dq", "dk", "dv", "dg", "dbeta")
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("T", [1, 15, 16, 63, 64, 65, 200])
+@pytest.mark.parametrize("gate,beta", [("key", False), ("head", True)])
+def test_chunk_edges(dev, D, T, gate, beta):
+    x = _inputs(2, T, 3, D, gate, beta, torch.bfloat16, seed=T + D)
+    got, ref = _run(dev, *x)
+    _check(got, ref, torch.bfloat16, NAMES)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("gate,beta", [("key", True), ("head", False)])
+def test_many_chunks_fp16(dev, D, gate, beta):
+    """Longer than the scan's prefetch, B * H past one XCD group, no final-state gradient."""
+    q, k, v, g, b, do, _ = _inputs(3, 700, 3, D, gate, beta, torch.float16, seed=D)
+    got, ref = _run(dev, q, k, v, g, b, do, None)
+    _check(got, ref, torch.float16, NAMES)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("gate,beta", [("key", True), ("head", True)])
+def test_steep_and_reset_gates(dev, D, gate, beta):
+    """Chunks that decay by more than 128 nats, with -inf gates that reset the state, beside ordinary
+    ones."""
+    x = _inputs(1, 230, 2, D, gate, beta, torch.bfloat16, seed=D + 9, steep=12.0)
+    got, ref = _run(dev, *x)
+    _check(got, ref, torch.bfloat16, NAMES)
+
+
+def test_only_the_final_state(dev):
+    """No gradient of o: only the final state's."""
+    q, k, v, g, b, _, ds = _inputs(2, 100, 2, 64, "key", True, torch.bfloat16, seed=4)
+    got, ref = _run(dev, q, k, v, g, b, None, ds)
+    _check(got, ref, torch.bfloat16, NAMES)
+
+
+@pytest.mark.parametrize("gate", ["key", "head"])
+def test_operator_views_and_padding(dev, gate, monkeypatch):
+    """The operator's autograd with strided q, k, v views, a non-contiguous beta and gate, and head
+    dims 48 (padded to 64): the chunk form and the token-serial kernels give the same gradients to
+    within a bf16 rounding of each."""
+    gen = torch.Generator().manual_seed(8)
+    B, T, H, D = 2, 150, 3, 48
+    qkv = torch.randn(B, T, 3, H, D, generator=gen).to(dev)
+    qkv[:, :, :2] = F.normalize(qkv[:, :, :2], dim=-1)
+    qkv = qkv.bfloat16().requires_grad_()
+    gw = (B, H, T) if gate == "head" else (B, H, T, D)
+    g = (F.logsigmoid(torch.randn(*gw, generator=gen)) / 4).bfloat16().to(dev).requires_grad_()
+    be = torch.sigmoid(torch.randn(B, H, T, generator=gen)).bfloat16().to(dev).requires_grad_()
+    do = torch.randn(B, T, H, D, generator=gen).bfloat16().to(dev)
+    res = []
+    for on in (True, False):
+        monkeypatch.setattr(FG, "_chunked_gdn_bwd_enabled", on)
+        o, _ = fast_chunk_gated_deltanet(qkv[:, :, 0], qkv[:, :, 1], qkv[:, :, 2], g.transpose(1, 2),
+                                         beta=be.transpose(1, 2))
+        res.append(torch.autograd.grad(o, (qkv, g, be), do))
+    torch.cuda.synchronize()
+    for x, y in zip(*res):
+        x, y = x.double().cpu(), y.double().cpu()
+        # the token-serial path rounds each key dim's part of a head gate's gradient: D roundings
+        slack = 4e-5 + (D**0.5 * 2.0**-9 if gate == "head" and x.dim() == 3 else 0.0)
+        assert bool(((x - y).abs() <= 2 * _ulp(y, torch.bfloat16) + slack * max(1.0, float(y.abs().max()))).all())

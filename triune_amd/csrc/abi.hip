@@ -1061,6 +1061,65 @@ int triune_hip_gdn_bwd(const void* q, const void* k, const void* v, const void* 
     return TRIUNE_OK;
 }
 
+// Chunk-form backward: per (b, h, chunk) the block-triangular tiles and three D x D matrices.
+static size_t gdn_bwd_chunked_bytes(int64_t B, int64_t T, int64_t H, int D) {
+    return (size_t)(B * H * ((T + 63) / 64)) * (3 * D * D + 20 * 256) * sizeof(float);
+}
+
+size_t triune_hip_gdn_bwd_chunked_workspace_size(int64_t B, int64_t T, int64_t H, int Dk, int Dv) {
+    if (B < 0 || T < 0 || H <= 0 || Dk != Dv || (Dk != 64 && Dk != 128)) return 0;
+    const size_t t = gdn_bwd_chunked_bytes(B, T, H, Dk);
+    return t > 0 ? t : 16;
+}
+
+int triune_hip_gdn_bwd_chunked(const void* q, const void* k, const void* v, const void* g, int io_dtype, int g_dtype,
+                               int g_head, const void* beta, int beta_dtype, int beta_kind, const int64_t* strides,
+                               const float* s0, const void* dout, const float* ds_final, void* dq, void* dk, void* dv,
+                               void* dg, void* dbeta, float* ds0, int64_t B, int64_t T, int64_t H, int Dk, int Dv,
+                               void* workspace, size_t workspace_bytes, void* stream) {
+    if (!q || !k || !v || !g || !strides || !dq || !dk || !dv || !dg) return TRIUNE_ERR_NULL;
+    if (beta_kind != TRIUNE_BETA_NONE && beta_kind != TRIUNE_BETA_HEAD) return TRIUNE_ERR_SHAPE;
+    if (beta_kind != TRIUNE_BETA_NONE && (!beta || !dbeta)) return TRIUNE_ERR_NULL;
+    if ((io_dtype != TRIUNE_DT_BF16 && io_dtype != TRIUNE_DT_F16) || !dtype_ok(g_dtype) ||
+        (beta_kind != TRIUNE_BETA_NONE && !dtype_ok(beta_dtype)))
+        return TRIUNE_ERR_DTYPE;
+    if (B < 0 || T < 0 || H <= 0 || Dk != Dv || (Dk != 64 && Dk != 128)) return TRIUNE_ERR_SHAPE;
+    const int D = Dk;
+    if (B * H * ((T + 63) / 64) > 0x7fffffff / 64) return TRIUNE_ERR_SHAPE;
+    if (reinterpret_cast<uintptr_t>(s0) % 16 || reinterpret_cast<uintptr_t>(ds_final) % 16 ||
+        reinterpret_cast<uintptr_t>(ds0) % 16 || reinterpret_cast<uintptr_t>(workspace) % 16)
+        return TRIUNE_ERR_LAYOUT;
+    if (B == 0) return TRIUNE_OK;
+    hipStream_t st = (hipStream_t)stream;
+    if (T == 0) {  // no tokens: the gradient of the initial state is that of the final state
+        if (!ds0) return TRIUNE_OK;
+        return launch_status(launch_gdn_slice_sum(ds_final, 1, 0, B * H * (int64_t)D * D, ds0, DT_F32, st));
+    }
+    if (!workspace || workspace_bytes < gdn_bwd_chunked_bytes(B, T, H, D)) return TRIUNE_ERR_WORKSPACE;
+    GdnChunkBwdParams p{};
+    GdnParams& a = p.f;
+    a.q = q; a.k = k; a.v = v; a.g = g; a.beta = beta;
+    a.io_dt = io_dtype; a.g_dt = g_dtype; a.beta_dt = beta_dtype; a.beta_kind = beta_kind;
+    a.q_sb = strides[0]; a.q_st = strides[1]; a.q_sh = strides[2];
+    a.k_sb = strides[3]; a.k_st = strides[4]; a.k_sh = strides[5];
+    a.v_sb = strides[6]; a.v_st = strides[7]; a.v_sh = strides[8];
+    a.g_sb = strides[9]; a.g_st = strides[10]; a.g_sh = strides[11];
+    a.b_sb = strides[12]; a.b_st = strides[13]; a.b_sh = strides[14];
+    a.s0 = s0;
+    a.B = B; a.T = T; a.H = H;
+    p.g_head = g_head != 0;
+    p.dout = dout; p.do_sb = strides[15]; p.do_st = strides[16]; p.do_sh = strides[17];
+    p.dsf = ds_final;
+    p.dq = dq; p.dk = dk; p.dv = dv; p.dg = dg; p.dbeta = dbeta; p.ds0 = ds0;
+    p.nc = (T + 63) / 64;
+    const int64_t n = B * H * p.nc;
+    p.ws_m = reinterpret_cast<float*>(workspace);
+    p.ws_s = p.ws_m + n * D * D;
+    p.ws_d = p.ws_s + n * D * D;
+    p.ws_t = p.ws_d + n * D * D;
+    return launch_status(launch_gdn_bwd_chunk(p, D, st));
+}
+
 }  // extern "C"
 
 namespace {

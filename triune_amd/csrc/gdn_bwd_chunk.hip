@@ -1,0 +1,874 @@
+// gdn_bwd_chunk.hip -- gradients of the Gated DeltaNet reference variant in chunk (WY/UT) form on the
+// fp32 matrix cores.
+//
+// Same arithmetic as gdn_bwd.hip (the reference differentiates fast_recurrent_gated_deltanet,
+// triune/kernels/fast_gla.py:781-836, with autograd).  Per 64-token chunk, with G the inclusive and
+// Gp the exclusive cumulative log-decay, w = beta k, S the state entering the chunk and D the
+// gradient reaching the state that leaves it:
+//   Q0 = q e^G,  B0 = k e^Gp,  Wc = w e^(G_C - G)                      (every factor at most 1)
+//   L[t][s] = k_t . e^(Gp_t - G_s) w_s (s < t),  A[t][s] = q_t . e^(G_t - G_s) w_s (s <= t)
+//   U = (I + L)^-1 (V - B0 S),   S_next = e^G_C S + Wc^T U,   dU = A^T dO + Wc D,   dR = (I + L)^-T dU
+//   D_prev = e^G_C D + Q0^T dO - B0^T dR,   dV = dR
+//   dA = tril(dO U^T),  dL = -tril(dR U^T, -1)
+//   dq = e^G (dO S^T) + [dA W],   dkB = -e^Gp (dR S^T) + [dL W],   dw = e^(G_C - G) (U D^T) + [dA^T Q + dL^T B]
+//   dk = beta dw + dkB,   dbeta = sum_d k dw
+//   dg_t = sum_{r >= t} (q dq - w dw)_r + sum_{r > t} (k dkB)_r + sum_c (D * S_next), 0 where g_t > 0
+// where [.] are the in-chunk pair sums with their factors e^(G_t - G_s) (or Gp_t), formed as
+// e^(G - m) e^(m - G) around the midpoint m = G_C / 2 of each key dim.
+//
+// S and D obey S_next = M S + N and D_prev = M^T D + K with M = e^G_C - Wc^T (I + L)^-1 B0,
+// N = Wc^T (I + L)^-1 V, K = Q0^T dO - B0^T (I + L)^-T A^T dO, all known per chunk.  Three launches:
+//   gdn_bwd_map_kernel   one workgroup per (b, h, chunk): L, (I + L)^-1's diagonal blocks, A, M, N, K
+//   gdn_bwd_scan_kernel  one workgroup per (b, h, 16 columns, direction): S entering and D leaving
+//                        every chunk, one D x D product per chunk
+//   gdn_bwd_grad_kernel  one workgroup per (b, h, chunk): the gradients
+// so only the scan is serial, and its step is one product.
+//
+// Products run on v_mfma_f32_16x16x4_f32: its operands are fp32 as they come out of the accumulators
+// (no splitting into bf16 parts, nothing lost), and a tile held in accumulator layout (lane 16 g4 +
+// r16: rows 4 g4 + r of column r16) is a B operand as it stands when product r contracts rows
+// 4 g4 + r.  Dependent products issue back to back (32 cycles each), so the block substitutions
+// with L cost no more than products with an explicit inverse would.
+//
+// Measured, forward and backward together (bf16): B=4, H=6, T=8192, D=64, gate and beta per head
+// 3064 -> 626 us; B=4, H=12, T=2048, D=128, gate per key dim 5934 -> 943 us, against the token-serial
+// kernels.  Of that the map kernel 156 / 220 us, the scan 106 / 211, the gradients 253 / 319.
+//
+// A chunk in which some key dim decays by more than GB_SPAN nats forms its pair sums from running
+// products of the decays instead (L and A in the map kernel, [.] in the gradient kernel); the
+// products with S and D use factors of at most 1 everywhere.
+#include "kernels.h"
+
+namespace triune {
+
+namespace {
+
+constexpr int GC = 64;            // tokens per chunk
+constexpr float GB_SPAN = 128.f;  // factors within e^(+-64)
+constexpr float GB_GMIN = -104.f; // e^-104 is 0 in fp32: gates below it (-inf resets) act alike
+constexpr int TSR = 20;           // row stride of a 16 x 16 tile in LDS (floats): rows and columns conflict-free
+constexpr int TSZ = 16 * TSR;
+constexpr int NTL = 10;           // lower-triangular 16 x 16 tiles of a 64 x 64 matrix
+
+__host__ __device__ constexpr int tl(int i, int j) { return i * (i + 1) / 2 + j; }
+
+// c + a b over 16 contracted indices: product r contracts index 4 g4 + r.
+__device__ __forceinline__ f32x4 mma(const f32x4& a, const f32x4& b, f32x4 c) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r], b[r], c, 0, 0, 0);
+    return c;
+}
+
+struct Lane {
+    int w, g4, r16;
+    __device__ __forceinline__ Lane() {
+        const int l = threadIdx.x & 63;
+        w = threadIdx.x >> 6;
+        g4 = l >> 4;
+        r16 = l & 15;
+    }
+};
+
+// Operand whose free index is the row of a row-major plane or tile (contracted index along the row).
+__device__ __forceinline__ f32x4 row_frag(const float* p, int ld, const Lane& L) {
+    return *reinterpret_cast<const f32x4*>(p + L.r16 * ld + 4 * L.g4);
+}
+// Operand whose free index is the column (contracted index down the rows).
+__device__ __forceinline__ f32x4 col_frag(const float* p, int ld, const Lane& L) {
+    const float* q = p + 4 * L.g4 * ld + L.r16;
+    return f32x4{q[0], q[ld], q[2 * ld], q[3 * ld]};
+}
+__device__ __forceinline__ void put_tile(float* p, int ld, const Lane& L, const f32x4& x) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) p[(4 * L.g4 + r) * ld + L.r16] = x[r];
+}
+
+// Four consecutive 16-bit elements of an LDS row as an operand.
+template <typename T>
+__device__ __forceinline__ f32x4 row_frag16(const T* p, int ld, const Lane& L) {
+    typedef T v4 __attribute__((ext_vector_type(4)));
+    const v4 x = *reinterpret_cast<const v4*>(p + L.r16 * ld + 4 * L.g4);
+    return f32x4{(float)x[0], (float)x[1], (float)x[2], (float)x[3]};
+}
+
+// A chunk's rows in accumulator layout: x[i][r] = row 16 i + 4 g4 + r of the lane's column, zero
+// past the nv valid rows.  p: the column's element in the chunk's first row; st: row stride.
+template <typename T>
+__device__ __forceinline__ void load_rows(const T* p, int64_t st, int nv, const Lane& L, f32x4 (&x)[4]) {
+    if (nv == GC) {
+        const T* q = p + 4 * L.g4 * st;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) x[i][r] = (float)q[(16 * i + r) * st];
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int t = 16 * i + 4 * L.g4 + r;
+                const float y = (float)p[(t < nv ? t : 0) * st];
+                x[i][r] = t < nv ? y : 0.f;
+            }
+    }
+}
+__device__ __forceinline__ void load_rows_dt(const void* p, int64_t off, int dt, int64_t st, int nv, const Lane& L,
+                                             f32x4 (&x)[4]) {
+    if (dt == DT_F32) load_rows(reinterpret_cast<const float*>(p) + off, st, nv, L, x);
+    else if (dt == DT_BF16) load_rows(reinterpret_cast<const __bf16*>(p) + off, st, nv, L, x);
+    else load_rows(reinterpret_cast<const _Float16*>(p) + off, st, nv, L, x);
+}
+
+template <typename T>
+__device__ __forceinline__ void store_rows(T* p, int64_t st, int nv, const Lane& L, const f32x4 (&x)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int t = 16 * i + 4 * L.g4 + r;
+            if (t < nv) p[t * st] = (T)x[i][r];
+        }
+}
+__device__ __forceinline__ void store_rows_dt(void* p, int64_t off, int dt, int64_t st, int nv, const Lane& L,
+                                              const f32x4 (&x)[4]) {
+    if (dt == DT_F32) store_rows(reinterpret_cast<float*>(p) + off, st, nv, L, x);
+    else if (dt == DT_BF16) store_rows(reinterpret_cast<__bf16*>(p) + off, st, nv, L, x);
+    else store_rows(reinterpret_cast<_Float16*>(p) + off, st, nv, L, x);
+}
+
+// Sum over the four row groups, in every lane.
+__device__ __forceinline__ float g4_sum(float x) { return xor_sum<32>(xor_sum<16>(x)); }
+
+// Sums over the chunk's tokens of the lane's column in accumulator layout: inc[i][r] over tokens up
+// to and with 16 i + 4 g4 + r, exc[i][r] without it; the total is returned.  REV: from the end.
+template <bool REV>
+__device__ __forceinline__ float token_scan(const f32x4 (&x)[4], const Lane& L, f32x4 (&inc)[4], f32x4 (&exc)[4]) {
+    float run = 0.f;
+#pragma unroll
+    for (int ii = 0; ii < 4; ++ii) {
+        const int i = REV ? 3 - ii : ii;
+        float s = 0.f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s += x[i][r];
+        const RowPair a = swap16(s);
+        const RowPair b = swap32(a.lo + a.hi);
+        float e = run;
+        if constexpr (REV) {
+            e += (L.g4 & 2) ? 0.f : b.hi;
+            e += (L.g4 & 1) ? 0.f : a.hi;
+        } else {
+            e += (L.g4 & 2) ? b.lo : 0.f;
+            e += (L.g4 & 1) ? a.lo : 0.f;
+        }
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr) {
+            const int r = REV ? 3 - rr : rr;
+            exc[i][r] = e;
+            e += x[i][r];
+            inc[i][r] = e;
+        }
+        run += b.lo + b.hi;
+    }
+    return run;
+}
+
+// What both chunk kernels know of a chunk: its place, its gates' sums and its rows.
+struct Chunk {
+    int64_t b, h, c, id;  // id: (b H + h) NC + c
+    int nv;
+};
+__device__ __forceinline__ Chunk chunk_of(const GdnChunkBwdParams& p) {
+    // heads fastest: neighbouring workgroups read neighbouring rows
+    const int64_t x = blockIdx.x;
+    Chunk k;
+    k.h = x % p.f.H;
+    const int64_t y = x / p.f.H;
+    k.c = y % p.nc;
+    k.b = y / p.nc;
+    k.id = (k.b * p.f.H + k.h) * p.nc + k.c;
+    const int64_t left = p.f.T - k.c * GC;
+    k.nv = left < GC ? (int)left : GC;
+    return k;
+}
+
+// The gate of the lane's key dim: x = min(g, 0), held at GB_GMIN.
+__device__ __forceinline__ void load_gate(const GdnChunkBwdParams& p, const Chunk& k, int col, const Lane& L,
+                                          f32x4 (&x)[4]) {
+    load_rows_dt(p.f.g, k.b * p.f.g_sb + k.c * GC * p.f.g_st + k.h * p.f.g_sh + (p.g_head ? 0 : col), p.f.g_dt,
+                 p.f.g_st, k.nv, L, x);
+}
+__device__ __forceinline__ float gate_val(float g) { return fmaxf(fminf(g, 0.f), GB_GMIN); }
+
+__device__ __forceinline__ void load_beta(const GdnChunkBwdParams& p, const Chunk& k, const Lane& L, f32x4 (&x)[4]) {
+    if (p.f.beta_kind == BETA_HEAD) {
+        load_rows_dt(p.f.beta, k.b * p.f.b_sb + k.c * GC * p.f.b_st + k.h * p.f.b_sh, p.f.beta_dt, p.f.b_st, k.nv, L,
+                     x);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = f32x4{1.f, 1.f, 1.f, 1.f};
+    }
+}
+
+template <typename T>
+__device__ __forceinline__ const T* row_ptr(const void* p, int64_t sb, int64_t st, int64_t sh, const Chunk& k) {
+    return reinterpret_cast<const T*>(p) + k.b * sb + k.c * GC * st + k.h * sh;
+}
+
+// X_i = T_ii (R_i - sum_{j<i} L_ij X_j), in place.  tiles: T_ii on the diagonal, -L_ij below it.
+__device__ __forceinline__ void solve(const float* tiles, const Lane& L, f32x4 (&x)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        f32x4 a = x[i];
+#pragma unroll
+        for (int j = 0; j < i; ++j) a = mma(row_frag(tiles + tl(i, j) * TSZ, TSR, L), x[j], a);
+        x[i] = mma(row_frag(tiles + tl(i, i) * TSZ, TSR, L), a, zero4());
+    }
+}
+// The same with the transpose: X_i = T_ii^T (Y_i - sum_{j>i} L_ji^T X_j).
+__device__ __forceinline__ void solve_t(const float* tiles, const Lane& L, f32x4 (&x)[4]) {
+#pragma unroll
+    for (int i = 3; i >= 0; --i) {
+        f32x4 a = x[i];
+#pragma unroll
+        for (int j = 3; j > i; --j) a = mma(col_frag(tiles + tl(j, i) * TSZ, TSR, L), x[j], a);
+        x[i] = mma(col_frag(tiles + tl(i, i) * TSZ, TSR, L), a, zero4());
+    }
+}
+
+__device__ __forceinline__ void tile_ij(int n, int& i, int& j) {
+    i = n >= 6 ? 3 : (n >= 3 ? 2 : (n >= 1 ? 1 : 0));
+    j = n - tl(i, 0);
+}
+
+// x where the tile entry lies below (or, with diag, on) the diagonal of tile (i, j), else 0.
+__device__ __forceinline__ f32x4 lower(const f32x4& x, bool on_diag, bool with_diag, const Lane& L) {
+    if (!on_diag) return x;
+    f32x4 y;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int t = 4 * L.g4 + r;
+        y[r] = (t > L.r16 || (with_diag && t == L.r16)) ? x[r] : 0.f;
+    }
+    return y;
+}
+
+// ---------------------------------------------------------------------------------------
+// Chunk maps
+// ---------------------------------------------------------------------------------------
+template <int D>
+struct MapLay {
+    static constexpr int NW = D / 16;
+    static constexpr int LD = D + 4;  // rows 4 banks apart for row reads, 4 rows 16 banks apart for column reads
+    static constexpr int PL = GC * LD;
+    static constexpr int BYTES = (3 * PL + 2 * NTL * TSZ + GC) * 4;
+};
+
+// MFMA-bound: 416 products of 32 cycles per wave and chunk at D = 64 (2 workgroups per CU).
+template <typename T, int D>
+__global__ __launch_bounds__(4 * D, 2) void gdn_bwd_map_kernel(GdnChunkBwdParams p) {
+    using Y = MapLay<D>;
+    constexpr int NW = Y::NW, LD = Y::LD;
+    __shared__ __attribute__((aligned(16))) char smem[Y::BYTES];
+    float* P0 = reinterpret_cast<float*>(smem);
+    float* P1 = P0 + Y::PL;
+    float* P2 = P1 + Y::PL;
+    float* sL = P2 + Y::PL;       // T_ii and -L_ij
+    float* sA = sL + NTL * TSZ;   // A
+    float* sB = sA + NTL * TSZ;   // beta (wide chunks)
+    const Lane L;
+    const int w = L.w, g4 = L.g4, r16 = L.r16, col = 16 * w + r16;
+    const Chunk k = chunk_of(p);
+
+    f32x4 q[4], kk[4], g[4], be[4], G[4], Gp[4];
+    load_rows(row_ptr<T>(p.f.q, p.f.q_sb, p.f.q_st, p.f.q_sh, k) + col, p.f.q_st, k.nv, L, q);
+    load_rows(row_ptr<T>(p.f.k, p.f.k_sb, p.f.k_st, p.f.k_sh, k) + col, p.f.k_st, k.nv, L, kk);
+    load_gate(p, k, col, L, g);
+    load_beta(p, k, L, be);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) g[i][r] = gate_val(g[i][r]);
+    const float gc = token_scan<false>(g, L, G, Gp);
+    const bool wide = __syncthreads_or(gc < -GB_SPAN);
+    const float ec = fast_exp(gc);
+
+    if (!wide) {
+        const float m = 0.5f * gc, em = fast_exp(m);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int a = (16 * i + 4 * g4 + r) * LD + col;
+                P0[a] = q[i][r] *= fast_exp(G[i][r] - m);
+                P2[a] = g[i][r] = kk[i][r] * be[i][r] * fast_exp(m - G[i][r]);  // g holds the W rows from here on
+                P1[a] = kk[i][r] *= fast_exp(Gp[i][r] - m);
+            }
+        __syncthreads();
+        for (int n = w; n < NTL; n += NW) {
+            int i, j;
+            tile_ij(n, i, j);
+            f32x4 a = zero4();
+#pragma unroll
+            for (int kt = 0; kt < NW; ++kt)
+                a = mma(row_frag(P1 + 16 * i * LD + 16 * kt, LD, L), row_frag(P2 + 16 * j * LD + 16 * kt, LD, L), a);
+            put_tile(sL + n * TSZ, TSR, L, i == j ? lower(a, true, false, L) : -a);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            q[i] *= em;
+            kk[i] *= em;
+            g[i] *= em;
+        }
+    } else {
+        for (int n = threadIdx.x; n < 2 * NTL * TSZ; n += 4 * D) sL[n] = 0.f;
+        f32x4 S[4], Se[4];
+        token_scan<true>(g, L, S, Se);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int t = 16 * i + 4 * g4 + r;
+                P0[t * LD + col] = q[i][r];
+                P1[t * LD + col] = kk[i][r];
+                P2[t * LD + col] = fast_exp(g[i][r]);
+                if (w == 0 && r16 == 0) sB[t] = be[i][r];
+                q[i][r] *= fast_exp(G[i][r]);
+                g[i][r] = kk[i][r] * be[i][r] * fast_exp(Se[i][r]);
+                kk[i][r] *= fast_exp(Gp[i][r]);
+            }
+        __syncthreads();
+        const int lane = threadIdx.x & 63;
+        for (int s = w; s < GC; s += NW) {
+            float run[D / 64], dot = 0.f;
+#pragma unroll
+            for (int e = 0; e < D / 64; ++e) {
+                run[e] = sB[s] * P1[s * LD + lane + 64 * e];
+                dot += P0[s * LD + lane + 64 * e] * run[e];
+            }
+            dot = g4_sum(dpp_sum16(dot));
+            if (lane == 0) sA[tl(s >> 4, s >> 4) * TSZ + (s & 15) * (TSR + 1)] = dot;
+            for (int t = s + 1; t < GC; ++t) {
+                float l = 0.f, a = 0.f;
+#pragma unroll
+                for (int e = 0; e < D / 64; ++e) {
+                    const int o = t * LD + lane + 64 * e;
+                    l += P1[o] * run[e];
+                    run[e] *= P2[o];
+                    a += P0[o] * run[e];
+                }
+                l = g4_sum(dpp_sum16(l));
+                a = g4_sum(dpp_sum16(a));
+                const int o = tl(t >> 4, s >> 4) * TSZ + (t & 15) * TSR + (s & 15);
+                if (lane == 0) {
+                    sL[o] = (t >> 4) == (s >> 4) ? l : -l;
+                    sA[o] = a;
+                }
+            }
+        }
+    }
+    __syncthreads();
+    if (w == 0) {
+        // T = (I + L_ii)^-1 of the four diagonal blocks, one column per lane: T[i] = 1[i = c] - sum L[i][k] T[k]
+        float* t = sL + (g4 * (g4 + 3) / 2) * TSZ;
+        float x[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            float a = i == r16 ? 1.f : 0.f;
+#pragma unroll
+            for (int k4 = 0; k4 < i; k4 += 4) {
+                const f32x4 l = *reinterpret_cast<const f32x4*>(t + i * TSR + k4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (k4 + e < i) a = fmaf(-l[e], x[k4 + e], a);
+            }
+            x[i] = a;
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) t[i * TSR + r16] = x[i];
+    } else if (!wide) {
+        for (int n = w - 1; n < NTL; n += NW - 1) {
+            int i, j;
+            tile_ij(n, i, j);
+            f32x4 a = zero4();
+#pragma unroll
+            for (int kt = 0; kt < NW; ++kt)
+                a = mma(row_frag(P0 + 16 * i * LD + 16 * kt, LD, L), row_frag(P2 + 16 * j * LD + 16 * kt, LD, L), a);
+            put_tile(sA + n * TSZ, TSR, L, lower(a, i == j, true, L));
+        }
+    }
+    f32x4 v[4], dO[4];
+    load_rows(row_ptr<T>(p.f.v, p.f.v_sb, p.f.v_st, p.f.v_sh, k) + col, p.f.v_st, k.nv, L, v);
+    if (p.dout)
+        load_rows(row_ptr<T>(p.dout, p.do_sb, p.do_st, p.do_sh, k) + col, p.do_st, k.nv, L, dO);
+    else
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dO[i] = zero4();
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int a = (16 * i + 4 * g4 + r) * LD + col;
+            P0[a] = q[i][r];
+            P1[a] = kk[i][r];
+            P2[a] = g[i][r];
+        }
+    float* wt = p.ws_t + k.id * (2 * NTL * 256);
+    for (int n = threadIdx.x; n < 2 * NTL * 64; n += 4 * D) {
+        const int tile = n >> 6, row = (n >> 2) & 15, c4 = (n & 3) * 4;
+        *reinterpret_cast<f32x4*>(wt + n * 4) = *reinterpret_cast<const f32x4*>(sL + tile * TSZ + row * TSR + c4);
+    }
+    __syncthreads();
+
+    float* wm = p.ws_m + k.id * (D * D);
+    float* wn = p.ws_s + k.id * (D * D);
+    float* wk = p.ws_d + k.id * (D * D);
+    // dR from A^T dO alone
+    f32x4 z[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        z[j] = zero4();
+#pragma unroll
+        for (int i = j; i < 4; ++i) z[j] = mma(col_frag(sA + tl(i, j) * TSZ, TSR, L), dO[i], z[j]);
+    }
+    solve_t(sL, L, z);
+    solve(sL, L, kk);
+    solve(sL, L, v);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) z[j] = -z[j];
+#pragma unroll 1
+    for (int rt = 0; rt < NW; ++rt) {
+        f32x4 am = zero4(), an = zero4(), ak = zero4();
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const f32x4 a = col_frag(P2 + 16 * i * LD + 16 * rt, LD, L);
+            am = mma(a, kk[i], am);
+            an = mma(a, v[i], an);
+            ak = mma(col_frag(P0 + 16 * i * LD + 16 * rt, LD, L), dO[i], ak);
+            ak = mma(col_frag(P1 + 16 * i * LD + 16 * rt, LD, L), z[i], ak);
+        }
+        f32x4 mm;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) mm[r] = ((rt == w && r16 == 4 * g4 + r) ? ec : 0.f) - am[r];
+        const int o = (rt * NW + w) * 256;
+        put_tile(wm + o, 16, L, mm);
+        put_tile(wn + o, 16, L, an);
+        put_tile(wk + o, 16, L, ak);
+    }
+}
+
+// ---------------------------------------------------------------------------------------
+// Scan over the chunks: S_next = M S + N forwards, D_prev = M^T D + K backwards
+// ---------------------------------------------------------------------------------------
+// One workgroup per (b, h, direction, strip of 16 columns), one wave per 16-row tile: latency-bound
+// (D / 4 products of 32 cycles and one barrier per chunk).  A pair's strips read the same maps, so
+// its workgroups share an XCD (workgroup x runs on XCD x mod 8).  The maps and N / K of the next PF
+// chunks are in flight.
+template <int D, int PF, bool REV>
+__device__ __forceinline__ void scan_walk(const GdnChunkBwdParams& p, float* sX, int64_t bh, int strip) {
+    constexpr int NW = D / 16, XLD = D + 4;
+    const Lane L;
+    const int w = L.w;
+    const int64_t DD = (int64_t)D * D, base = bh * p.nc;
+    float* io = REV ? p.ws_d : p.ws_s;
+    const int own = (w * NW + strip) * 256;  // this wave's tile of the state
+    const float* x0 = REV ? p.dsf : p.f.s0;
+    f32x4 x = zero4();
+    const int64_t flat = bh * DD + (16 * w + 4 * L.g4) * D + 16 * strip + L.r16;
+    if (x0)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[r] = x0[flat + r * D];
+    f32x4 mf[PF][NW], yf[PF];
+    auto fetch = [&](int64_t n, f32x4(&m)[NW], f32x4& y) {
+        const int64_t c = base + (REV ? p.nc - 1 - n : n);
+        const float* M = p.ws_m + c * DD;
+#pragma unroll
+        for (int kt = 0; kt < NW; ++kt)
+            m[kt] = REV ? col_frag(M + (kt * NW + w) * 256, 16, L) : row_frag(M + (w * NW + kt) * 256, 16, L);
+        y = col_frag(io + c * DD + own, 16, L);
+    };
+#pragma unroll
+    for (int u = 0; u < PF; ++u) fetch(u < p.nc ? u : p.nc - 1, mf[u], yf[u]);
+    for (int64_t n0 = 0; n0 < p.nc; n0 += PF) {
+#pragma unroll
+        for (int u = 0; u < PF; ++u) {
+            const int64_t n = n0 + u;
+            if (n >= p.nc) break;
+            const int64_t c = base + (REV ? p.nc - 1 - n : n);
+            put_tile(io + c * DD + own, 16, L, x);
+            float* X = sX + (n & 1) * 16 * XLD;
+            *reinterpret_cast<f32x4*>(X + L.r16 * XLD + 16 * w + 4 * L.g4) = x;
+            __syncthreads();
+            f32x4 a = yf[u], b = zero4();
+#pragma unroll
+            for (int kt = 0; kt < NW; kt += 2) {
+                a = mma(mf[u][kt], row_frag(X + 16 * kt, XLD, L), a);
+                b = mma(mf[u][kt + 1], row_frag(X + 16 * (kt + 1), XLD, L), b);
+            }
+            x = a + b;
+            if (n + PF < p.nc) fetch(n + PF, mf[u], yf[u]);
+        }
+    }
+    if (REV && p.ds0)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) p.ds0[flat + r * D] = x[r];
+}
+
+template <int D, int PF>
+__global__ __launch_bounds__(4 * D) void gdn_bwd_scan_kernel(GdnChunkBwdParams p) {
+    constexpr int NW = D / 16;
+    __shared__ __attribute__((aligned(16))) float sX[2 * 16 * (D + 4)];
+    const int64_t BH = p.f.B * p.f.H;
+    const int64_t slot = blockIdx.x / 8;
+    const int64_t bh = slot / (2 * NW) * 8 + blockIdx.x % 8;
+    if (bh >= BH) return;
+    const int s = (int)(slot % (2 * NW));
+    if (s < NW) scan_walk<D, PF, false>(p, sX, bh, s);
+    else scan_walk<D, PF, true>(p, sX, bh, s - NW);
+}
+
+// ---------------------------------------------------------------------------------------
+// Gradients
+// ---------------------------------------------------------------------------------------
+template <int D>
+struct GradLay {
+    static constexpr int NW = D / 16;
+    static constexpr int LD = D + 4;
+    static constexpr int PL = GC * LD;
+    static constexpr int LO = D + 8;  // 16-bit row stride of the dO plane
+    static constexpr int BYTES = (2 * PL + 2 * NTL * TSZ + 2 * NW * GC) * 4 + GC * LO * 2;
+};
+
+// The pair sums of a wide chunk for the lane's key dim and its 16 tokens: running products of the
+// decays from each token outwards, with the other tokens' rows read again from memory.  pq and pb
+// go to rows of two LDS planes, pw to rows of D floats in memory (the lane's own elements).
+template <typename T, int D, int LD>
+__device__ __forceinline__ void wide_pairs(const GdnChunkBwdParams& p, const Chunk& k, int col, const float* sdA,
+                                        const float* sdL, float* pq, float* pb, float* pw) {
+    const Lane L;
+    const T* q = row_ptr<T>(p.f.q, p.f.q_sb, p.f.q_st, p.f.q_sh, k) + col;
+    const T* kr = row_ptr<T>(p.f.k, p.f.k_sb, p.f.k_st, p.f.k_sh, k) + col;
+    const int64_t goff = k.b * p.f.g_sb + k.c * GC * p.f.g_st + k.h * p.f.g_sh + (p.g_head ? 0 : col);
+    const int64_t boff = k.b * p.f.b_sb + k.c * GC * p.f.b_st + k.h * p.f.b_sh;
+    auto any = [](const void* b, int64_t o, int dt) {
+        return dt == DT_F32 ? reinterpret_cast<const float*>(b)[o]
+                            : (dt == DT_BF16 ? (float)reinterpret_cast<const __bf16*>(b)[o]
+                                             : (float)reinterpret_cast<const _Float16*>(b)[o]);
+    };
+    auto decay = [&](int t) { return fast_exp(gate_val(any(p.f.g, goff + t * p.f.g_st, p.f.g_dt))); };
+    auto wrow = [&](int t) {
+        const float b = p.f.beta_kind == BETA_HEAD ? any(p.f.beta, boff + t * p.f.b_st, p.f.beta_dt) : 1.f;
+        return b * (float)kr[t * p.f.k_st];
+    };
+#pragma unroll 1
+    for (int e = 0; e < 16; ++e) {
+        const int t = 16 * (e >> 2) + 4 * L.g4 + (e & 3);
+        float aq = 0.f, ab = 0.f, aw = 0.f;
+        if (t < k.nv) {
+            float rq = 1.f, rb = 1.f;  // products of the decays over (s, t] and (s, t - 1]
+#pragma unroll 1
+            for (int s = t; s >= 0; --s) {
+                const int o = tl(t >> 4, s >> 4) * TSZ + (t & 15) * TSR + (s & 15);
+                const float ws = wrow(s), a = decay(s);
+                aq += sdA[o] * ws * rq;
+                if (s < t) {
+                    ab += sdL[o] * ws * rb;
+                    rb *= a;
+                }
+                rq *= a;
+            }
+            float rw = 1.f;
+            aw = sdA[tl(t >> 4, t >> 4) * TSZ + (t & 15) * (TSR + 1)] * (float)q[t * p.f.q_st];
+#pragma unroll 1
+            for (int s = t + 1; s < k.nv; ++s) {
+                const int o = tl(s >> 4, t >> 4) * TSZ + (s & 15) * TSR + (t & 15);
+                aw += sdL[o] * (float)kr[s * p.f.k_st] * rw;
+                rw *= decay(s);
+                aw += sdA[o] * (float)q[s * p.f.q_st] * rw;
+            }
+        }
+        pq[t * LD + col] = aq;
+        pb[t * LD + col] = ab;
+        pw[t * D + col] = aw;
+    }
+}
+
+// MFMA-bound: 680 products of 32 cycles per wave and chunk at D = 64 (2 workgroups per CU).
+template <typename T, int D>
+__global__ __launch_bounds__(4 * D, 2) void gdn_bwd_grad_kernel(GdnChunkBwdParams p) {
+    using Y = GradLay<D>;
+    constexpr int NW = Y::NW, LD = Y::LD, LO = Y::LO;
+    __shared__ __attribute__((aligned(16))) char smem[Y::BYTES];
+    float* P1 = reinterpret_cast<float*>(smem);  // B0 rows, then U
+    float* P2 = P1 + Y::PL;                      // Wc rows, then dR
+    float* sL = P2 + Y::PL;                      // T_ii and -L_ij, then dL
+    float* sA = sL + NTL * TSZ;                  // A, then dA
+    float* red = sA + NTL * TSZ;                 // [2][NW][64] sums over each wave's key dims
+    T* sO = reinterpret_cast<T*>(red + 2 * NW * GC);
+    const Lane L;
+    const int w = L.w, g4 = L.g4, r16 = L.r16, col = 16 * w + r16;
+    const Chunk k = chunk_of(p);
+
+    f32x4 q[4], kk[4], g[4], be[4], G[4], Gp[4];
+    load_rows(row_ptr<T>(p.f.q, p.f.q_sb, p.f.q_st, p.f.q_sh, k) + col, p.f.q_st, k.nv, L, q);
+    load_rows(row_ptr<T>(p.f.k, p.f.k_sb, p.f.k_st, p.f.k_sh, k) + col, p.f.k_st, k.nv, L, kk);
+    load_gate(p, k, col, L, g);
+    load_beta(p, k, L, be);
+    f32x4 v[4], dO[4];
+    load_rows(row_ptr<T>(p.f.v, p.f.v_sb, p.f.v_st, p.f.v_sh, k) + col, p.f.v_st, k.nv, L, v);
+    if (p.dout)
+        load_rows(row_ptr<T>(p.dout, p.do_sb, p.do_st, p.do_sh, k) + col, p.do_st, k.nv, L, dO);
+    else
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dO[i] = zero4();
+    uint32_t pass = 0;  // tokens whose gate takes a gradient: not clamped, and not reset to 0
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if (!(g[i][r] > 0.f) && g[i][r] > GB_GMIN) pass |= 1u << (4 * i + r);
+            g[i][r] = gate_val(g[i][r]);
+        }
+    const float gc = token_scan<false>(g, L, G, Gp);
+    const bool wide = __syncthreads_or(gc < -GB_SPAN);
+    const float m = wide ? 0.f : 0.5f * gc;
+    f32x4 ew[4];  // e^(G_C - G)
+    if (wide) {
+        f32x4 S[4], Se[4];
+        token_scan<true>(g, L, S, Se);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) ew[i][r] = fast_exp(Se[i][r]);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) ew[i][r] = fast_exp(gc - G[i][r]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int t = 16 * i + 4 * g4 + r;
+            P1[t * LD + col] = kk[i][r] * fast_exp(Gp[i][r]);
+            P2[t * LD + col] = kk[i][r] * be[i][r] * ew[i][r];
+            sO[t * LO + col] = (T)dO[i][r];
+        }
+    const float* wt = p.ws_t + k.id * (2 * NTL * 256);
+    for (int n = threadIdx.x; n < 2 * NTL * 64; n += 4 * D) {
+        const int tile = n >> 6, row = (n >> 2) & 15, c4 = (n & 3) * 4;
+        *reinterpret_cast<f32x4*>(sL + tile * TSZ + row * TSR + c4) = *reinterpret_cast<const f32x4*>(wt + n * 4);
+    }
+    __syncthreads();
+
+    const float* S = p.ws_s + k.id * (D * D);
+    const float* Dn = p.ws_d + k.id * (D * D);
+    // value columns [16 w, 16 w + 16): U in v, dR in z
+    f32x4 z[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        z[j] = zero4();
+#pragma unroll
+        for (int i = j; i < 4; ++i) z[j] = mma(col_frag(sA + tl(i, j) * TSZ, TSR, L), dO[i], z[j]);
+    }
+#pragma unroll 2
+    for (int kt = 0; kt < NW; ++kt) {
+        const f32x4 s = -col_frag(S + (kt * NW + w) * 256, 16, L);
+        const f32x4 d = col_frag(Dn + (kt * NW + w) * 256, 16, L);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[i] = mma(row_frag(P1 + 16 * i * LD + 16 * kt, LD, L), s, v[i]);
+            z[i] = mma(row_frag(P2 + 16 * i * LD + 16 * kt, LD, L), d, z[i]);
+        }
+    }
+    solve(sL, L, v);
+    solve_t(sL, L, z);
+    const int64_t orow = ((k.b * p.f.T + k.c * GC) * p.f.H + k.h) * D + col, ost = p.f.H * D;
+    store_rows(reinterpret_cast<T*>(p.dv) + orow, ost, k.nv, L, z);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        put_tile(P1 + 16 * i * LD + 16 * w, LD, L, v[i]);
+        put_tile(P2 + 16 * i * LD + 16 * w, LD, L, z[i]);
+    }
+    __syncthreads();
+    for (int n = w; n < 2 * NTL; n += NW) {
+        const bool isA = n < NTL;
+        int i, j;
+        tile_ij(isA ? n : n - NTL, i, j);
+        f32x4 a = zero4();
+        if (isA) {
+#pragma unroll
+            for (int kt = 0; kt < NW; ++kt)
+                a = mma(row_frag16(sO + 16 * i * LO + 16 * kt, LO, L), row_frag(P1 + 16 * j * LD + 16 * kt, LD, L), a);
+            put_tile(sA + n * TSZ, TSR, L, lower(a, i == j, true, L));
+        } else {
+#pragma unroll
+            for (int kt = 0; kt < NW; ++kt)
+                a = mma(row_frag(P2 + 16 * i * LD + 16 * kt, LD, L), row_frag(P1 + 16 * j * LD + 16 * kt, LD, L), a);
+            put_tile(sL + (n - NTL) * TSZ, TSR, L, -lower(a, i == j, false, L));
+        }
+    }
+    __syncthreads();
+
+    // key dims [16 w, 16 w + 16): products with the states first
+    f32x4 aq[4], ab[4], aw[4];
+    float es = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) aq[i] = ab[i] = aw[i] = zero4();
+#pragma unroll 2
+    for (int kt = 0; kt < NW; ++kt) {
+        const f32x4 s = row_frag(S + (w * NW + kt) * 256, 16, L);
+        const f32x4 d = row_frag(Dn + (w * NW + kt) * 256, 16, L);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) es = fmaf(s[r], d[r], es);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            aq[i] = mma(row_frag16(sO + 16 * i * LO + 16 * kt, LO, L), s, aq[i]);
+            ab[i] = mma(row_frag(P2 + 16 * i * LD + 16 * kt, LD, L), s, ab[i]);
+            aw[i] = mma(row_frag(P1 + 16 * i * LD + 16 * kt, LD, L), d, aw[i]);
+        }
+    }
+    es = g4_sum(es) * fast_exp(gc);
+    float ew_sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            aq[i][r] *= fast_exp(G[i][r]);
+            ab[i][r] *= -fast_exp(Gp[i][r]);
+            aw[i][r] *= ew[i][r];
+            ew_sum = fmaf(kk[i][r] * be[i][r], aw[i][r], ew_sum);
+        }
+    es += g4_sum(ew_sum);  // sum over the value columns of D * S_next
+
+    if (!wide) {
+        f32x4 x[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) x[i][r] = kk[i][r] * be[i][r] * fast_exp(m - G[i][r]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            f32x4 a = zero4(), b = zero4();
+#pragma unroll
+            for (int j = 0; j <= i; ++j) {
+                a = mma(row_frag(sA + tl(i, j) * TSZ, TSR, L), x[j], a);
+                b = mma(row_frag(sL + tl(i, j) * TSZ, TSR, L), x[j], b);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                aq[i][r] = fmaf(a[r], fast_exp(G[i][r] - m), aq[i][r]);
+                ab[i][r] = fmaf(b[r], fast_exp(Gp[i][r] - m), ab[i][r]);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            f32x4 a = zero4();
+#pragma unroll
+            for (int i = j; i < 4; ++i) {
+                f32x4 y;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) y[r] = q[i][r] * fast_exp(G[i][r] - m);
+                a = mma(col_frag(sA + tl(i, j) * TSZ, TSR, L), y, a);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) y[r] = kk[i][r] * fast_exp(Gp[i][r] - m);
+                a = mma(col_frag(sL + tl(i, j) * TSZ, TSR, L), y, a);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) aw[j][r] = fmaf(a[r], fast_exp(m - G[j][r]), aw[j][r]);
+        }
+    } else {
+        // once every wave is past its reads of U, dR and D, their places take the three sums
+        __syncthreads();
+        float* P3 = p.ws_d + k.id * (D * D);
+        wide_pairs<T, D, LD>(p, k, col, sA, sL, P1, P2, P3);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int a = (16 * i + 4 * g4 + r) * LD + col;
+                aq[i][r] += P1[a];
+                ab[i][r] += P2[a];
+                aw[i][r] += P3[(16 * i + 4 * g4 + r) * D + col];
+            }
+    }
+    store_rows(reinterpret_cast<T*>(p.dq) + orow, ost, k.nv, L, aq);
+    // q dq - w dw (x) and k dkB (y): dg_t = D * S_next + sum_{r >= t} x_r + sum_{r > t} y_r
+    f32x4 y[4], inc[4], exc[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float wdw = kk[i][r] * be[i][r] * aw[i][r];
+            q[i][r] = q[i][r] * aq[i][r] - wdw;
+            y[i][r] = q[i][r] + kk[i][r] * ab[i][r];
+            ab[i][r] = fmaf(be[i][r], aw[i][r], ab[i][r]);
+            aw[i][r] *= kk[i][r];
+        }
+    store_rows(reinterpret_cast<T*>(p.dk) + orow, ost, k.nv, L, ab);
+    token_scan<true>(y, L, inc, exc);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) exc[i][r] = (pass >> (4 * i + r) & 1) ? exc[i][r] + q[i][r] + es : 0.f;
+    if (!p.g_head) store_rows_dt(p.dg, orow, p.f.g_dt, ost, k.nv, L, exc);
+    const bool dbeta = p.f.beta_kind == BETA_HEAD;
+    if (!p.g_head && !dbeta) return;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float a = dpp_sum16(exc[i][r]), b = dpp_sum16(aw[i][r]);
+            const int t = 16 * i + 4 * g4 + r;
+            if (r16 == 0) {
+                red[w * GC + t] = a;
+                red[(NW + w) * GC + t] = b;
+            }
+        }
+    __syncthreads();
+    if (threadIdx.x < 2 * GC) {
+        const int t = threadIdx.x & (GC - 1), which = threadIdx.x >> 6;
+        float s = 0.f;
+#pragma unroll
+        for (int u = 0; u < NW; ++u) s += red[(which * NW + u) * GC + t];
+        void* o = which ? (dbeta ? p.dbeta : nullptr) : (p.g_head ? p.dg : nullptr);
+        const int dt = which ? p.f.beta_dt : p.f.g_dt;
+        const int64_t at = (k.b * p.f.T + k.c * GC + t) * p.f.H + k.h;
+        if (o && t < k.nv) {
+            if (dt == DT_F32) reinterpret_cast<float*>(o)[at] = s;
+            else if (dt == DT_BF16) reinterpret_cast<__bf16*>(o)[at] = (__bf16)s;
+            else reinterpret_cast<_Float16*>(o)[at] = (_Float16)s;
+        }
+    }
+}
+
+template <typename T, int D>
+hipError_t launch_t(const GdnChunkBwdParams& p, hipStream_t stream) {
+    constexpr int PF = D == 64 ? 4 : 2;
+    const unsigned chunks = (unsigned)(p.f.B * p.f.H * p.nc);
+    hipError_t e;
+    hipLaunchKernelGGL((gdn_bwd_map_kernel<T, D>), dim3(chunks), dim3(4 * D), 0, stream, p);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    const unsigned pairs8 = (unsigned)((p.f.B * p.f.H + 7) / 8 * 8);
+    hipLaunchKernelGGL((gdn_bwd_scan_kernel<D, PF>), dim3(pairs8 * 2 * (D / 16)), dim3(4 * D), 0, stream, p);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    hipLaunchKernelGGL((gdn_bwd_grad_kernel<T, D>), dim3(chunks), dim3(4 * D), 0, stream, p);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_gdn_bwd_chunk(const GdnChunkBwdParams& p, int D, hipStream_t stream) {
+    if (p.f.io_dt == DT_BF16) {
+        if (D == 64) return launch_t<__bf16, 64>(p, stream);
+        if (D == 128) return launch_t<__bf16, 128>(p, stream);
+    } else if (p.f.io_dt == DT_F16) {
+        if (D == 64) return launch_t<_Float16, 64>(p, stream);
+        if (D == 128) return launch_t<_Float16, 128>(p, stream);
+    }
+    return hipErrorInvalidValue;
+}
+
+}  // namespace triune

@@ -163,6 +163,24 @@ struct GdnBwdParams {
     float* seg_de;           // gradient reaching the last state of segment s
 };
 
+// Gradients of the Gated DeltaNet reference variant in chunk form (gdn_bwd_chunk.hip): 16-bit I/O,
+// D = Dk = Dv in {64, 128}, beta none or per (token, head).  Outputs contiguous [B, T, H, D].
+struct GdnChunkBwdParams {
+    GdnParams f;             // forward inputs and shapes; f.s0 the initial state or null
+    int g_head;              // one gate per (token, head): f.g is [B, T, H] and dg its sum over the key dims
+    const void* dout;        // [B, T, H, D] upstream gradient of o in the I/O dtype (strides below) or null
+    int64_t do_sb, do_st, do_sh;
+    const float* dsf;        // [B, H, D, D] upstream gradient of the final state or null
+    void* dq; void* dk; void* dv; void* dg; void* dbeta;
+    float* ds0;              // [B, H, D, D] or null
+    int64_t nc;              // chunks per sequence
+    // per (b, h, chunk), fp32; D x D matrices as row-major grids of row-major 16 x 16 tiles
+    float* ws_t;             // ten tiles of (I + L)'s blocks, ten of A
+    float* ws_m;             // M
+    float* ws_s;             // N, then the state entering the chunk
+    float* ws_d;             // K, then the gradient reaching the state that leaves it
+};
+
 // GLA input pre-processing (in place): q, k in qkv [B, T, 3, H, HD] (element strides sb, st, sp
 // between the q/k/v parts, sh), g [B, T, H, HD]; cos/sin [T, HD] rows cs_st apart.
 struct PrepParams {
@@ -228,6 +246,7 @@ hipError_t launch_gdn_decode(const GdnParams& a, int D, int max_blocks, hipStrea
 int gdn_bwd_chunk_tokens(int D, int64_t waves, int64_t cus);
 int gdn_bwd_col_slices(int D);
 hipError_t launch_gdn_bwd(const GdnBwdParams& p, int D, hipStream_t stream);
+hipError_t launch_gdn_bwd_chunk(const GdnChunkBwdParams& p, int D, hipStream_t stream);
 hipError_t launch_gdn_slice_sum(const float* src, int nsl, int64_t stride, int64_t n, void* out, int dt,
                                 hipStream_t stream);
 // Prefill: K1 segment states, K2 scan, K3 outputs (and, for varlen, K0 plan).

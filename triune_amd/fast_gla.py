@@ -38,6 +38,9 @@ _DECODE_PAIRS = ((32, 32), (64, 64), (64, 128), (128, 64), (128, 128))
 # unless this is False, in which case every call takes the token-serial kernel (kept for fp32 I/O
 # at head dim 128 and single tokens).
 _chunked_gdn_enabled = True
+# Gradients that are all 16-bit come from the chunk-form kernels unless this is False (then from the
+# token-serial ones, which serve every other call).
+_chunked_gdn_bwd_enabled = True
 # Gates with one value per (token, head) take the scalar-decay chunked kernels unless this is False
 # (then they run the per-key-dim chunked kernels on the broadcast gate).
 _scalar_gdn_enabled = True
@@ -636,14 +639,15 @@ def _scalar_gate(g):
 
 def _gdn(q, k, v, g, beta, initial_state, beta_kind, out_dtype=None):
     _check_io(q, k, v, g)
+    _on_device(beta, initial_state)
+    grad = _needs_grad(q, k, v, g, beta, initial_state)
     if g.dim() == 3 or g.shape[-1] != q.shape[-1]:  # one gate per (token, head): the per-dim kernels take it broadcast
         sg = _scalar_gate(g)
         if sg is None:
             raise ValueError(f"Gated DeltaNet gate of shape {tuple(g.shape)}: expected [B, T, H], [B, T, H, 1], "
                              "[B, T, H, D] broadcast over the head dim, or [B, T, H, Dk]")
-        g = sg.unsqueeze(-1).expand(*sg.shape, q.shape[-1])
-    _on_device(beta, initial_state)
-    if _needs_grad(q, k, v, g, beta, initial_state):
+        g = sg if grad else sg.unsqueeze(-1).expand(*sg.shape, q.shape[-1])
+    if grad:
         # the reference differentiates its PyTorch recurrence here (fast_gla.py:885-904)
         return _GatedDeltaNet.apply(q, k, v, g, beta, initial_state, beta_kind, out_dtype)
     return _gdn_fwd(q, k, v, g, beta, initial_state, beta_kind, out_dtype)
@@ -665,6 +669,14 @@ def _gdn_bwd(q, k, v, g, beta, initial_state, beta_kind, do, ds):
             ds0 = (ds if ds is not None else torch.zeros_like(initial_state)).to(initial_state.dtype)
         return z(q), z(k), z(v), z(g), None if beta is None else z(beta), ds0
     qp, kp, vp = (_vec_layout(_pad_last(x, D), 1) for x in (q, k, v))
+    # every gradient rounded to 16 bits: the chunk form on the matrix cores
+    if (beta_kind in (_lib.BETA_NONE, _lib.BETA_HEAD) and q.dtype != torch.float32 and g.dtype == q.dtype and
+            (beta is None or beta.dtype == q.dtype) and (do is None or do.dtype == q.dtype) and
+            initial_state is None and _chunked_gdn_bwd_enabled):
+        return _gdn_bwd_chunked(qp, kp, vp, g, beta, beta_kind, do, ds, Dk0, Dv0, D)
+    if g.dim() == 3:
+        r = _gdn_bwd(q, k, v, g.unsqueeze(-1).expand(*g.shape, Dk0), beta, initial_state, beta_kind, do, ds)
+        return (*r[:3], r[3].sum(-1), *r[4:])
     gp = _vec_layout(_pad_last(g, D), 1)
     bp, bst = None, (0, 0, 0)
     if beta is not None:
@@ -701,13 +713,42 @@ def _gdn_bwd(q, k, v, g, beta, initial_state, beta_kind, do, ds):
     return dq, dk, dv, dg.to(g.dtype), None if db is None else db.to(beta.dtype), ds0
 
 
+def _gdn_bwd_chunked(q, k, v, g, beta, beta_kind, do, ds, Dk0, Dv0, D):
+    """_gdn_bwd on triune_hip_gdn_bwd_chunked for q, k, v of the kernel width D; g is [B, T, H, Dk0]
+    or, one gate per (token, head), [B, T, H] (its gradient then comes back summed over the key
+    dims)."""
+    B, T, H, _ = q.shape
+    head = g.dim() == 3
+    gp = g if head else _vec_layout(_pad_last(g, D), 1)
+    dop = None if do is None else _vec_layout(_pad_last(do, D), 1)
+    dsf = _state_in(ds, D, D)
+    dq, dk, dv = (torch.empty(B, T, H, D, device=q.device, dtype=q.dtype) for _ in range(3))
+    dg = torch.empty((B, T, H) if head else (B, T, H, D), device=q.device, dtype=g.dtype)
+    db = None if beta is None else torch.empty(B, T, H, device=q.device, dtype=beta.dtype)
+    L = lib()
+    wsb = L.triune_hip_gdn_bwd_chunked_workspace_size(B, T, H, D, D)
+    ws = torch.empty(max(int(wsb), 16), device=q.device, dtype=torch.uint8)
+    st = strides(_tok3(q), _tok3(k), _tok3(v), _tok3(gp), (0, 0, 0) if beta is None else _tok3(beta),
+                 _tok3(dop) if dop is not None else (0, 0, 0))
+    rc = L.triune_hip_gdn_bwd_chunked(
+        ptr(q), ptr(k), ptr(v), ptr(gp), dtype_code(q), dtype_code(gp), int(head), ptr(beta),
+        dtype_code(beta) if beta is not None else 0, beta_kind, st, None, ptr(dop), ptr(dsf), ptr(dq), ptr(dk),
+        ptr(dv), ptr(dg), ptr(db), None, B, T, H, D, D, ptr(ws), ws.numel(), stream_of(q),
+    )
+    check(rc, "triune_hip_gdn_bwd_chunked")
+    if not head:
+        dg = dg[..., :Dk0]
+    return dq[..., :Dk0], dk[..., :Dk0], dv[..., :Dv0], dg, db, None
+
+
 class _GatedDeltaNet(torch.autograd.Function):
     """Gated DeltaNet with gradients: forward on the HIP forward kernels, backward on
     triune_hip_gdn_bwd (states recomputed from checkpoints)."""
 
     @staticmethod
     def forward(ctx, q, k, v, g, beta, initial_state, beta_kind, out_dtype):
-        o, s = _gdn_fwd(q, k, v, g, beta, initial_state, beta_kind, out_dtype)
+        gf = g.unsqueeze(-1).expand(*g.shape, q.shape[-1]) if g.dim() == 3 else g
+        o, s = _gdn_fwd(q, k, v, gf, beta, initial_state, beta_kind, out_dtype)
         ctx.save_for_backward(q, k, v, g, beta, initial_state)
         ctx.beta_kind = beta_kind
         return o, s
