@@ -10,7 +10,6 @@
 namespace triune {
 
 constexpr int CHUNK = 64;
-constexpr float SPAN_MAX = 64.f;
 constexpr int PAD = 4;  // row padding (elements) of LDS planes: spreads rows over banks
 
 struct Work {
@@ -76,7 +75,18 @@ struct Prec {
     static constexpr bool F32 = std::is_same<TIn, float>::value;
     static constexpr int NS = F32 ? 3 : 2;                                             // parts of derived operands
     static constexpr int NX = F32 ? 3 : (std::is_same<TIn, _Float16>::value ? 2 : 1);  // parts of V
+    // Largest chunk decay span (-G_C of a key dim, nats) of the GLA chunk kernels' factored form;
+    // chunks past it run token by token.  16-bit I/O: every factor lies in e^[-64, 64], where both
+    // bf16 parts are normal numbers; the non-causal products, up to e^128, overflow, but they lie
+    // in diagonal tiles, where a bit mask drops them.  fp32 I/O keeps half of that: the exponents'
+    // own rounding (about |x| 2^-24) would otherwise reach the third parts' size.  Gates of
+    // logsigmoid(N(0, 1)), the reference model's at initialisation, span 52 +- 5 nats: with a limit
+    // of 64 one chunk in five (4 heads of 64 dims) ran token by token and held up the whole launch
+    // (1024-token tile from raw projections 102 us against 20 us without such chunks).
+    static constexpr float SPAN_MAX = F32 ? 64.f : 128.f;
 };
+// Log-decay limit of the scalar-gate Gated DeltaNet chunks (gdn_scalar.hip).
+constexpr float GDN_SG_SPAN_MAX = 64.f;
 
 // Every LDS operand is stored token-major as NP planes of bf16 parts (x ~= p0 + p1 (+ p2)).
 // Fragments whose K index is the token come out of the same planes through the transposed

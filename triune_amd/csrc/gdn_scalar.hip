@@ -18,7 +18,7 @@
 // and U are split into bf16 parts.  (I + L)^{-1} is applied block-wise on 16-token blocks,
 // U_i = T_ii (R_i - sum_{j<i} L_ij U_j), with the state-independent products T_ii L_ij and
 // T_ii diag(e^{gamp}) K_i formed once per chunk; each T_ii comes from an fp32 back substitution
-// on T_ii^T = (I + L_ii^T)^{-1}, one wave per block.  Chunks whose total log-decay exceeds SPAN_MAX
+// on T_ii^T = (I + L_ii^T)^{-1}, one wave per block.  Chunks whose total log-decay exceeds GDN_SG_SPAN_MAX
 // (or is not finite) run token by token: the exponent differences come from prefix sums, whose
 // rounding grows with the chunk total.
 // The segment decomposition is the one of gdn_chunk.hip and shares its workspace layout and scan:
@@ -241,7 +241,7 @@ __device__ __forceinline__ void sg_load(SIn<TIn>& c, const SgCtx& x, int64_t tc,
 }
 
 // Token-by-token update of one wave's 16 state columns (chunks whose total log-decay is below
-// -SPAN_MAX or not finite).  S tile db holds S[16*db + 4*g4 + i][c0 + r16]; with_v false reads V
+// -GDN_SG_SPAN_MAX or not finite).  S tile db holds S[16*db + 4*g4 + i][c0 + r16]; with_v false reads V
 // as zero.  Rows come from the context's token-0 addresses.
 template <typename TIn, bool OUT>
 __device__ void sg_tokenwise(const SgCtx& x, int c0, int64_t tc, int nv, int g4, int r16, bool with_v,
@@ -386,7 +386,7 @@ struct SgStep {
                 }
                 if (lane == 0) {
                     sF[L::F_MISC] = __builtin_amdgcn_exp2f(e3);
-                    sF[L::F_MISC + 1] = (e3 >= -SPAN_MAX * LOG2E) ? 0.f : 1.f;  // false for NaN too
+                    sF[L::F_MISC + 1] = (e3 >= -GDN_SG_SPAN_MAX * LOG2E) ? 0.f : 1.f;  // false for NaN too
                 }
             }
         }

@@ -282,7 +282,7 @@ __global__ __launch_bounds__(OP_THREADS, 1) void gla_onepass_kernel(PrefillParam
     {
         bool bad = tail_unclamped;
 #pragma unroll
-        for (int i = 0; i < DL; ++i) bad |= !(GC[i] >= -SPAN_MAX);
+        for (int i = 0; i < DL; ++i) bad |= !(GC[i] >= -Prec<TIn>::SPAN_MAX);
         const bool any_bad = __any(bad);
         if (lane == 0) sFLAG[wave] = any_bad ? 1 : 0;
         if (tg == 0) {
@@ -466,15 +466,18 @@ __global__ __launch_bounds__(OP_THREADS, 1) void gla_onepass_kernel(PrefillParam
 #pragma unroll
                 for (int t = 0; t < MT; ++t) acc[t] = mfma_split<NS, NS, NS>(kf[t], qf[t], acc[t]);
             }
-            f32x4 diag;
+            // causal: bit masks of a diagonal tile (key 4*g4 + j <= query r16; the others may overflow)
+            typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+            u32x4 diag;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) diag[j] = (4 * g4 + j > r16) ? 0.f : 1.f;
+            for (int j = 0; j < 4; ++j) diag[j] = 4 * g4 + j > r16 ? 0u : ~0u;
 #pragma unroll
             for (int t = 0; t < MT; ++t) {
                 const int i = wave + t * NW;
                 if (i >= 10) continue;
-                const f32x4 m = sb[t] == tb[t] ? diag : f32x4{1.f, 1.f, 1.f, 1.f};
-                const float xx[4] = {acc[t][0] * m[0], acc[t][1] * m[1], acc[t][2] * m[2], acc[t][3] * m[3]};
+                const u32x4 m = sb[t] == tb[t] ? diag : u32x4{~0u, ~0u, ~0u, ~0u};
+                const f32x4 y = __builtin_bit_cast(f32x4, __builtin_bit_cast(u32x4, acc[t]) & m);
+                const float xx[4] = {y[0], y[1], y[2], y[3]};
                 lds_put_row<NS, 4>(sAT, L::ATP, (i * 64 + lane) * 4, xx);
             }
         }

@@ -367,7 +367,7 @@ struct OutStep {
             chunk_cumsum<DL>(G, GC, lane);
             bool bad = tail_unclamped;
 #pragma unroll
-            for (int i = 0; i < DL; ++i) bad |= !(GC[i] >= -SPAN_MAX);
+            for (int i = 0; i < DL; ++i) bad |= !(GC[i] >= -Prec<TIn>::SPAN_MAX);
             float mh[DL];  // -m log2(e), m = GC / 2
 #pragma unroll
             for (int i = 0; i < DL; ++i) mh[i] = -0.5f * LOG2E * GC[i];
@@ -448,16 +448,18 @@ struct OutStep {
 #pragma unroll
                     for (int t = 0; t < MT; ++t) acc[t] = mfma_split<NS, NS, NS>(kf[t], qf[t], acc[t]);
                 }
-                // causal mask of a diagonal tile (row = key 4*g4 + j, column = query r16) as factors
-                f32x4 diag;
+                // causal: bit masks of a diagonal tile (key 4*g4 + j <= query r16; the others may overflow)
+                typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+                u32x4 diag;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) diag[j] = (4 * g4 + j > r16) ? 0.f : 1.f;
+                for (int j = 0; j < 4; ++j) diag[j] = 4 * g4 + j > r16 ? 0u : ~0u;
 #pragma unroll
                 for (int t = 0; t < MT; ++t) {
                     const int i = wave + t * NW;
                     if (i >= 10) continue;
-                    const f32x4 m = sb[t] == tb[t] ? diag : f32x4{1.f, 1.f, 1.f, 1.f};
-                    const float x[4] = {acc[t][0] * m[0], acc[t][1] * m[1], acc[t][2] * m[2], acc[t][3] * m[3]};
+                    const u32x4 m = sb[t] == tb[t] ? diag : u32x4{~0u, ~0u, ~0u, ~0u};
+                    const f32x4 y = __builtin_bit_cast(f32x4, __builtin_bit_cast(u32x4, acc[t]) & m);
+                    const float x[4] = {y[0], y[1], y[2], y[3]};
                     lds_put_row<NS, 4>(sAT, L::ATP, (i * 64 + lane) * 4, x);
                 }
             }
