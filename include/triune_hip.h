@@ -117,6 +117,12 @@ int triune_hip_gla_decode_step(const void* q, const void* k, const void* v, cons
                                int g_dtype, const int64_t* strides, const float* state_in, float* state_out,
                                const int32_t* slots, int64_t n_state_rows, void* o, int o_dtype, int64_t B,
                                int64_t H, int Dk, int Dv, void* stream);
+/* The same, and with offsets != NULL (int64, one per state row, 8-byte aligned; needs slots) one is
+ * added to offsets[slots[b]] for every slot inside the pool. */
+int triune_hip_gla_decode_step_count(const void* q, const void* k, const void* v, const void* g, int io_dtype,
+                                     int g_dtype, const int64_t* strides, const float* state_in, float* state_out,
+                                     const int32_t* slots, int64_t n_state_rows, int64_t* offsets, void* o,
+                                     int o_dtype, int64_t B, int64_t H, int Dk, int Dv, void* stream);
 
 /* The reference's own decode-step signatures, for callers that bind them by name (device
  * pointers instead of the reference's host pointers; both run triune_hip_gla_decode_step in
@@ -410,6 +416,14 @@ int triune_hip_gla_fused_decode_step_slots(const void* qkvg, int io_dtype, const
                                            int state_dtype, const int32_t* slots, int64_t n_slots, void* o,
                                            int o_dtype, const int64_t* o_strides, int64_t B, int64_t H, int HD,
                                            void* stream);
+/* The same, and with offsets != NULL (int64 [n_slots], 8-byte aligned) one is added to
+ * offsets[slots[b]] for every slot inside the pool. */
+int triune_hip_gla_fused_decode_step_slots_count(const void* qkvg, int io_dtype, const int64_t* strides,
+                                                 const void* cos, const void* sin, int cs_dtype, int use_rope,
+                                                 void* state_pool, int state_dtype, const int32_t* slots,
+                                                 int64_t n_slots, int64_t* offsets, void* o, int o_dtype,
+                                                 const int64_t* o_strides, int64_t B, int64_t H, int HD,
+                                                 void* stream);
 
 #ifdef __cplusplus
 }

@@ -9,6 +9,7 @@ a call fails, a TriuneHipError is raised.
 from __future__ import annotations
 
 import ctypes
+import functools
 from pathlib import Path
 
 import torch
@@ -45,6 +46,10 @@ def _bind(lib):
         "triune_hip_set_output_kernel_events": ([_vp, _vp], _i),
         "triune_hip_gla_decode_step": (
             [_vp, _vp, _vp, _vp, _i, _i, _i64p, _vp, _vp, _vp, _i64, _vp, _i, _i64, _i64, _i, _i, _vp],
+            _i,
+        ),
+        "triune_hip_gla_decode_step_count": (
+            [_vp, _vp, _vp, _vp, _i, _i, _i64p, _vp, _vp, _vp, _i64, _vp, _vp, _i, _i64, _i64, _i, _i, _vp],
             _i,
         ),
         "triune_hip_last_error": ([], _i),
@@ -107,6 +112,10 @@ def _bind(lib):
             [_vp, _i, _i64p, _vp, _vp, _i, _i, _vp, _i, _vp, _i64, _vp, _i, _i64p, _i64, _i64, _i, _vp],
             _i,
         ),
+        "triune_hip_gla_fused_decode_step_slots_count": (
+            [_vp, _i, _i64p, _vp, _vp, _i, _i, _vp, _i, _vp, _i64, _vp, _vp, _i, _i64p, _i64, _i64, _i, _vp],
+            _i,
+        ),
         "triune_hip_gdn_prefill_chunked_workspace_size": ([_i64, _i64, _i64, _i, _i], _sz),
         "triune_hip_gdn_prefill_chunked": (
             [_vp, _vp, _vp, _vp, _i, _i, _vp, _i, _i, _i64p, _vp, _vp, _i, _vp, _i64, _i64, _i64, _i, _i, _vp, _sz,
@@ -144,6 +153,7 @@ EXPORTS = (
     "triune_hip_error_string",
     "triune_hip_set_output_kernel_events",
     "triune_hip_gla_decode_step",
+    "triune_hip_gla_decode_step_count",
     "triune_hip_last_error",
     "launch_gla_decode_step",
     "triune_gla_recurrent_step_f32",
@@ -175,6 +185,7 @@ EXPORTS = (
     "triune_hip_gla_qkvg_prep",
     "triune_hip_gla_fused_decode_step",
     "triune_hip_gla_fused_decode_step_slots",
+    "triune_hip_gla_fused_decode_step_slots_count",
 )
 
 
@@ -206,29 +217,47 @@ def dtype_code(t: torch.Tensor) -> int:
 
 
 def ptr(t: torch.Tensor | None):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
-def strides(*pairs) -> ctypes.Array:
+@functools.lru_cache(maxsize=1024)
+def _stride_array(*pairs) -> ctypes.Array:
     flat = [int(s) for p in pairs for s in p]
     return (ctypes.c_int64 * len(flat))(*flat)
 
 
-def stream_of(t: torch.Tensor):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+def strides(*pairs) -> ctypes.Array:
+    """The strides of several tensors as one int64 array.  The library only reads it, so calls of one
+    layout share the array."""
+    return _stride_array(*map(tuple, pairs))
+
+
+def stream_of(t: torch.Tensor) -> int:
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
+
+
+@functools.lru_cache(maxsize=1024)
+def _plan(device_index: int, name: str, *args) -> int:
+    return int(getattr(lib(), name)(*args))
+
+
+def plan(t: torch.Tensor, name: str, *args) -> int:
+    """The value of one of the library's size or support queries (a function of its arguments and of
+    the device) for a call on t's device."""
+    return _plan(t.get_device(), name, *args)
 
 
 _CTRL: dict = {}
 
 
-def onepass_ctrl(device: torch.device, nbytes: int) -> torch.Tensor:
-    """The control block of triune_hip_gla_prefill_onepass for calls on the current stream of
-    `device`: zero when first made, left ready for the next call by every call, one per (device,
+def onepass_ctrl(t: torch.Tensor, nbytes: int) -> torch.Tensor:
+    """The control block of triune_hip_gla_prefill_onepass for calls on the current stream of t's
+    device: zero when first made, left ready for the next call by every call, one per (device,
     stream) so that calls on different streams never share one.  Grown (as a new zeroed block)
     when a call needs more flags than the block holds."""
-    key = (device.index, torch.cuda.current_stream(device).cuda_stream)
+    key = (t.get_device(), stream_of(t))
     blk = _CTRL.get(key)
     if blk is None or blk.numel() < nbytes:
-        blk = torch.zeros(max(int(nbytes), 4096), device=device, dtype=torch.uint8)
+        blk = torch.zeros(max(int(nbytes), 4096), device=t.device, dtype=torch.uint8)
         _CTRL[key] = blk
     return blk

@@ -231,6 +231,16 @@ int triune_hip_gla_decode_step(const void* q, const void* k, const void* v, cons
                                int g_dtype, const int64_t* strides, const float* state_in, float* state_out,
                                const int32_t* slots, int64_t n_state_rows, void* o, int o_dtype, int64_t B,
                                int64_t H, int Dk, int Dv, void* stream) {
+    return triune_hip_gla_decode_step_count(q, k, v, g, io_dtype, g_dtype, strides, state_in, state_out, slots,
+                                            n_state_rows, nullptr, o, o_dtype, B, H, Dk, Dv, stream);
+}
+
+int triune_hip_gla_decode_step_count(const void* q, const void* k, const void* v, const void* g, int io_dtype,
+                                     int g_dtype, const int64_t* strides, const float* state_in, float* state_out,
+                                     const int32_t* slots, int64_t n_state_rows, int64_t* offsets, void* o,
+                                     int o_dtype, int64_t B, int64_t H, int Dk, int Dv, void* stream) {
+    if (offsets && !slots) return TRIUNE_ERR_NULL;
+    if (reinterpret_cast<uintptr_t>(offsets) % 8) return TRIUNE_ERR_LAYOUT;
     if (!q || !k || !v || !g || !strides || !state_in || !state_out || !o) return TRIUNE_ERR_NULL;
     if (!dtype_ok(io_dtype) || !dtype_ok(g_dtype) || !dtype_ok(o_dtype)) return TRIUNE_ERR_DTYPE;
     if (B < 0 || H <= 0 || n_state_rows < 0) return TRIUNE_ERR_SHAPE;
@@ -254,6 +264,7 @@ int triune_hip_gla_decode_step(const void* q, const void* k, const void* v, cons
     a.g_sb = strides[6]; a.g_sh = strides[7];
     a.o_sb = strides[8]; a.o_sh = strides[9];
     a.state_in = state_in; a.state_out = state_out; a.slots = slots; a.n_state_rows = n_state_rows;
+    a.offsets = offsets;
     a.o = o; a.B = B; a.H = H;
     return launch_status(launch_gla_decode(a, Dk, Dv, 4 * device_cus(), (hipStream_t)stream));
 }
@@ -1343,6 +1354,18 @@ int triune_hip_gla_fused_decode_step_slots(const void* qkvg, int io_dtype, const
                                            int state_dtype, const int32_t* slots, int64_t n_slots, void* o,
                                            int o_dtype, const int64_t* o_strides, int64_t B, int64_t H, int HD,
                                            void* stream) {
+    return triune_hip_gla_fused_decode_step_slots_count(qkvg, io_dtype, strides, cos, sin, cs_dtype, use_rope,
+                                                        state_pool, state_dtype, slots, n_slots, nullptr, o, o_dtype,
+                                                        o_strides, B, H, HD, stream);
+}
+
+int triune_hip_gla_fused_decode_step_slots_count(const void* qkvg, int io_dtype, const int64_t* strides,
+                                                 const void* cos, const void* sin, int cs_dtype, int use_rope,
+                                                 void* state_pool, int state_dtype, const int32_t* slots,
+                                                 int64_t n_slots, int64_t* offsets, void* o, int o_dtype,
+                                                 const int64_t* o_strides, int64_t B, int64_t H, int HD,
+                                                 void* stream) {
+    if (reinterpret_cast<uintptr_t>(offsets) % 8) return TRIUNE_ERR_LAYOUT;
     if (!qkvg || !strides || !o || !o_strides || !state_pool || !slots || (use_rope && (!cos || !sin)))
         return TRIUNE_ERR_NULL;
     if (!dtype_ok(io_dtype) || !dtype_ok(o_dtype) || !dtype_ok(state_dtype)) return TRIUNE_ERR_DTYPE;
@@ -1363,6 +1386,7 @@ int triune_hip_gla_fused_decode_step_slots(const void* qkvg, int io_dtype, const
     a.has_init = 1; a.save_final = 1;
     a.state_in = state_pool; a.state_out = state_pool;
     a.slots = slots; a.n_state_rows = n_slots;
+    a.offsets = offsets;
     a.o = o; a.o_dt = o_dtype; a.o_sb = o_strides[0]; a.o_sh = o_strides[1];
     a.B = B; a.H = H; a.max_blocks = kFusedDecodeBlocksPerCU * device_cus();
     return launch_status(

@@ -112,6 +112,7 @@ __global__ __launch_bounds__(DK * DV / (4 * RPT)) void gla_decode_kernel(DecodeP
 #pragma unroll
             for (int m = 0; m < RPT; ++m) __builtin_nontemporal_store(y[m], reinterpret_cast<f32x4*>(sout + m * DV));
         }
+        if (a.offsets && srow >= 0 && tid == 0 && row % H32 == 0) count_token(a.offsets, srow, a.H);
         // reduce over the row groups of a wave (lanes tid ^ CG*2^k share a column group) ...
 #pragma unroll
         for (int c = 0; c < 4; ++c) o4[c] = xor_group_sum<CG>(o4[c]);

@@ -355,6 +355,7 @@ __global__ __launch_bounds__(FusedDecodeTiling<HD>::TPB) void gla_fused_decode_k
                 __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), ro, voff + m * HD * SB, 0, 2);
             }
         }
+        if (a.offsets && h == 0 && sr >= 0 && tid == 0) count_token(a.offsets, sr, a.H);
 #pragma unroll
         for (int c = 0; c < 4; ++c) o4[c] = xor_group_sum<CG>(o4[c]);
         if (lane < CG) red[buf][wave][cg] = f32x4{o4[0], o4[1], o4[2], o4[3]};

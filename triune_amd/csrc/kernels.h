@@ -118,6 +118,7 @@ struct DecodeParams {
     float* state_out;       // may equal state_in
     const int32_t* slots;   // optional: state row of batch b is slots[b] (state pool), or null
     int64_t n_state_rows;   // rows of state_in / state_out; a slot outside [0, n_state_rows) is skipped
+    int64_t* offsets;       // optional, with slots: offsets[slots[b]] += 1 for slots of the pool
     void* o;
     int64_t B, H;
 };
@@ -214,6 +215,7 @@ struct FusedDecodeParams {
     // state_out; a slot outside [0, n_state_rows) reads no state, stores none and outputs zeros.
     const int32_t* slots;
     int64_t n_state_rows;
+    int64_t* offsets;  // optional, with slots: offsets[slots[b]] += 1 for slots of the pool
 };
 
 // Control block of the single-launch prefill (gla_onepass.hip): hdr[0] epoch, hdr[1] workgroups of
@@ -228,6 +230,12 @@ struct OnePassCtl {
     int64_t npair;  // chunk pairs per sequence: ceil(nch / 2), one workgroup each
     int64_t nh8;    // (sequence, head) pairs per XCD: ceil(B * H / 8)
 };
+
+// Head 0 of a decode step counts its session's token: srow = slot * H.
+__device__ __forceinline__ void count_token(int64_t* offsets, int64_t srow, int64_t H) {
+    __hip_atomic_fetch_add(reinterpret_cast<unsigned long long*>(offsets) + srow / H, 1ull, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+}
 
 hipError_t launch_recurrent_scan(const ScanParams& a, hipStream_t stream);
 hipError_t launch_recurrent_scan_bwd(const ScanBwdParams& a, hipStream_t stream);

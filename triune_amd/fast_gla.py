@@ -13,11 +13,13 @@ Differences from the reference, by design:
 
 from __future__ import annotations
 
+import functools
+
 import torch
 import torch.nn.functional as F
 
 from . import _lib
-from ._lib import TriuneHipError, check, dtype_code, lib, onepass_ctrl, ptr, stream_of, strides
+from ._lib import TriuneHipError, check, dtype_code, lib, onepass_ctrl, plan, ptr, stream_of, strides
 
 __all__ = [
     "fast_chunk_gla",
@@ -59,6 +61,7 @@ def _round_dk(d: int) -> int:
     raise ValueError(f"key head dim {d} > 128 is not supported")
 
 
+@functools.lru_cache(maxsize=256)
 def _pair(dk: int, dv: int, pairs=_PAIRS) -> tuple[int, int]:
     """Smallest supported (Dk, Dv) >= (dk, dv); inputs are zero-padded up to it."""
     best = None
@@ -74,11 +77,14 @@ def _vec_ok(x: torch.Tensor, tok_dim: int | None = None) -> bool:
     """Unit innermost stride and 16-byte aligned rows; tok_dim: the token axis of a token tensor
     ([B, T, H, D]: 1, packed [N, H, D]: 0), whose stride must also be at least the row width (the
     chunk kernels read a sequence's rows only up to its last token, so rows must not overlap)."""
-    m = 4 if x.dtype == torch.float32 else 8
-    ok = x.stride(-1) == 1 and x.data_ptr() % 16 == 0 and all(s % m == 0 for s in x.stride()[:-1])
-    if ok and tok_dim is not None and x.shape[tok_dim] > 1 and x.stride(tok_dim) < x.shape[-1]:
-        ok = False
-    return ok
+    st = x.stride()
+    m = 3 if x.dtype == torch.float32 else 7
+    if st[-1] != 1 or x.data_ptr() & 15:
+        return False
+    for s in st[:-1]:
+        if s & m:
+            return False
+    return tok_dim is None or st[tok_dim] >= x.shape[-1] or x.shape[tok_dim] <= 1
 
 
 def _vec_layout(x: torch.Tensor, tok_dim: int | None = None) -> torch.Tensor:
@@ -93,7 +99,8 @@ def _pad_last(x: torch.Tensor, d: int) -> torch.Tensor:
 def _state_in(s: torch.Tensor | None, dk: int, dv: int) -> torch.Tensor | None:
     if s is None:
         return None
-    s = s.to(torch.float32)
+    if s.dtype != torch.float32:
+        s = s.to(torch.float32)
     if s.shape[-2] != dk or s.shape[-1] != dv:
         s = F.pad(s, (0, dv - s.shape[-1], 0, dk - s.shape[-2]))
     return s.contiguous()
@@ -108,7 +115,7 @@ def _check_io(q, k, v, g):
 
 
 def _tok3(x: torch.Tensor):
-    return (x.stride(0), x.stride(1), x.stride(2))
+    return x.stride()[:3]
 
 
 # ---------------------------------------------------------------------------------------
@@ -164,12 +171,12 @@ def _prefill(q, k, v, g, initial_state, out, flags, save_final=True, out_dtype=N
     sf = torch.empty(B, H, Dk, Dv, device=q.device, dtype=torch.float32) if save_final else None
     L = lib()
     st = strides(_tok3(qp), _tok3(kp), _tok3(vp), _tok3(gp), _tok3(o))
-    if ONEPASS and Dk == Dv == 64 and L.triune_hip_gla_prefill_onepass_supported(
-            B, T, H, 64, dtype_code(qp), dtype_code(gp), 0, flags):
+    if ONEPASS and Dk == Dv == 64 and plan(q, "triune_hip_gla_prefill_onepass_supported", B, T, H, 64, dtype_code(qp),
+                                           dtype_code(gp), 0, flags):
         # few chunks: states and outputs in one launch (triune_hip_gla_prefill_onepass)
-        ws = torch.empty(int(L.triune_hip_gla_prefill_onepass_workspace_size(B, T, H, 64)), device=q.device,
+        ws = torch.empty(plan(q, "triune_hip_gla_prefill_onepass_workspace_size", B, T, H, 64), device=q.device,
                          dtype=torch.uint8)
-        ctrl = onepass_ctrl(q.device, int(L.triune_hip_gla_prefill_onepass_ctrl_size(B, T, H, 64)))
+        ctrl = onepass_ctrl(q, plan(q, "triune_hip_gla_prefill_onepass_ctrl_size", B, T, H, 64))
         rc = L.triune_hip_gla_prefill_onepass(
             ptr(qp), ptr(kp), ptr(vp), ptr(gp), dtype_code(qp), dtype_code(gp), st, None, None, 0, 0, 0, ptr(s0),
             ptr(o), dtype_code(o), ptr(sf), B, T, H, 64, flags, ptr(ws), ws.numel(), ptr(ctrl), ctrl.numel(),
@@ -177,8 +184,8 @@ def _prefill(q, k, v, g, initial_state, out, flags, save_final=True, out_dtype=N
         )
         check(rc, "triune_hip_gla_prefill_onepass")
     else:
-        wsb = L.triune_hip_gla_prefill_workspace_size(B, T, H, Dk, Dv, flags)
-        ws = torch.empty(max(int(wsb), 256), device=q.device, dtype=torch.uint8)
+        wsb = plan(q, "triune_hip_gla_prefill_workspace_size", B, T, H, Dk, Dv, flags)
+        ws = torch.empty(max(wsb, 256), device=q.device, dtype=torch.uint8)
         rc = L.triune_hip_gla_prefill(
             ptr(qp), ptr(kp), ptr(vp), ptr(gp), dtype_code(qp), dtype_code(gp), st, ptr(s0), ptr(o), dtype_code(o),
             ptr(sf), B, T, H, Dk, Dv, flags, ptr(ws), ws.numel(), stream_of(q),
@@ -203,6 +210,12 @@ def gla_decode_step(q, k, v, g, state, out=None, *, inplace=False, slots=None, o
     [B, H, Dk, Dv] (or a pool [N, H, Dk, Dv] addressed by int32 `slots` [B]).
     Returns (o shaped like v, state).  With inplace=True the state tensor is updated in place
     (it must then be a contiguous float32 tensor); otherwise a new state is returned."""
+    return _decode_step(q, k, v, g, state, out, inplace, slots, out_dtype, None)
+
+
+def _decode_step(q, k, v, g, state, out, inplace, slots, out_dtype, offsets):
+    """gla_decode_step that also adds one to offsets[slots[b]] (int64, one per row of the pool, or
+    None) for every slot of the pool."""
     _check_io(q, k, v, g)
     squeeze = q.dim() == 4
     if squeeze:
@@ -236,9 +249,9 @@ def gla_decode_step(q, k, v, g, state, out=None, *, inplace=False, slots=None, o
     if slots is not None:
         slots = slots.to(device=q.device, dtype=torch.int32).contiguous()
     st = strides(qp.stride()[:2], kp.stride()[:2], vp.stride()[:2], gp.stride()[:2], o.stride()[:2])
-    rc = lib().triune_hip_gla_decode_step(
+    rc = lib().triune_hip_gla_decode_step_count(
         ptr(qp), ptr(kp), ptr(vp), ptr(gp), dtype_code(qp), dtype_code(gp), st, ptr(s_in), ptr(s_out), ptr(slots),
-        s_in.shape[0], ptr(o), dtype_code(o), B, H, Dk, Dv, stream_of(q),
+        s_in.shape[0], ptr(offsets), ptr(o), dtype_code(o), B, H, Dk, Dv, stream_of(q),
     )
     check(rc, "triune_hip_gla_decode_step")
     if not inplace and padded:
@@ -288,8 +301,8 @@ def _prefill_bwd(q, k, v, g, s0, do, ds, flags, grad_dtype=None, outs=None, acc=
         dg = torch.empty(B, T, H, D, device=q.device, dtype=grad_dtype or gp.dtype)
     ds0 = torch.empty(B, H, D, D, device=q.device, dtype=torch.float32) if s0 is not None else None
     L = lib()
-    wsb = L.triune_hip_gla_prefill_bwd_workspace_size(B, max(T, 1), H, D, D, flags)
-    ws = torch.empty(max(int(wsb), 256), device=q.device, dtype=torch.uint8)
+    wsb = plan(q, "triune_hip_gla_prefill_bwd_workspace_size", B, max(T, 1), H, D, D, flags)
+    ws = torch.empty(max(wsb, 256), device=q.device, dtype=torch.uint8)
     st = strides(_tok3(qp), _tok3(kp), _tok3(vp), _tok3(gp), _tok3(dop), _tok3(dq), _tok3(dk), _tok3(dv), _tok3(dg))
     rc = L.triune_hip_gla_prefill_bwd(
         ptr(qp), ptr(kp), ptr(vp), ptr(gp), dtype_code(qp), dtype_code(gp), ptr(dop), st, ptr(s0p), ptr(dsf),
@@ -726,8 +739,8 @@ def _gdn_bwd_chunked(q, k, v, g, beta, beta_kind, do, ds, Dk0, Dv0, D):
     dg = torch.empty((B, T, H) if head else (B, T, H, D), device=q.device, dtype=g.dtype)
     db = None if beta is None else torch.empty(B, T, H, device=q.device, dtype=beta.dtype)
     L = lib()
-    wsb = L.triune_hip_gdn_bwd_chunked_workspace_size(B, T, H, D, D)
-    ws = torch.empty(max(int(wsb), 16), device=q.device, dtype=torch.uint8)
+    wsb = plan(q, "triune_hip_gdn_bwd_chunked_workspace_size", B, T, H, D, D)
+    ws = torch.empty(max(wsb, 16), device=q.device, dtype=torch.uint8)
     st = strides(_tok3(q), _tok3(k), _tok3(v), _tok3(gp), (0, 0, 0) if beta is None else _tok3(beta),
                  _tok3(dop) if dop is not None else (0, 0, 0))
     rc = L.triune_hip_gdn_bwd_chunked(
@@ -795,8 +808,8 @@ def _gdn_fwd(q, k, v, g, beta, initial_state, beta_kind, out_dtype=None):
     sf = torch.empty(B, H, D, D, device=q.device, dtype=torch.float32)
     st = strides(_tok3(qp), _tok3(kp), _tok3(vp), _tok3(gp), bst, _tok3(o))
     if scalar:
-        ws_bytes = lib().triune_hip_gdn_prefill_scalar_decay_workspace_size(B, T, H, D, D)
-        ws = torch.empty(max(int(ws_bytes), 16), device=q.device, dtype=torch.uint8)
+        ws_bytes = plan(q, "triune_hip_gdn_prefill_scalar_decay_workspace_size", B, T, H, D, D)
+        ws = torch.empty(max(ws_bytes, 16), device=q.device, dtype=torch.uint8)
         rc = lib().triune_hip_gdn_prefill_scalar_decay(
             ptr(qp), ptr(kp), ptr(vp), ptr(gp), dtype_code(qp), dtype_code(gp), ptr(bp),
             dtype_code(bp) if bp is not None else 0, beta_kind, st, ptr(s0), ptr(o), dtype_code(o), ptr(sf),
@@ -804,8 +817,8 @@ def _gdn_fwd(q, k, v, g, beta, initial_state, beta_kind, out_dtype=None):
         )
         check(rc, "triune_hip_gdn_prefill_scalar_decay")
     elif chunked:
-        ws_bytes = lib().triune_hip_gdn_prefill_chunked_workspace_size(B, T, H, D, D)
-        ws = torch.empty(max(int(ws_bytes), 16), device=q.device, dtype=torch.uint8)
+        ws_bytes = plan(q, "triune_hip_gdn_prefill_chunked_workspace_size", B, T, H, D, D)
+        ws = torch.empty(max(ws_bytes, 16), device=q.device, dtype=torch.uint8)
         rc = lib().triune_hip_gdn_prefill_chunked(
             ptr(qp), ptr(kp), ptr(vp), ptr(gp), dtype_code(qp), dtype_code(gp), ptr(bp),
             dtype_code(bp) if bp is not None else 0, beta_kind, st, ptr(s0), ptr(o), dtype_code(o), ptr(sf),

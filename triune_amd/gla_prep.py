@@ -24,7 +24,8 @@ from __future__ import annotations
 
 import torch
 
-from ._lib import check, dtype_code, lib, onepass_ctrl, ptr, stream_of, strides
+from . import fast_gla as _fg
+from ._lib import check, dtype_code, lib, onepass_ctrl, plan, ptr, stream_of, strides
 
 __all__ = ["fused_qkv_g_prep_inplace", "fused_qkvg_decode_step", "fused_qkvg_decode_step_pool",
            "fused_qkv_g_prep_chunk_gla"]
@@ -143,39 +144,46 @@ def fused_qkvg_decode_step_pool(qkvg: torch.Tensor, state_pool: torch.Tensor, sl
     qkvg.dtype; slots: int32 [B] on the device, batch row b updating pool row slots[b].  A slot
     outside [0, n_slots) (a padded batch row) reads no state, stores none and outputs zeros.
     Returns the output [B, 1, H, HD] in qkvg.dtype."""
+    return _fused_decode_pool(qkvg, state_pool, slots, cos, sin, use_rope, out, None)
+
+
+def _fused_decode_pool(qkvg, state_pool, slots, cos, sin, use_rope, out, offsets):
+    """fused_qkvg_decode_step_pool that also adds one to offsets[slots[b]] (int64, one per pool row,
+    or None) for every slot of the pool."""
     _cuda(qkvg, cos, sin, state_pool, slots)
     if qkvg.dim() != 4 or qkvg.shape[1] != 4:
         raise ValueError("qkvg must be [B, 4, H, HD]")
     B, _, H, HD = qkvg.shape
+    xst = qkvg.stride()
     if HD not in _HD:
         raise ValueError(f"head dim {HD} not supported (32, 64 or 128)")
-    if qkvg.stride(-1) != 1:
+    if xst[3] != 1:
         raise ValueError("the head dim of qkvg must be contiguous")
-    if state_pool.dim() != 4 or tuple(state_pool.shape[1:]) != (H, HD, HD) or not state_pool.is_contiguous():
+    if state_pool.dim() != 4 or state_pool.shape[1:] != (H, HD, HD) or not state_pool.is_contiguous():
         raise ValueError(f"state_pool must be a contiguous [n_slots, {H}, {HD}, {HD}] tensor")
-    if state_pool.dtype not in (torch.float32, qkvg.dtype):
+    dtype = qkvg.dtype
+    if state_pool.dtype not in (torch.float32, dtype):
         raise TypeError("the state dtype must be float32 or the dtype of qkvg")
-    if slots.dtype != torch.int32 or slots.dim() != 1 or slots.numel() != B:
+    if slots.dtype != torch.int32 or slots.dim() != 1 or slots.shape[0] != B:
         raise ValueError("slots must be an int32 [B] tensor")
     slots = slots.contiguous()
     cs_dt = 0
     if use_rope:
         if cos is None or sin is None:
             raise ValueError("use_rope needs cos and sin")
-        cos, sin = cos.reshape(-1), sin.reshape(-1)
         if cos.numel() != HD or sin.numel() != HD or cos.dtype != sin.dtype:
             raise ValueError("cos and sin must hold HD values of one dtype")
         cos, sin = cos.contiguous(), sin.contiguous()
         cs_dt = dtype_code(cos)
     if out is None:
-        out = torch.empty(B, 1, H, HD, device=qkvg.device, dtype=qkvg.dtype)
-    if tuple(out.shape) != (B, 1, H, HD) or out.stride(-1) != 1:
+        out = torch.empty(B, 1, H, HD, device=qkvg.device, dtype=dtype)
+    ost = out.stride()
+    if out.shape != (B, 1, H, HD) or ost[3] != 1:
         raise ValueError("out must be [B, 1, H, HD] with a contiguous head dim")
-    ov = out[:, 0]
-    rc = lib().triune_hip_gla_fused_decode_step_slots(
-        ptr(qkvg), dtype_code(qkvg), strides(qkvg.stride()[:3]), ptr(cos) if use_rope else None,
+    rc = lib().triune_hip_gla_fused_decode_step_slots_count(
+        ptr(qkvg), dtype_code(qkvg), strides(xst[:3]), ptr(cos) if use_rope else None,
         ptr(sin) if use_rope else None, cs_dt, 1 if use_rope else 0, ptr(state_pool), dtype_code(state_pool),
-        ptr(slots), state_pool.shape[0], ptr(ov), dtype_code(ov), strides(ov.stride()[:2]), B, H, HD,
+        ptr(slots), state_pool.shape[0], ptr(offsets), ptr(out), dtype_code(out), strides((ost[0], ost[2])), B, H, HD,
         stream_of(qkvg),
     )
     check(rc, "triune_hip_gla_fused_decode_step_slots")
@@ -218,32 +226,30 @@ def fused_qkv_g_prep_chunk_gla(qkv: torch.Tensor, g: torch.Tensor, cos=None, sin
         raise ValueError(f"head dim {HD} not supported (32, 64 or 128)")
     if qkv.dtype not in (torch.bfloat16, torch.float16) or g.dtype != qkv.dtype:
         raise TypeError("qkv and g must share one 16-bit dtype (bfloat16 or float16)")
-    from .fast_gla import _tok3, _triton_chunk_gla_tc_fwd, _vec_layout
-
-    from . import fast_gla as _fg
-
-    L = lib()
-    onepass = _fg.ONEPASS and HD == 64 and bool(
-        L.triune_hip_gla_prefill_onepass_supported(B, T, H, HD, dtype_code(qkv), dtype_code(qkv), 1, 0))
-    cus = torch.cuda.get_device_properties(qkv.device).multi_processor_count
-    if not onepass and B * H * ((T + 63) // 64) > FUSED_MAX_CHUNK_HEADS_PER_CU * cus:
-        fused_qkv_g_prep_inplace(qkv, g, cos, sin, use_rope=use_rope)
-        return _triton_chunk_gla_tc_fwd(qkv[:, :, 0], qkv[:, :, 1], qkv[:, :, 2], g, initial_state=initial_state,
-                                        out=g if out is None else out, save_final=save_final)
-    views = [qkv[:, :, 0], qkv[:, :, 1], qkv[:, :, 2], g]
+    dt = dtype_code(qkv)
+    onepass = _fg.ONEPASS and HD == 64 and plan(qkv, "triune_hip_gla_prefill_onepass_supported", B, T, H, HD, dt, dt, 1,
+                                                0)
+    if not onepass:
+        cus = torch.cuda.get_device_properties(qkv.device).multi_processor_count
+        if B * H * ((T + 63) // 64) > FUSED_MAX_CHUNK_HEADS_PER_CU * cus:
+            fused_qkv_g_prep_inplace(qkv, g, cos, sin, use_rope=use_rope)
+            return _fg._triton_chunk_gla_tc_fwd(*(qkv.select(2, i) for i in range(3)), g, initial_state=initial_state,
+                                                out=g if out is None else out, save_final=save_final)
+    _tok3, _vec_layout = _fg._tok3, _fg._vec_layout
+    views = (*(qkv.select(2, i) for i in range(3)), g)
     q, k, v, gp = (_vec_layout(x, 1) for x in views)  # copies only for unaligned layouts
     if out is None:
         out = g
     if tuple(out.shape) != (B, T, H, HD):
         raise ValueError("out must be [B, T, H, HD]")
-    o = out if _vec_layout(out, 1) is out else torch.empty(B, T, H, HD, device=qkv.device, dtype=out.dtype)
+    o = out if _fg._vec_ok(out, 1) else torch.empty(B, T, H, HD, device=qkv.device, dtype=out.dtype)
     cs_st = 0
     if use_rope:
         if cos is None or sin is None:
             raise ValueError("use_rope needs cos and sin")
         if tuple(cos.shape) != (T, HD) or tuple(sin.shape) != (T, HD):
             raise ValueError("cos and sin must be [T, HD]")
-        cos, sin = (_vec_layout(x.to(torch.float32), 0) for x in (cos, sin))
+        cos, sin = (_vec_layout(x if x.dtype == torch.float32 else x.to(torch.float32), 0) for x in (cos, sin))
         if cos.stride(0) != sin.stride(0):
             sin = sin.contiguous()
             cos = cos.contiguous()
@@ -252,19 +258,19 @@ def fused_qkv_g_prep_chunk_gla(qkv: torch.Tensor, g: torch.Tensor, cos=None, sin
     sf = torch.empty(B, H, HD, HD, device=qkv.device, dtype=torch.float32) if save_final else None
     st = strides(_tok3(q), _tok3(k), _tok3(v), _tok3(gp), _tok3(o))
     if onepass:  # pre-processing, states and outputs in one launch
-        ws = torch.empty(int(L.triune_hip_gla_prefill_onepass_workspace_size(B, T, H, HD)), device=qkv.device,
+        ws = torch.empty(plan(qkv, "triune_hip_gla_prefill_onepass_workspace_size", B, T, H, HD), device=qkv.device,
                          dtype=torch.uint8)
-        ctrl = onepass_ctrl(qkv.device, int(L.triune_hip_gla_prefill_onepass_ctrl_size(B, T, H, HD)))
-        rc = L.triune_hip_gla_prefill_onepass(
+        ctrl = onepass_ctrl(qkv, plan(qkv, "triune_hip_gla_prefill_onepass_ctrl_size", B, T, H, HD))
+        rc = lib().triune_hip_gla_prefill_onepass(
             ptr(q), ptr(k), ptr(v), ptr(gp), dtype_code(q), dtype_code(gp), st, ptr(cos) if use_rope else None,
             ptr(sin) if use_rope else None, cs_st, 1, 1 if use_rope else 0, ptr(s0), ptr(o), dtype_code(o), ptr(sf),
             B, T, H, HD, 0, ptr(ws), ws.numel(), ptr(ctrl), ctrl.numel(), stream_of(qkv),
         )
         check(rc, "triune_hip_gla_prefill_onepass")
     else:
-        wsb = L.triune_hip_gla_prefill_workspace_size(B, T, H, HD, HD, 0)
-        ws = torch.empty(max(int(wsb), 256), device=qkv.device, dtype=torch.uint8)
-        rc = L.triune_hip_gla_prefill_prep(
+        wsb = plan(qkv, "triune_hip_gla_prefill_workspace_size", B, T, H, HD, HD, 0)
+        ws = torch.empty(max(wsb, 256), device=qkv.device, dtype=torch.uint8)
+        rc = lib().triune_hip_gla_prefill_prep(
             ptr(q), ptr(k), ptr(v), ptr(gp), dtype_code(q), st, ptr(cos) if use_rope else None,
             ptr(sin) if use_rope else None, cs_st, 1 if use_rope else 0, ptr(s0), ptr(o), dtype_code(o), ptr(sf),
             B, T, H, HD, ptr(ws), ws.numel(), stream_of(qkv),

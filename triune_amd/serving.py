@@ -26,8 +26,8 @@ from typing import Any, Dict, List, Optional, Tuple
 
 import torch
 
-from .fast_gla import _DECODE_PAIRS, fast_chunk_gla_varlen, gla_decode_step
-from .gla_prep import fused_qkvg_decode_step_pool
+from .fast_gla import _DECODE_PAIRS, _decode_step, fast_chunk_gla_varlen, gla_decode_step
+from .gla_prep import _fused_decode_pool
 
 __all__ = [
     "parse_cache",
@@ -110,7 +110,8 @@ class StateSlotPool:
     offset).  Sessions map to slots in LRU order with a time-to-live, as in the reference's
     SessionRecurrentStateManager (srsm.py:11-112), whose get / update / clear / stats interface
     this class keeps; a new session's slot starts from a zero state.  Thread-safe for the
-    bookkeeping; kernel calls follow the caller's stream order.
+    bookkeeping; kernel calls follow the caller's stream order.  The decode kernels count the tokens
+    themselves (the count as separate tensor operations took seven launches, 40 us of host time).
 
     prefill() and decode_step() run only device work (the kernels and a device-side update of
     the offsets), with no host synchronisation, so a serving loop can capture them in one graph
@@ -244,9 +245,8 @@ class StateSlotPool:
 
     def decode_step(self, layer: int, q, k, v, g, slots: torch.Tensor, out=None, count_tokens: bool = True):
         """One token for each of len(slots) sessions; states updated in place in their slots."""
-        o, _ = gla_decode_step(q, k, v, g, self.states[layer], out=out, inplace=True, slots=slots)
-        if count_tokens:
-            self._count(layer, slots, torch.ones_like(slots, dtype=torch.int64))
+        o, _ = _decode_step(q, k, v, g, self.states[layer], out, True, slots, None,
+                            self.offsets[layer] if count_tokens else None)
         return o
 
     def fused_decode_step(self, layer: int, qkvg, slots: torch.Tensor, cos=None, sin=None, use_rope: bool = True,
@@ -254,10 +254,8 @@ class StateSlotPool:
         """decode_step from raw projections (qkvg [B, 4, H, HD]): VectorisedGLA's fused decode
         (attention.py:81-179; ELU+1, L2 norm, RoPE, logsigmoid, then the update) on the slots'
         states, in place."""
-        o = fused_qkvg_decode_step_pool(qkvg, self.states[layer], slots, cos, sin, use_rope=use_rope, out=out)
-        if count_tokens:
-            self._count(layer, slots, torch.ones_like(slots, dtype=torch.int64))
-        return o
+        return _fused_decode_pool(qkvg, self.states[layer], slots, cos, sin, use_rope, out,
+                                  self.offsets[layer] if count_tokens else None)
 
 
 # ---------------------------------------------------------------------------------------
