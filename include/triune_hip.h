@@ -366,11 +366,11 @@ int triune_hip_gdn_bwd(const void* q, const void* k, const void* v, const void* 
                        void* dg, void* dbeta, float* ds0, int64_t B, int64_t T, int64_t H, int Dk, int Dv,
                        void* workspace, size_t workspace_bytes, void* stream);
 
-/* triune_hip_gdn_bwd for 16-bit I/O in chunk form on the fp32 matrix cores: io_dtype bf16 or fp16,
- * dout in io_dtype, beta none or per (token, head).  With g_head != 0 the gate is one value per
+/* triune_hip_gdn_bwd for 16-bit I/O in chunk form on the matrix cores: io_dtype bf16 or fp16, g,
+ * beta and dout in io_dtype, beta none or per (token, head).  With g_head != 0 the gate is one value per
  * (token, head) (strides[9..11] of a [B, T, H] tensor) and dg is [B, T, H], the sum over the key
  * dims; otherwise g and dg are [B, T, H, D].  Other arguments as triune_hip_gdn_bwd; rows need unit
- * innermost stride only.  workspace: at least triune_hip_gdn_bwd_chunked_workspace_size(B, T, H,
+ * innermost stride and token strides of at most 2^31 / 160 elements (H D too).  workspace: at least triune_hip_gdn_bwd_chunked_workspace_size(B, T, H,
  * Dk, Dv) bytes, 16-byte aligned.
  * Replaces: autograd through fast_recurrent_gated_deltanet (fast_gla.py:781-836). */
 size_t triune_hip_gdn_bwd_chunked_workspace_size(int64_t B, int64_t T, int64_t H, int Dk, int Dv);

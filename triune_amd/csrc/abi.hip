@@ -1072,9 +1072,9 @@ int triune_hip_gdn_bwd(const void* q, const void* k, const void* v, const void* 
     return TRIUNE_OK;
 }
 
-// Chunk-form backward: per (b, h, chunk) the block-triangular tiles and three D x D matrices.
+// Chunk-form backward: per (b, h, chunk) the block-triangular tiles and four D x D matrices.
 static size_t gdn_bwd_chunked_bytes(int64_t B, int64_t T, int64_t H, int D) {
-    return (size_t)(B * H * ((T + 63) / 64)) * (3 * D * D + 20 * 256) * sizeof(float);
+    return (size_t)(B * H * ((T + 63) / 64)) * (4 * D * D + 20 * 256) * sizeof(float);
 }
 
 size_t triune_hip_gdn_bwd_chunked_workspace_size(int64_t B, int64_t T, int64_t H, int Dk, int Dv) {
@@ -1091,8 +1091,8 @@ int triune_hip_gdn_bwd_chunked(const void* q, const void* k, const void* v, cons
     if (!q || !k || !v || !g || !strides || !dq || !dk || !dv || !dg) return TRIUNE_ERR_NULL;
     if (beta_kind != TRIUNE_BETA_NONE && beta_kind != TRIUNE_BETA_HEAD) return TRIUNE_ERR_SHAPE;
     if (beta_kind != TRIUNE_BETA_NONE && (!beta || !dbeta)) return TRIUNE_ERR_NULL;
-    if ((io_dtype != TRIUNE_DT_BF16 && io_dtype != TRIUNE_DT_F16) || !dtype_ok(g_dtype) ||
-        (beta_kind != TRIUNE_BETA_NONE && !dtype_ok(beta_dtype)))
+    if ((io_dtype != TRIUNE_DT_BF16 && io_dtype != TRIUNE_DT_F16) || g_dtype != io_dtype ||
+        (beta_kind != TRIUNE_BETA_NONE && beta_dtype != io_dtype))
         return TRIUNE_ERR_DTYPE;
     if (B < 0 || T < 0 || H <= 0 || Dk != Dv || (Dk != 64 && Dk != 128)) return TRIUNE_ERR_SHAPE;
     const int D = Dk;
@@ -1100,6 +1100,12 @@ int triune_hip_gdn_bwd_chunked(const void* q, const void* k, const void* v, cons
     if (reinterpret_cast<uintptr_t>(s0) % 16 || reinterpret_cast<uintptr_t>(ds_final) % 16 ||
         reinterpret_cast<uintptr_t>(ds0) % 16 || reinterpret_cast<uintptr_t>(workspace) % 16)
         return TRIUNE_ERR_LAYOUT;
+    // 64 rows of a tensor are addressed in 32 bits
+    for (int i = 0; i < 6; ++i) {
+        const int64_t ts = i == 4 && beta_kind == TRIUNE_BETA_NONE ? 0 : (i == 5 && !dout ? 0 : strides[3 * i + 1]);
+        if (ts < 0 || ts > 0x7fffffff / 160) return TRIUNE_ERR_LAYOUT;
+    }
+    if (H > 0x7fffffff / (160 * D)) return TRIUNE_ERR_LAYOUT;
     if (B == 0) return TRIUNE_OK;
     hipStream_t st = (hipStream_t)stream;
     if (T == 0) {  // no tokens: the gradient of the initial state is that of the final state
@@ -1125,7 +1131,7 @@ int triune_hip_gdn_bwd_chunked(const void* q, const void* k, const void* v, cons
     p.nc = (T + 63) / 64;
     const int64_t n = B * H * p.nc;
     p.ws_m = reinterpret_cast<float*>(workspace);
-    p.ws_s = p.ws_m + n * D * D;
+    p.ws_s = p.ws_m + 2 * n * D * D;
     p.ws_d = p.ws_s + n * D * D;
     p.ws_t = p.ws_d + n * D * D;
     return launch_status(launch_gdn_bwd_chunk(p, D, st));

@@ -43,6 +43,7 @@ _chunked_gdn_enabled = True
 # Gradients that are all 16-bit come from the chunk-form kernels unless this is False (then from the
 # token-serial ones, which serve every other call).
 _chunked_gdn_bwd_enabled = True
+_GDN_BWD_MAX_STRIDE = 0x7fffffff // 160  # token stride (elements) the chunk-form kernels address
 # Gates with one value per (token, head) take the scalar-decay chunked kernels unless this is False
 # (then they run the per-key-dim chunked kernels on the broadcast gate).
 _scalar_gdn_enabled = True
@@ -685,7 +686,9 @@ def _gdn_bwd(q, k, v, g, beta, initial_state, beta_kind, do, ds):
     # every gradient rounded to 16 bits: the chunk form on the matrix cores
     if (beta_kind in (_lib.BETA_NONE, _lib.BETA_HEAD) and q.dtype != torch.float32 and g.dtype == q.dtype and
             (beta is None or beta.dtype == q.dtype) and (do is None or do.dtype == q.dtype) and
-            initial_state is None and _chunked_gdn_bwd_enabled):
+            initial_state is None and _chunked_gdn_bwd_enabled and
+            max(H * D, *(x.stride(1) for x in (qp, kp, vp, g, *((beta,) if beta is not None else ()),
+                                               *((do,) if do is not None else ())))) <= _GDN_BWD_MAX_STRIDE):
         return _gdn_bwd_chunked(qp, kp, vp, g, beta, beta_kind, do, ds, Dk0, Dv0, D)
     if g.dim() == 3:
         r = _gdn_bwd(q, k, v, g.unsqueeze(-1).expand(*g.shape, Dk0), beta, initial_state, beta_kind, do, ds)
