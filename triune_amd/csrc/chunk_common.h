@@ -10,7 +10,14 @@
 namespace triune {
 
 constexpr int CHUNK = 64;
-constexpr int PAD = 4;  // row padding (elements) of LDS planes: spreads rows over banks
+// Row padding (elements) of LDS planes with D bf16 elements per row: spreads rows over banks.
+//  * A row of (D + pad) / 2 words is read as row fragments (16 rows, 8 bytes each: the strides must
+//    fall on distinct bank pairs), as transposed fragments (ds_read_b64_tr_b16: 4 rows x 4 pairs per
+//    16 lanes) and written 4 rows apart.  At D = 128, 74 words (10 mod 64) satisfy all three; 66
+//    words (pad 4) put four pairs of every transposed read on one bank: a third of the D = 128
+//    state kernel's cycles went to bank conflicts.
+constexpr int PAD = 4;
+constexpr int PAD128 = 20;
 
 struct Work {
     int64_t seq, b, row0, t_begin, t_end, len;

@@ -405,7 +405,7 @@ __device__ __forceinline__ void copy_tiles(char* tiles, float* mem) {
 template <int D>
 struct MapLay {
     static constexpr int NW = D / 16;
-    static constexpr int RS = D + PAD;     // elements per plane row
+    static constexpr int RS = D + (D == 128 ? PAD128 : PAD);  // elements per plane row
     static constexpr int ROWP = GC * RS * 2;
     static constexpr int BYTES = 3 * 2 * ROWP + 2 * NTL * TLB + GC * 4;
 };
@@ -750,7 +750,7 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_scan_kernel(GdnChunkBwdParam
 template <int D, int NX>
 struct GradLay {
     static constexpr int NW = D / 16;
-    static constexpr int RS = D + PAD;
+    static constexpr int RS = D + (D == 128 ? PAD128 : PAD);
     static constexpr int ROWP = GC * RS * 2;
     static constexpr int BYTES = (2 * 2 + NX) * ROWP + 2 * NTL * TLB + 2 * NW * GC * 4;
 };

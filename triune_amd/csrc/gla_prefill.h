@@ -46,7 +46,9 @@ struct Lay {
     using P = Prec<TIn>;
     static constexpr int NW = DV / 16;             // waves per workgroup
     static constexpr int DPW = DK / NW;            // key dims per wave in stage 1
-    static constexpr int RS = DK + PAD;            // row stride (elements) of [token][dim] planes
+    // row stride (elements) of [token][dim] planes; at 128 dims the wide padding where it leaves the
+    // input tiles room (16-bit I/O with one V plane)
+    static constexpr int RS = DK + (DK == 128 && P::NX == 1 ? PAD128 : PAD);
     static constexpr int VS = 16;                  // row stride of a wave's [token][16 columns] V planes
     static constexpr int ROWP = CHUNK * RS * 2;    // bytes per [token][dim] plane
     static constexpr int VPP = CHUNK * VS * 2;     // bytes per V plane of one wave
