@@ -10,12 +10,7 @@
 namespace triune {
 
 constexpr int CHUNK = 64;
-// Row padding (elements) of LDS planes with D bf16 elements per row: spreads rows over banks.
-//  * A row of (D + pad) / 2 words is read as row fragments (16 rows, 8 bytes each: the strides must
-//    fall on distinct bank pairs), as transposed fragments (ds_read_b64_tr_b16: 4 rows x 4 pairs per
-//    16 lanes) and written 4 rows apart.  At D = 128, 74 words (10 mod 64) satisfy all three; 66
-//    words (pad 4) put four pairs of every transposed read on one bank: a third of the D = 128
-//    state kernel's cycles went to bank conflicts.
+// Row padding (elements) of LDS planes that are not swizzled (see Plane): spreads rows over banks.
 constexpr int PAD = 4;
 constexpr int PAD128 = 20;
 
@@ -149,6 +144,81 @@ __device__ __forceinline__ Split8<NP> lds_frag_tr(const char* base, int plane_by
     }
     return f;
 }
+
+// ---- swizzled planes ---------------------------------------------------------------------
+// A [64 tokens][D] plane of bf16 parts without row padding (D = 64 or 128).  Within each block of 32
+// dims the eight that a lane's K = 32 fragment takes (4 g4 + [0, 4) and 16 + 4 g4 + [0, 4)) are
+// stored together as one 16-byte unit, so a row fragment is one ds_read_b128 per part, and the units
+// of a row are permuted by an XOR with f(row):
+//  * ds_read_b128 moves 256 bytes per cycle when the 16 lanes of a cycle (8 rows x 2 units) fall on
+//    distinct bank quads, and half of that otherwise: measured 4.1 (D = 64) to 5.0 (128) cycles per
+//    wave instruction, against 9.0 at padded strides and 9.6 for the two ds_read_b64 it replaces;
+//  * a transposed read (4 rows x 4 units per 16 lanes) takes 5.6 cycles, against 5.1 at its best
+//    padded stride and 8.3 at 66 words.
+// f is linear in the row's low four bits and does not depend on its upper ones.
+template <int D>
+struct Plane {
+    static constexpr bool SWZ = D == 64 || D == 128;
+    static constexpr int RS = SWZ ? D : D + PAD;
+    static constexpr int BYTES = CHUNK * RS * 2;
+
+    __device__ __forceinline__ static int swz(int r) {
+        if constexpr (D == 128) return (((r ^ (r >> 2)) & 3) << 2) | (((r >> 2) & 1) << 1);
+        else return ((((r >> 1) ^ (r >> 2)) & 1) << 2) | (((r >> 2) & 1) << 1);
+    }
+    // element offset in its row of dims [d0, d0 + 4) (d0 a multiple of 4), for a row with f = fr
+    __device__ __forceinline__ static int unit(int d0, int fr) {
+        return 8 * ((((d0 >> 5) << 2) | ((d0 >> 2) & 3)) ^ fr) + ((d0 >> 2) & 4);
+    }
+
+    // lds_frag over dims [32 ks, 32 ks + 32) of row row0 + r16 (row0 a multiple of 16)
+    template <int NP>
+    __device__ __forceinline__ static Split8<NP> frag(const char* base, int row0, int r16, int ks, int g4) {
+        if constexpr (!SWZ) {
+            return lds_frag<NP>(base, BYTES, RS, row0 + r16, 32 * ks, g4);
+        } else {
+            Split8<NP> f;
+            const int off = (row0 + r16) * RS + 8 * ((4 * ks + g4) ^ swz(r16));
+#pragma unroll
+            for (int pl = 0; pl < NP; ++pl)
+                f.p[pl] = *reinterpret_cast<const bf16x8*>(reinterpret_cast<const __bf16*>(base + pl * BYTES) + off);
+            return f;
+        }
+    }
+    // lds_frag_tr over rows [row0, row0 + 32) (row0 a multiple of 16) of dims [16 db, 16 db + 16)
+    template <int NP>
+    __device__ __forceinline__ static Split8<NP> frag_tr(const char* base, int row0, int db, int g4, int r16) {
+        if constexpr (!SWZ) {
+            return lds_frag_tr<NP>(base, BYTES, RS, row0, 16 * db, g4, r16);
+        } else {
+            Split8<NP> f;
+            const int r = 4 * g4 + (r16 >> 2);
+            const int off = (row0 + r) * RS + 8 * ((4 * (db >> 1) + (r16 & 3)) ^ swz(r)) + 4 * (db & 1);
+#pragma unroll
+            for (int pl = 0; pl < NP; ++pl) {
+                const __bf16* p = reinterpret_cast<const __bf16*>(base + pl * BYTES) + off;
+                const bf16x4 a = lds_read_tr(p);
+                const bf16x4 b = lds_read_tr(p + 16 * RS);
+                f.p[pl] = bf16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+            }
+            return f;
+        }
+    }
+    // N (a multiple of 4) values of a row from dim d0 (a multiple of 4), split into NP parts
+    template <int NP, int N>
+    __device__ __forceinline__ static void put(char* base, int row, int d0, const float* x) {
+#pragma unroll
+        for (int c = 0; c < N; c += 4) {
+            float r[4] = {x[c], x[c + 1], x[c + 2], x[c + 3]};
+            uint32_t w[NP][2];
+            split_pairs<NP, 2>(r, w);
+            const int off = row * RS + (SWZ ? unit(d0 + c, swz(row & 15)) : d0 + c);
+#pragma unroll
+            for (int pl = 0; pl < NP; ++pl)
+                *reinterpret_cast<uint2*>(reinterpret_cast<__bf16*>(base + pl * BYTES) + off) = uint2{w[pl][0], w[pl][1]};
+        }
+    }
+};
 
 // N (multiple of 4) consecutive values at element index idx (a multiple of 4), split into NP
 // bf16 planes.

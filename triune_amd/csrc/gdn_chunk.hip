@@ -44,8 +44,9 @@ template <typename TIn, bool OUT, int D>
 struct GLay {
     using P = Prec<TIn>;
     static constexpr int DK = D, DV = D, NW = D / 16, DPW = 16, DL = 4;
-    static constexpr int RS = DK + PAD, VS = 16;
-    static constexpr int ROWP = CHUNK * RS * 2;
+    using PL = Plane<D>;  // [token][dim] planes
+    static constexpr int VS = 16;
+    static constexpr int ROWP = PL::BYTES;
     static constexpr int VPP = CHUNK * VS * 2;
     static constexpr int TILEP = 10 * 64 * 4 * 2;  // ten 16x16 tiles (causal blocks), one bf16 part
     static constexpr int LTP = 6 * 64 * 4 * 2;     // the six off-diagonal blocks of L^T
@@ -225,7 +226,7 @@ struct GdnStep {
                 for (int j = 0; j < 4; ++j) {
 #pragma unroll
                     for (int i = 0; i < DL; ++i) x[j][i] *= fq[j][i];
-                    lds_put_row<NS, DL>(sQT, L::ROWP, (4 * tg + j) * L::RS + dl0, x[j]);
+                    L::PL::template put<NS, DL>(sQT, 4 * tg + j, dl0, x[j]);
                 }
             }
             float kx[4][DL];
@@ -235,7 +236,7 @@ struct GdnStep {
             for (int j = 0; j < 4; ++j) {
 #pragma unroll
                 for (int i = 0; i < DL; ++i) x[j][i] = kx[j][i] * fast_exp(G[j][i] - Gc[j][i] - 0.5f * GC[i]);
-                lds_put_row<NS, DL>(sBT, L::ROWP, (4 * tg + j) * L::RS + dl0, x[j]);
+                L::PL::template put<NS, DL>(sBT, 4 * tg + j, dl0, x[j]);
             }
             // Wt = beta k exp(m - G)
             float bt[4];
@@ -268,7 +269,7 @@ struct GdnStep {
             for (int j = 0; j < 4; ++j) {
 #pragma unroll
                 for (int i = 0; i < DL; ++i) x[j][i] = kx[j][i] * bkx[j][i] * __builtin_amdgcn_rcpf(fq[j][i]);
-                lds_put_row<NS, DL>(sWT, L::ROWP, (4 * tg + j) * L::RS + dl0, x[j]);
+                L::PL::template put<NS, DL>(sWT, 4 * tg + j, dl0, x[j]);
             }
             // V rows of this wave's columns
             float vx[4][4];
@@ -317,8 +318,8 @@ struct GdnStep {
                 f32x4 acc = zero4();
 #pragma unroll
                 for (int ks = 0; ks < NKS; ++ks) {
-                    const Split8<NS> wf = lds_frag<NS>(sWT, L::ROWP, L::RS, 16 * sb + r16, 32 * ks, g4);
-                    const Split8<NS> rf = lds_frag<NS>(rhs, L::ROWP, L::RS, 16 * tb + r16, 32 * ks, g4);
+                    const Split8<NS> wf = L::PL::template frag<NS>(sWT, 16 * sb, r16, ks, g4);
+                    const Split8<NS> rf = L::PL::template frag<NS>(rhs, 16 * tb, r16, ks, g4);
                     acc = mfma_split<NS, NS, NS>(wf, rf, acc);
                 }
                 if (is_a && sb == tb) {  // row = s (4*g4 + j), column = t (r16): keep s <= t
@@ -336,8 +337,8 @@ struct GdnStep {
                 f32x4 Lm = zero4();
 #pragma unroll
                 for (int ks = 0; ks < NKS; ++ks) {
-                    const Split8<NS> bf = lds_frag<NS>(sBT, L::ROWP, L::RS, 16 * ib + r16, 32 * ks, g4);
-                    const Split8<NS> wf = lds_frag<NS>(sWT, L::ROWP, L::RS, 16 * ib + r16, 32 * ks, g4);
+                    const Split8<NS> bf = L::PL::template frag<NS>(sBT, 16 * ib, r16, ks, g4);
+                    const Split8<NS> wf = L::PL::template frag<NS>(sWT, 16 * ib, r16, ks, g4);
                     Lm = mfma_split<NS, NS, NS>(bf, wf, Lm);  // Lm[t = 4*g4+j][s = r16]
                 }
                 float* sL = reinterpret_cast<float*>(sTI) + ib * 256;
@@ -351,8 +352,8 @@ struct GdnStep {
                 f32x4 Lm = zero4(), LmT = zero4();
 #pragma unroll
                 for (int ks = 0; ks < NKS; ++ks) {
-                    const Split8<NS> bf = lds_frag<NS>(sBT, L::ROWP, L::RS, 16 * ib + r16, 32 * ks, g4);
-                    const Split8<NS> wf = lds_frag<NS>(sWT, L::ROWP, L::RS, 16 * ib + r16, 32 * ks, g4);
+                    const Split8<NS> bf = L::PL::template frag<NS>(sBT, 16 * ib, r16, ks, g4);
+                    const Split8<NS> wf = L::PL::template frag<NS>(sWT, 16 * ib, r16, ks, g4);
                     Lm = mfma_split<NS, NS, NS>(bf, wf, Lm);    // Lm[t = 4*g4+j][s = r16]
                     LmT = mfma_split<NS, NS, NS>(wf, bf, LmT);  // LmT[s = 4*g4+j][t = r16]
                 }
@@ -430,7 +431,7 @@ struct GdnStep {
             f32x4 p = zero4();
 #pragma unroll
             for (int ks = 0; ks < NKS; ++ks) {
-                const Split8<NS> bf = lds_frag<NS>(sBT, L::ROWP, L::RS, 16 * i + r16, 32 * ks, g4);
+                const Split8<NS> bf = L::PL::template frag<NS>(sBT, 16 * i, r16, ks, g4);
                 p = mfma_split<NS, NS, NS>(bf, sf[ks], p);
             }
             f32x4 vv = zero4();
@@ -455,7 +456,7 @@ struct GdnStep {
                 f32x4 o = zero4();
 #pragma unroll
                 for (int ks = 0; ks < NKS; ++ks) {
-                    const Split8<NS> qf = lds_frag<NS>(sQT, L::ROWP, L::RS, 16 * tb + r16, 32 * ks, g4);
+                    const Split8<NS> qf = L::PL::template frag<NS>(sQT, 16 * tb, r16, ks, g4);
                     o = mfma_split<NS, NS, NS>(sf[ks], qf, o);
                 }
                 Ot[tb] = o;
@@ -535,7 +536,7 @@ struct GdnStep {
             f32x4 acc = Sp[db];
 #pragma unroll
             for (int k2 = 0; k2 < 2; ++k2) {
-                const Split8<NS> wf = lds_frag_tr<NS>(sWT, L::ROWP, L::RS, 32 * k2, 16 * db, g4, r16);
+                const Split8<NS> wf = L::PL::template frag_tr<NS>(sWT, 32 * k2, db, g4, r16);
                 acc = mfma_split<NS, NS, NS>(wf, uf[k2], acc);
             }
             const f32x4 em = *reinterpret_cast<const f32x4*>(sEM + 16 * db + 4 * g4);

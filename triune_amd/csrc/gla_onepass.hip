@@ -339,13 +339,13 @@ __global__ __launch_bounds__(OP_THREADS, 1) void gla_onepass_kernel(PrefillParam
         for (int j = 0; j < 4; ++j) {
 #pragma unroll
             for (int i = 0; i < DL; ++i) x[j][i] *= G[j][i];
-            lds_put_row<NS, DL>(sQT, L::ROWP, (4 * tg + j) * L::RS + dl0, x[j]);
+            L::PL::template put<NS, DL>(sQT, 4 * tg + j, dl0, x[j]);
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
 #pragma unroll
             for (int i = 0; i < DL; ++i) y[j][i] *= __builtin_amdgcn_rcpf(G[j][i]);
-            lds_put_row<NS, DL>(sKT, L::ROWP, (4 * tg + j) * L::RS + dl0, y[j]);
+            L::PL::template put<NS, DL>(sKT, 4 * tg + j, dl0, y[j]);
         }
     } else {  // the rows as the scan reads them, staged for the token-by-token walks
         char* stg = smem + L::OFF_QT;
@@ -378,7 +378,7 @@ __global__ __launch_bounds__(OP_THREADS, 1) void gla_onepass_kernel(PrefillParam
             P[db] = zero4();
 #pragma unroll
             for (int k2 = 0; k2 < 2; ++k2) {
-                const Split8<NS> kf = lds_frag_tr<NS>(sKT, L::ROWP, L::RS, 32 * k2, 16 * db, g4, r16);
+                const Split8<NS> kf = L::PL::template frag_tr<NS>(sKT, 32 * k2, db, g4, r16);
                 P[db] = mfma_split<NS, NX, NS>(kf, vf[k2], P[db]);
             }
             const f32x4 em = *reinterpret_cast<const f32x4*>(sEM + 16 * db + 4 * g4);
@@ -460,8 +460,8 @@ __global__ __launch_bounds__(OP_THREADS, 1) void gla_onepass_kernel(PrefillParam
                 Split8<NS> kf[MT], qf[MT];
 #pragma unroll
                 for (int t = 0; t < MT; ++t) {
-                    kf[t] = lds_frag<NS>(sKT, L::ROWP, L::RS, 16 * sb[t] + r16, 32 * ks, g4);
-                    qf[t] = lds_frag<NS>(sQT, L::ROWP, L::RS, 16 * tb[t] + r16, 32 * ks, g4);
+                    kf[t] = L::PL::template frag<NS>(sKT, 16 * sb[t], r16, ks, g4);
+                    qf[t] = L::PL::template frag<NS>(sQT, 16 * tb[t], r16, ks, g4);
                 }
 #pragma unroll
                 for (int t = 0; t < MT; ++t) acc[t] = mfma_split<NS, NS, NS>(kf[t], qf[t], acc[t]);
@@ -601,7 +601,7 @@ __global__ __launch_bounds__(OP_THREADS, 1) void gla_onepass_kernel(PrefillParam
             const Split8<NS> sf = split8<NS>(xx);
 #pragma unroll
             for (int tb = 0; tb < 4; ++tb) {
-                const Split8<NS> qf = lds_frag<NS>(sQT, L::ROWP, L::RS, 16 * tb + r16, 32 * ks, g4);
+                const Split8<NS> qf = L::PL::template frag<NS>(sQT, 16 * tb, r16, ks, g4);
                 Ot[tb] = mfma_split<NS, NS, NS>(sf, qf, Ot[tb]);
             }
         }

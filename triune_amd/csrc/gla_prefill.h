@@ -46,11 +46,9 @@ struct Lay {
     using P = Prec<TIn>;
     static constexpr int NW = DV / 16;             // waves per workgroup
     static constexpr int DPW = DK / NW;            // key dims per wave in stage 1
-    // row stride (elements) of [token][dim] planes; at 128 dims the wide padding where it leaves the
-    // input tiles room (16-bit I/O with one V plane)
-    static constexpr int RS = DK + (DK == 128 && P::NX == 1 ? PAD128 : PAD);
+    using PL = Plane<DK>;                          // [token][dim] planes
     static constexpr int VS = 16;                  // row stride of a wave's [token][16 columns] V planes
-    static constexpr int ROWP = CHUNK * RS * 2;    // bytes per [token][dim] plane
+    static constexpr int ROWP = PL::BYTES;         // bytes per [token][dim] plane
     static constexpr int VPP = CHUNK * VS * 2;     // bytes per V plane of one wave
     static constexpr int ATP = 10 * 64 * 4 * 2;    // bytes per plane of the ten A^T tiles
     // K3: Qt rows, Kt rows, A^T tiles.  K1: exp-weighted k rows (in the Kt slot).
@@ -393,7 +391,7 @@ struct OutStep {
             for (int j = 0; j < 4; ++j) {
 #pragma unroll
                 for (int i = 0; i < DL; ++i) x[j][i] *= G[j][i];
-                lds_put_row<NS, DL>(sQT, L::ROWP, (4 * tg + j) * L::RS + dl0, x[j]);
+                L::PL::template put<NS, DL>(sQT, 4 * tg + j, dl0, x[j]);
             }
             // Kt rows (stage 2 reads them as rows, the state update through the transposed read)
             chunk_float<CK>(cur.k, x, tg, nv);
@@ -401,7 +399,7 @@ struct OutStep {
             for (int j = 0; j < 4; ++j) {
 #pragma unroll
                 for (int i = 0; i < DL; ++i) x[j][i] *= __builtin_amdgcn_rcpf(G[j][i]);
-                lds_put_row<NS, DL>(sKT, L::ROWP, (4 * tg + j) * L::RS + dl0, x[j]);
+                L::PL::template put<NS, DL>(sKT, 4 * tg + j, dl0, x[j]);
             }
             // V rows: tokens 4*tg + j, this wave's columns 4*row .. 4*row+3
             lds_put_v_rows<TIn, NX, CK>(sVP, L::VPP, L::VS, 4 * row, cur.v, tg, nv);
@@ -444,8 +442,8 @@ struct OutStep {
                     Split8<NS> kf[MT], qf[MT];
 #pragma unroll
                     for (int t = 0; t < MT; ++t) {
-                        kf[t] = lds_frag<NS>(sKT, L::ROWP, L::RS, 16 * sb[t] + r16, 32 * ks, g4);
-                        qf[t] = lds_frag<NS>(sQT, L::ROWP, L::RS, 16 * tb[t] + r16, 32 * ks, g4);
+                        kf[t] = L::PL::template frag<NS>(sKT, 16 * sb[t], r16, ks, g4);
+                        qf[t] = L::PL::template frag<NS>(sQT, 16 * tb[t], r16, ks, g4);
                     }
 #pragma unroll
                     for (int t = 0; t < MT; ++t) acc[t] = mfma_split<NS, NS, NS>(kf[t], qf[t], acc[t]);
@@ -487,7 +485,7 @@ struct OutStep {
                 const Split8<NS> sf = split8<NS>(x);
 #pragma unroll
                 for (int tb = 0; tb < 4; ++tb) {
-                    const Split8<NS> qf = lds_frag<NS>(sQT, L::ROWP, L::RS, 16 * tb + r16, 32 * ks, g4);
+                    const Split8<NS> qf = L::PL::template frag<NS>(sQT, 16 * tb, r16, ks, g4);
                     Ot[tb] = mfma_split<NS, NS, NS>(sf, qf, Ot[tb]);
                 }
             }
@@ -517,7 +515,7 @@ struct OutStep {
                 f32x4 P = zero4();
 #pragma unroll
                 for (int k2 = 0; k2 < 2; ++k2) {
-                    const Split8<NS> kf = lds_frag_tr<NS>(sKT, L::ROWP, L::RS, 32 * k2, 16 * db, g4, r16);
+                    const Split8<NS> kf = L::PL::template frag_tr<NS>(sKT, 32 * k2, db, g4, r16);
                     P = mfma_split<NS, NX, NS>(kf, vf[k2], P);
                 }
                 const f32x4 em = *reinterpret_cast<const f32x4*>(sEM + 16 * db + 4 * g4);
@@ -760,7 +758,7 @@ struct StateStep {
             for (int j = 0; j < 4; ++j) {
 #pragma unroll
                 for (int i = 0; i < DL; ++i) y[j][i] *= __builtin_amdgcn_exp2f(fmaf(X[j][i], LOG2E, gs[i]));
-                lds_put_row<NS, DL>(sKW, L::ROWP, (4 * tg + j) * L::RS + dl0, y[j]);
+                L::PL::template put<NS, DL>(sKW, 4 * tg + j, dl0, y[j]);
             }
 #pragma unroll
             for (int i = 0; i < DL; ++i) Gseg[i] += GC[i];
@@ -784,7 +782,7 @@ struct StateStep {
             for (int j = 0; j < 4; ++j) {
 #pragma unroll
                 for (int i = 0; i < DL; ++i) x[j][i] *= __builtin_amdgcn_exp2f(fmaf(X[j][i], LOG2E, gs[i]));
-                lds_put_row<NS, DL>(sKW, L::ROWP, (4 * tg + j) * L::RS + dl0, x[j]);
+                L::PL::template put<NS, DL>(sKW, 4 * tg + j, dl0, x[j]);
             }
 #pragma unroll
             for (int i = 0; i < DL; ++i) Gseg[i] += GC[i];
@@ -799,7 +797,7 @@ struct StateStep {
         for (int db = 0; db < NDB; ++db)
 #pragma unroll
             for (int k2 = 0; k2 < 2; ++k2) {
-                const Split8<NS> kf = lds_frag_tr<NS>(sKW, L::ROWP, L::RS, 32 * k2, 16 * db, g4, r16);
+                const Split8<NS> kf = L::PL::template frag_tr<NS>(sKW, 32 * k2, db, g4, r16);
                 Lst[db] = mfma_split<NS, NX, NS>(kf, vf[k2], Lst[db]);
             }
         // the next chunk rewrites LDS (DMA: after the barrier that opens it)
