@@ -12,7 +12,6 @@ namespace triune {
 constexpr int CHUNK = 64;
 // Row padding (elements) of LDS planes that are not swizzled (see Plane): spreads rows over banks.
 constexpr int PAD = 4;
-constexpr int PAD128 = 20;
 
 struct Work {
     int64_t seq, b, row0, t_begin, t_end, len;

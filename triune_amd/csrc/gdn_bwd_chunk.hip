@@ -168,26 +168,32 @@ __device__ __forceinline__ f32x4 mms(const Split8<NA>& a, const Split8<2>& b, co
     return mfma_split<NA, 2, 2>(a, b, c);
 }
 
-// Column block x (accumulator layout) into the NP planes of a token-major matrix: p at its first row
-// and column, rs elements per row, pb bytes per plane.
-template <int NP>
-__device__ __forceinline__ void put_col(char* base, int pb, int rs, int row0, int col, const Lane& L, const f32x4& x) {
+// Column block x (accumulator layout) of rows row0 + [0, 16) and column col into NP planes.
+template <int NP, int D>
+__device__ __forceinline__ void put_col(char* base, int row0, int col, const Lane& L, const f32x4& x) {
+    using PL = Plane<D>;
     float r[4] = {x[0], x[1], x[2], x[3]};
     uint32_t w[NP][2];
     split_pairs<NP, 2>(r, w);
 #pragma unroll
-    for (int pl = 0; pl < NP; ++pl) {
-        uint16_t* p = reinterpret_cast<uint16_t*>(base + pl * pb) + (row0 + 4 * L.g4) * rs + col;
-        p[0] = (uint16_t)w[pl][0];
-        p[rs] = (uint16_t)(w[pl][0] >> 16);
-        p[2 * rs] = (uint16_t)w[pl][1];
-        p[3 * rs] = (uint16_t)(w[pl][1] >> 16);
+    for (int e = 0; e < 4; ++e) {
+        const int row = 4 * L.g4 + e;
+        uint16_t* p = reinterpret_cast<uint16_t*>(base) + (row0 + row) * PL::RS + PL::unit(col & ~3, PL::swz(row)) + (col & 3);
+#pragma unroll
+        for (int pl = 0; pl < NP; ++pl) p[pl * (PL::BYTES / 2)] = (uint16_t)(w[pl][e >> 1] >> (16 * (e & 1)));
     }
 }
 
 // Lower-triangular tiles in two bf16 parts: part n of tile t at t * TLB + n * TLB / 2, rows TSR apart.
 __device__ __forceinline__ void put_ltile(char* tiles, int t, const Lane& L, const f32x4& x) {
-    put_col<2>(tiles + t * TLB, TLB / 2, TSR, 0, L.r16, L, x);
+    float r[4] = {x[0], x[1], x[2], x[3]};
+    uint32_t w[2][2];
+    split_pairs<2, 2>(r, w);
+    uint16_t* p = reinterpret_cast<uint16_t*>(tiles + t * TLB) + 4 * L.g4 * TSR + L.r16;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int pl = 0; pl < 2; ++pl) p[pl * TSZ + e * TSR] = (uint16_t)(w[pl][e >> 1] >> (16 * (e & 1)));
 }
 __device__ __forceinline__ bf16x4 tile_row(const char* tiles, int t, int part, const Lane& L) {
     return *reinterpret_cast<const bf16x4*>(reinterpret_cast<const __bf16*>(tiles + t * TLB + part * (TLB / 2)) +
@@ -405,8 +411,7 @@ __device__ __forceinline__ void copy_tiles(char* tiles, float* mem) {
 template <int D>
 struct MapLay {
     static constexpr int NW = D / 16;
-    static constexpr int RS = D + (D == 128 ? PAD128 : PAD);  // elements per plane row
-    static constexpr int ROWP = GC * RS * 2;
+    static constexpr int ROWP = Plane<D>::BYTES;
     static constexpr int BYTES = 3 * 2 * ROWP + 2 * NTL * TLB + GC * 4;
 };
 
@@ -420,7 +425,8 @@ __device__ __forceinline__ void put_at(char* tiles, int t, int s, float x) {
 template <typename T, int D>
 __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_map_kernel(GdnChunkBwdParams p) {
     using Y = MapLay<D>;
-    constexpr int NW = Y::NW, RS = Y::RS, NKS = D / 32, NX = Prec<T>::NX;
+    using PL = Plane<D>;
+    constexpr int NW = Y::NW, NKS = D / 32, NX = Prec<T>::NX;
     __shared__ __attribute__((aligned(16))) char smem[Y::BYTES];
     char* P0 = smem;                   // Qt rows, then Q0
     char* P1 = P0 + 2 * Y::ROWP;       // Bt rows, then B0
@@ -459,9 +465,9 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_map_kernel(GdnChunkBwdParams
                 g[i][r] = kk[i][r] * be[i][r] * fast_exp(m - G[i][r]);  // g holds the W rows from here on
                 kk[i][r] *= fast_exp(Gp[i][r] - m);
             }
-            put_col<2>(P0, Y::ROWP, RS, 16 * i, col, L, q[i]);
-            put_col<2>(P1, Y::ROWP, RS, 16 * i, col, L, kk[i]);
-            put_col<2>(P2, Y::ROWP, RS, 16 * i, col, L, g[i]);
+            put_col<2, D>(P0, 16 * i, col, L, q[i]);
+            put_col<2, D>(P1, 16 * i, col, L, kk[i]);
+            put_col<2, D>(P2, 16 * i, col, L, g[i]);
         }
         lds_sync();
         for (int n = w; n < NTL; n += NW) {
@@ -470,8 +476,8 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_map_kernel(GdnChunkBwdParams
             f32x4 a = zero4();
 #pragma unroll
             for (int ks = 0; ks < NKS; ++ks)
-                a = mms(lds_frag<2>(P1, Y::ROWP, RS, 16 * i + r16, 32 * ks, g4),
-                        lds_frag<2>(P2, Y::ROWP, RS, 16 * j + r16, 32 * ks, g4), a);
+                a = mms(PL::template frag<2>(P1, 16 * i, r16, ks, g4),
+                        PL::template frag<2>(P2, 16 * j, r16, ks, g4), a);
             if (i == j) {
                 a = lower(a, true, false, L);
                 float* t = reinterpret_cast<float*>(sL + n * TLB) + 4 * g4 * TSR + r16;
@@ -490,7 +496,7 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_map_kernel(GdnChunkBwdParams
     } else {
         // rows of q, k and the decays in fp32; L and A from running products of the decays, a lane
         // (pair of lanes' elements at D = 128) per key dim
-        constexpr int LD = RS;
+        constexpr int LD = D;
         float* F0 = reinterpret_cast<float*>(P0);
         float* F1 = reinterpret_cast<float*>(P1);
         float* F2 = reinterpret_cast<float*>(P2);
@@ -575,17 +581,17 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_map_kernel(GdnChunkBwdParams
             f32x4 a = zero4();
 #pragma unroll
             for (int ks = 0; ks < NKS; ++ks)
-                a = mms(lds_frag<2>(P0, Y::ROWP, RS, 16 * i + r16, 32 * ks, g4),
-                        lds_frag<2>(P2, Y::ROWP, RS, 16 * j + r16, 32 * ks, g4), a);
+                a = mms(PL::template frag<2>(P0, 16 * i, r16, ks, g4),
+                        PL::template frag<2>(P2, 16 * j, r16, ks, g4), a);
             put_ltile(sA, n, L, lower(a, i == j, true, L));
         }
     }
     lds_sync();
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        put_col<2>(P0, Y::ROWP, RS, 16 * i, col, L, q[i]);
-        put_col<2>(P1, Y::ROWP, RS, 16 * i, col, L, kk[i]);
-        put_col<2>(P2, Y::ROWP, RS, 16 * i, col, L, g[i]);
+        put_col<2, D>(P0, 16 * i, col, L, q[i]);
+        put_col<2, D>(P1, 16 * i, col, L, kk[i]);
+        put_col<2, D>(P2, 16 * i, col, L, g[i]);
     }
     copy_tiles<true, 4 * D>(sL, p.ws_t + k.id * (2 * NTL * 256));
     lds_sync();
@@ -607,12 +613,12 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_map_kernel(GdnChunkBwdParams
         f32x4 am = zero4(), at = zero4(), an = zero4(), ak = zero4();
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
-            const Split8<2> a = lds_frag_tr<2>(P2, Y::ROWP, RS, 32 * ks, 16 * rt, g4, r16);
+            const Split8<2> a = PL::template frag_tr<2>(P2, 32 * ks, rt, g4, r16);
             am = mms(a, xs[ks], am);
             at = mms(xs[ks], a, at);  // the same tile transposed
             an = mms(a, vs[ks], an);
-            ak = mfma_split<2, NX, 2>(lds_frag_tr<2>(P0, Y::ROWP, RS, 32 * ks, 16 * rt, g4, r16), ds[ks], ak);
-            ak = mms(lds_frag_tr<2>(P1, Y::ROWP, RS, 32 * ks, 16 * rt, g4, r16), zs[ks], ak);
+            ak = mfma_split<2, NX, 2>(PL::template frag_tr<2>(P0, 32 * ks, rt, g4, r16), ds[ks], ak);
+            ak = mms(PL::template frag_tr<2>(P1, 32 * ks, rt, g4, r16), zs[ks], ak);
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -750,8 +756,7 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_scan_kernel(GdnChunkBwdParam
 template <int D, int NX>
 struct GradLay {
     static constexpr int NW = D / 16;
-    static constexpr int RS = D + (D == 128 ? PAD128 : PAD);
-    static constexpr int ROWP = GC * RS * 2;
+    static constexpr int ROWP = Plane<D>::BYTES;
     static constexpr int BYTES = (2 * 2 + NX) * ROWP + 2 * NTL * TLB + 2 * NW * GC * 4;
 };
 
@@ -809,7 +814,8 @@ template <typename T, int D>
 __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_grad_kernel(GdnChunkBwdParams p) {
     constexpr int NX = Prec<T>::NX;
     using Y = GradLay<D, NX>;
-    constexpr int NW = Y::NW, RS = Y::RS, NKS = D / 32;
+    using PL = Plane<D>;
+    constexpr int NW = Y::NW, NKS = D / 32;
     __shared__ __attribute__((aligned(16))) char smem[Y::BYTES];
     char* P1 = smem;                  // B0 rows, then U
     char* P2 = P1 + 2 * Y::ROWP;      // Wc rows, then dR
@@ -862,9 +868,9 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_grad_kernel(GdnChunkBwdParam
             b0[r] = kk[i][r] * fast_exp(Gp[i][r]);
             wc[r] = kk[i][r] * be[i][r] * ew[i][r];
         }
-        put_col<2>(P1, Y::ROWP, RS, 16 * i, col, L, b0);
-        put_col<2>(P2, Y::ROWP, RS, 16 * i, col, L, wc);
-        put_col<NX>(sO, Y::ROWP, RS, 16 * i, col, L, dO[i]);
+        put_col<2, D>(P1, 16 * i, col, L, b0);
+        put_col<2, D>(P2, 16 * i, col, L, wc);
+        put_col<NX, D>(sO, 16 * i, col, L, dO[i]);
     }
     copy_tiles<false, 4 * D>(sL, p.ws_t + k.id * (2 * NTL * 256));
     lds_sync();
@@ -884,8 +890,8 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_grad_kernel(GdnChunkBwdParam
         const Split8<2> d = split_pair(mem_col(Dn, o, L), mem_col(Dn, o + NW, L));
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            v[i] = mms(lds_frag<2>(P1, Y::ROWP, RS, 16 * i + r16, 32 * ks, g4), s, v[i]);
-            z[i] = mms(lds_frag<2>(P2, Y::ROWP, RS, 16 * i + r16, 32 * ks, g4), d, z[i]);
+            v[i] = mms(PL::template frag<2>(P1, 16 * i, r16, ks, g4), s, v[i]);
+            z[i] = mms(PL::template frag<2>(P2, 16 * i, r16, ks, g4), d, z[i]);
         }
     }
     solve<false>(sL, L, v);
@@ -894,8 +900,8 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_grad_kernel(GdnChunkBwdParam
     lds_sync();
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        put_col<2>(P1, Y::ROWP, RS, 16 * i, col, L, v[i]);
-        put_col<2>(P2, Y::ROWP, RS, 16 * i, col, L, z[i]);
+        put_col<2, D>(P1, 16 * i, col, L, v[i]);
+        put_col<2, D>(P2, 16 * i, col, L, z[i]);
     }
     lds_sync();
     for (int n = w; n < 2 * NTL; n += NW) {
@@ -905,9 +911,9 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_grad_kernel(GdnChunkBwdParam
         f32x4 a = zero4();
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks) {
-            const Split8<2> u = lds_frag<2>(P1, Y::ROWP, RS, 16 * j + r16, 32 * ks, g4);
-            if (isA) a = mms(lds_frag<NX>(sO, Y::ROWP, RS, 16 * i + r16, 32 * ks, g4), u, a);
-            else a = mms(lds_frag<2>(P2, Y::ROWP, RS, 16 * i + r16, 32 * ks, g4), u, a);
+            const Split8<2> u = PL::template frag<2>(P1, 16 * j, r16, ks, g4);
+            if (isA) a = mms(PL::template frag<NX>(sO, 16 * i, r16, ks, g4), u, a);
+            else a = mms(PL::template frag<2>(P2, 16 * i, r16, ks, g4), u, a);
         }
         if (isA) put_ltile(sA, n, L, lower(a, i == j, true, L));
         else put_ltile(sL, n - NTL, L, -lower(a, i == j, false, L));
@@ -929,9 +935,9 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_grad_kernel(GdnChunkBwdParam
         const Split8<2> s = split_pair(s0, s1), d = split_pair(d0, d1);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            aq[i] = mms(lds_frag<NX>(sO, Y::ROWP, RS, 16 * i + r16, 32 * ks, g4), s, aq[i]);
-            ab[i] = mms(lds_frag<2>(P2, Y::ROWP, RS, 16 * i + r16, 32 * ks, g4), s, ab[i]);
-            aw[i] = mms(lds_frag<2>(P1, Y::ROWP, RS, 16 * i + r16, 32 * ks, g4), d, aw[i]);
+            aq[i] = mms(PL::template frag<NX>(sO, 16 * i, r16, ks, g4), s, aq[i]);
+            ab[i] = mms(PL::template frag<2>(P2, 16 * i, r16, ks, g4), s, ab[i]);
+            aw[i] = mms(PL::template frag<2>(P1, 16 * i, r16, ks, g4), d, aw[i]);
         }
     }
     es = g4_sum(es) * fast_exp(gc);
@@ -985,7 +991,7 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_grad_kernel(GdnChunkBwdParam
     } else {
         // once every wave is past its reads of U, dR and D, their places take the three sums
         __syncthreads();
-        constexpr int LD = RS;  // an fp32 row takes the place of the two parts' rows
+        constexpr int LD = D;  // an fp32 row takes the place of the two parts' rows
         float* F1 = reinterpret_cast<float*>(P1);
         float* F2 = reinterpret_cast<float*>(P2);
         float* F3 = p.ws_d + k.id * (D * D);
