@@ -95,6 +95,11 @@ def _bind(lib):
              _i64, _i64, _i64, _i, _i, _i, _vp, ctypes.c_size_t, _vp],
             _i,
         ),
+        "triune_hip_gla_prefill_bwd_after": (
+            [_vp, _vp, _vp, _vp, _i, _i, _vp, _i64p, _vp, _vp, _vp, _vp, _vp, _i, _vp, _i, _vp,
+             _i64, _i64, _i64, _i, _i, _i, _vp, _vp, _sz, _vp],
+            _i,
+        ),
         "triune_hip_recurrent_scan_bwd": (
             [_vp, _i, _vp, _i, _vp, _i, _vp, _vp, _vp, _vp, _i, _i64, _i64, _i64, _i, _i, _vp],
             _i,
@@ -172,6 +177,7 @@ EXPORTS = (
     "triune_hip_gla_prefill_varlen_pool",
     "triune_hip_gla_prefill_bwd_workspace_size",
     "triune_hip_gla_prefill_bwd",
+    "triune_hip_gla_prefill_bwd_after",
     "triune_hip_recurrent_scan_bwd",
     "triune_hip_gdn_prefill",
     "triune_hip_gdn_prefill_chunked_workspace_size",

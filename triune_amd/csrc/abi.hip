@@ -673,6 +673,17 @@ int triune_hip_gla_prefill_bwd(const void* q, const void* k, const void* v, cons
                                void* dq, void* dk, void* dv, int d_dtype, void* dg, int dg_dtype, float* ds0,
                                int64_t B, int64_t T, int64_t H, int Dk, int Dv, int flags, void* workspace,
                                size_t workspace_bytes, void* stream) {
+    return triune_hip_gla_prefill_bwd_after(q, k, v, g, io_dtype, g_dtype, dout, strides, s0, ds_final, dq, dk, dv,
+                                            d_dtype, dg, dg_dtype, ds0, B, T, H, Dk, Dv, flags, nullptr, workspace,
+                                            workspace_bytes, stream);
+}
+
+int triune_hip_gla_prefill_bwd_after(const void* q, const void* k, const void* v, const void* g, int io_dtype,
+                                     int g_dtype, const void* dout, const int64_t* strides, const float* s0,
+                                     const float* ds_final, void* dq, void* dk, void* dv, int d_dtype, void* dg,
+                                     int dg_dtype, float* ds0, int64_t B, int64_t T, int64_t H, int Dk, int Dv,
+                                     int flags, const void* fwd_workspace, void* workspace, size_t workspace_bytes,
+                                     void* stream) {
     if (!q || !k || !v || !g || !dout || !strides || !dq || !dk || !dv || !dg) return TRIUNE_ERR_NULL;
     if (!dtype_ok(io_dtype) || !dtype_ok(g_dtype) || !dtype_ok(d_dtype) || !dtype_ok(dg_dtype)) return TRIUNE_ERR_DTYPE;
     if (!gate_dtype_ok(io_dtype, g_dtype)) return TRIUNE_ERR_DTYPE;
@@ -710,7 +721,9 @@ int triune_hip_gla_prefill_bwd(const void* q, const void* k, const void* v, cons
     const BwdPlan pl = plan_bwd(B, T, H, Dk, flags);
     if (!workspace || workspace_bytes < pl.total) return TRIUNE_ERR_WORKSPACE;
     char* ws = reinterpret_cast<char*>(workspace);
-    if (reinterpret_cast<uintptr_t>(ws) % 16) return TRIUNE_ERR_LAYOUT;
+    if (reinterpret_cast<uintptr_t>(ws) % 16 || reinterpret_cast<uintptr_t>(fwd_workspace) % 16) return TRIUNE_ERR_LAYOUT;
+    // the forward's segment states and decays: its own workspace (read only), or recomputed here
+    char* fws = fwd_workspace ? reinterpret_cast<char*>(const_cast<void*>(fwd_workspace)) : ws;
 
     BwdParams a{};
     PrefillParams& f = a.f;
@@ -720,8 +733,8 @@ int triune_hip_gla_prefill_bwd(const void* q, const void* k, const void* v, cons
     fill_tok(f.g, g, st + 9, B, T, H, Dk, g_dtype);
     f.g_dt = g_dtype; f.o_dt = d_dtype;
     f.s0 = s0;
-    f.ws_state = reinterpret_cast<float*>(ws + pl.f.off_state);
-    f.ws_gamma = reinterpret_cast<float*>(ws + pl.f.off_gamma);
+    f.ws_state = reinterpret_cast<float*>(fws + pl.f.off_state);
+    f.ws_gamma = reinterpret_cast<float*>(fws + pl.f.off_gamma);
     f.n_seqs = B; f.H = H; f.T = T; f.Dk = Dk; f.Dv = Dv;
     f.P = pl.f.P; f.nseg_dense = (int)pl.f.nseg; f.varlen = 0; f.flags = flags & TRIUNE_FLAG_TAIL_UNCLAMPED;
     fill_tok(a.dout, dout, st + 12, B, T, H, Dv, io_dtype);
@@ -737,18 +750,19 @@ int triune_hip_gla_prefill_bwd(const void* q, const void* k, const void* v, cons
     a.nchunks = pl.nchunks;
     const int64_t nseg = pl.f.nseg;
 
-    // forward: segment-local states, then the carried-in state of every segment
-    if (launch_gla_seg_state(f, pl.f.n_work, io_dtype, hs) != hipSuccess) return TRIUNE_ERR_LAUNCH;
-    ScanParams sc{};
-    sc.kv = f.ws_state; sc.kv_dt = DT_F32;
-    sc.kv_so = nseg * H * DD; sc.kv_sh = DD; sc.kv_sn = H * DD;
-    sc.dec = f.ws_gamma; sc.dec_dt = DT_F32; sc.dec_is_log = 1;
-    sc.d_so = nseg * H * D; sc.d_sh = D; sc.d_sn = H * D;
-    sc.init = s0; sc.i_so = H * DD; sc.i_sh = DD;
-    sc.s_all = f.ws_state; sc.sa_dt = DT_F32; sc.sa_so = sc.kv_so; sc.sa_sh = sc.kv_sh; sc.sa_sn = sc.kv_sn;
-    sc.fin = nullptr; sc.fin_dt = DT_F32;
-    sc.n_outer = B; sc.H = H; sc.Dk = Dk; sc.Dv = Dv; sc.N = nseg;
-    if (launch_recurrent_scan(sc, hs) != hipSuccess) return TRIUNE_ERR_LAUNCH;
+    if (!fwd_workspace) {  // forward: segment-local states, then the carried-in state of every segment
+        if (launch_gla_seg_state(f, pl.f.n_work, io_dtype, hs) != hipSuccess) return TRIUNE_ERR_LAUNCH;
+        ScanParams sc{};
+        sc.kv = f.ws_state; sc.kv_dt = DT_F32;
+        sc.kv_so = nseg * H * DD; sc.kv_sh = DD; sc.kv_sn = H * DD;
+        sc.dec = f.ws_gamma; sc.dec_dt = DT_F32; sc.dec_is_log = 1;
+        sc.d_so = nseg * H * D; sc.d_sh = D; sc.d_sn = H * D;
+        sc.init = s0; sc.i_so = H * DD; sc.i_sh = DD;
+        sc.s_all = f.ws_state; sc.sa_dt = DT_F32; sc.sa_so = sc.kv_so; sc.sa_sh = sc.kv_sh; sc.sa_sn = sc.kv_sn;
+        sc.fin = nullptr; sc.fin_dt = DT_F32;
+        sc.n_outer = B; sc.H = H; sc.Dk = Dk; sc.Dv = Dv; sc.N = nseg;
+        if (launch_recurrent_scan(sc, hs) != hipSuccess) return TRIUNE_ERR_LAUNCH;
+    }
     // chunk starting states, segment end states, segment maps R
     if (launch_gla_bwd_state(a, pl.f.n_work, io_dtype, hs) != hipSuccess) return TRIUNE_ERR_LAUNCH;
     // the same scan over the segments in reverse order: the gradient reaching each segment's end

@@ -134,7 +134,8 @@ def _gate(g, q):
 ONEPASS = True
 
 
-def _prefill(q, k, v, g, initial_state, out, flags, save_final=True, out_dtype=None):
+def _prefill(q, k, v, g, initial_state, out, flags, save_final=True, out_dtype=None, keep=None):
+    # keep: a list that receives the workspace of a three-launch call (its segment states and decays)
     B, T, H, Dk0 = q.shape
     Dv0 = v.shape[-1]
     # value columns evolve independently: wide values run as column slices, 128 wide, or 64 wide
@@ -192,6 +193,8 @@ def _prefill(q, k, v, g, initial_state, out, flags, save_final=True, out_dtype=N
             ptr(sf), B, T, H, Dk, Dv, flags, ptr(ws), ws.numel(), stream_of(q),
         )
         check(rc, "triune_hip_gla_prefill")
+        if keep is not None:
+            keep.append(ws)
     if o is not out:
         res = o[..., :Dv0]
         if out is not None:
@@ -271,12 +274,13 @@ def _needs_grad(*ts) -> bool:
     return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in ts)
 
 
-def _prefill_bwd(q, k, v, g, s0, do, ds, flags, grad_dtype=None, outs=None, acc=0):
+def _prefill_bwd(q, k, v, g, s0, do, ds, flags, grad_dtype=None, outs=None, acc=0, fwd_ws=None):
     """Gradients (dq, dk, dv, dg, ds0) of _prefill for upstream do (of o) and ds (of the fp32
     final state), either of which may be None.  grad_dtype: dtype of dq, dk, dv, dg (default:
     the inputs' own dtypes).  outs: fp32 (dq, dk, dv, dg) views of exactly the kernel width to
     write into (or, for the parts acc names, add into: _lib.FLAG_BWD_ACC_QKG / FLAG_BWD_ACC_V);
-    they are returned in place of new tensors."""
+    they are returned in place of new tensors.  fwd_ws: the workspace _prefill kept for these inputs
+    (heads the gradient kernels hold whole), or None to recompute the segment states."""
     B, T, H, Dk0 = q.shape
     Dv0 = v.shape[-1]
     lim = 32 if q.dtype == torch.float32 else 64  # widest head the gradient kernels hold
@@ -305,10 +309,10 @@ def _prefill_bwd(q, k, v, g, s0, do, ds, flags, grad_dtype=None, outs=None, acc=
     wsb = plan(q, "triune_hip_gla_prefill_bwd_workspace_size", B, max(T, 1), H, D, D, flags)
     ws = torch.empty(max(wsb, 256), device=q.device, dtype=torch.uint8)
     st = strides(_tok3(qp), _tok3(kp), _tok3(vp), _tok3(gp), _tok3(dop), _tok3(dq), _tok3(dk), _tok3(dv), _tok3(dg))
-    rc = L.triune_hip_gla_prefill_bwd(
+    rc = L.triune_hip_gla_prefill_bwd_after(
         ptr(qp), ptr(kp), ptr(vp), ptr(gp), dtype_code(qp), dtype_code(gp), ptr(dop), st, ptr(s0p), ptr(dsf),
         ptr(dq), ptr(dk), ptr(dv), dtype_code(dq), ptr(dg), dtype_code(dg), ptr(ds0), B, T, H, D, D, flags | acc,
-        ptr(ws), ws.numel(), stream_of(q),
+        ptr(fwd_ws), ptr(ws), ws.numel(), stream_of(q),
     )
     check(rc, "triune_hip_gla_prefill_bwd")
     if outs is not None:
@@ -368,15 +372,21 @@ class _ChunkGLA(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, v, g, initial_state, flags):
-        o, s = _prefill(q, k, v, g, initial_state, None, flags)
-        ctx.save_for_backward(q, k, v, g, initial_state)
+        # The segment states stay for the backward (16 KB per segment and head at D = 64, 8 MB for
+        # 512 segment-heads: recomputing them took 16 of its 98 us there); heads wider than the
+        # gradient kernels hold run in blocks, which recompute theirs.
+        keep = []
+        o, s = _prefill(q, k, v, g, initial_state, None, flags, keep=keep)
+        whole = max(q.shape[-1], v.shape[-1]) <= (32 if q.dtype == torch.float32 else 64)
+        ctx.save_for_backward(q, k, v, g, initial_state, keep[0] if whole and keep else None)
         ctx.flags = flags
+        ctx.set_materialize_grads(False)  # an unused output's gradient stays None: no zeros made and read
         return o, s
 
     @staticmethod
     def backward(ctx, do, ds):
-        q, k, v, g, s0 = ctx.saved_tensors
-        dq, dk, dv, dg, ds0 = _prefill_bwd(q, k, v, g, s0, do, ds, ctx.flags)
+        q, k, v, g, s0, ws = ctx.saved_tensors
+        dq, dk, dv, dg, ds0 = _prefill_bwd(q, k, v, g, s0, do, ds, ctx.flags, fwd_ws=ws)
         return dq, dk, dv, dg, ds0, None
 
 
@@ -767,6 +777,7 @@ class _GatedDeltaNet(torch.autograd.Function):
         o, s = _gdn_fwd(q, k, v, gf, beta, initial_state, beta_kind, out_dtype)
         ctx.save_for_backward(q, k, v, g, beta, initial_state)
         ctx.beta_kind = beta_kind
+        ctx.set_materialize_grads(False)
         return o, s
 
     @staticmethod
