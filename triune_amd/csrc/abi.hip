@@ -4,6 +4,7 @@
 #include "kernels.h"
 
 #include <atomic>
+#include <cmath>
 #include <initializer_list>
 #include <map>
 #include <mutex>
@@ -83,29 +84,75 @@ int64_t resident_slots(int Dk, int Dv, bool ck) {
     return slots;
 }
 
-// Segments per sequence (dense): fill the resident workgroup slots once with near-equal
-// segments; never more segments than chunks.  flags bits 8..15 force a chunk count instead.
+// Time of a segmented prefill in chunk steps: `jobs` (segment, head) workgroups of `chunks` chunk
+// steps each run in rounds of `slots`, every workgroup paying about two more steps (its state, its
+// first loads and its last stores, with nothing to overlap them), and the carry scan moves every
+// segment's state twice (at D = 128 a job's 128 KB take 0.0032 of a step's 8 us).
+// spill: part of a round that the last one must leave empty not to count as one more (jobs estimated).
+double seg_cost(double jobs, int64_t chunks, int64_t slots, int Dk, int Dv, double spill = 0) {
+    return std::ceil(jobs / (double)slots + spill) * (double)(chunks + 2) + jobs * 0.0032 * (Dk * Dv / 16384.0);
+}
+
+// nseg near-equal segments, or the fewest with the same longest one where that drops 15 % of them: the
+// time of a round is its longest workgroup's, and the others' slack goes into more states and a longer
+// carry scan.  47 chunks on 21 slots per (sequence, head): 16 segments of 3 or 2 chunks 41.1 us, 21
+// segments 45.2 us (B = 3, T = 3001, H = 8, fp32 gates); at 256 chunks (20 for 21) the
+// lighter average load of more segments was worth 0.6 %.
+int64_t fewest_segments(int64_t nchunks, int64_t nseg) {
+    const int64_t longest = (nchunks + nseg - 1) / nseg, fewest = (nchunks + longest - 1) / longest;
+    return 20 * fewest <= 17 * nseg ? fewest : nseg;
+}
+
+// Segments per sequence (dense): near-equal segments that fill the resident workgroup slots once, or
+// two to four times where one round leaves enough slots empty for that to cost 5 % less (B = 8,
+// H = 12, T = 8192, D = 128: 96 (sequence, head) pairs on 256 slots, 2 segments 618 us, 8 segments
+// 510 us); never more segments than chunks.  flags bits 8..15 force a chunk count instead.
 int64_t dense_segments(int64_t B, int64_t H, int64_t nchunks, int Dk, int Dv, int flags, bool ck) {
     const int forced = (flags >> TRIUNE_FLAG_SEG_SHIFT) & 0xff;
     if (forced > 0) return (nchunks + forced - 1) / forced;
-    int64_t nseg = resident_slots(Dk, Dv, ck) / (B * H);
-    if (nseg < 1) nseg = 1;
-    if (nseg > nchunks) nseg = nchunks;
-    return nseg;
+    if (B * H <= 0 || nchunks <= 1) return 1;
+    const int64_t slots = resident_slots(Dk, Dv, ck);
+    int64_t best = 1;
+    double least = 0;
+    for (int rounds = 1; rounds <= 4; ++rounds) {
+        int64_t nseg = rounds * slots / (B * H);
+        nseg = fewest_segments(nchunks, nseg < 1 ? 1 : (nseg > nchunks ? nchunks : nseg));
+        const double c = seg_cost((double)(B * H * nseg), (nchunks + nseg - 1) / nseg, slots, Dk, Dv);
+        if (rounds == 1 || c < 0.95 * least) {
+            best = nseg;
+            least = c;
+        }
+    }
+    return best;
 }
 
-// Chunks per segment (varlen): about eight resident rounds of workgroups.  Sequence lengths
-// vary, so segments sized for a single round leave the longest walks (up to a whole sequence)
-// on the critical path; at config 4 (32 sequences of 128..8192 tokens, D = 128) one round
-// (111 chunks per segment) took 3.2 ms and eight rounds (14) 2.1 ms, with 4..32 all within 10 %.
-int varlen_seg_chunks(int64_t chunk_jobs, int Dk, int Dv, int flags) {
+// Chunks per segment (varlen): about eight rounds of resident workgroups (lengths vary, so segments
+// sized for one round leave the longest walks on the critical path: 3.2 against 2.1 ms at 32
+// sequences of 128..8192 tokens, D = 128), at least 4, unless another length is estimated at least
+// 7 % cheaper.  Lengths are not known on the host, so the estimate takes every sequence to end in half
+// a segment and other lengths' last rounds to spill when nearly full.  28,956 tokens in 8 sequences
+// (H = 12, D = 128): 323 us with 4 chunks, 285 with 13; 4,243 tokens in 5 sequences stay at 4 (61 us;
+// 83 with 3, which needs a second round).
+int varlen_seg_chunks(int64_t n_seqs, int64_t total_tokens, int64_t H, int Dk, int Dv, int flags) {
     const int forced = (flags >> TRIUNE_FLAG_SEG_SHIFT) & 0xff;
     if (forced > 0) return forced;
-    const int64_t slots = resident_slots(Dk, Dv, true) * 8;  // varlen runs the checked instances
-    int64_t p = (chunk_jobs + slots - 1) / slots;
-    if (p < 4) p = 4;
-    if (p > 255) p = 255;
-    return (int)p;
+    const int64_t slots = resident_slots(Dk, Dv, true);  // varlen runs the checked instances
+    auto cost = [&](int64_t p, double spill) {
+        const double jobs = (double)H * ((double)total_tokens / (64.0 * (double)p) + 0.5 * (double)n_seqs);
+        return seg_cost(jobs, p, slots, Dk, Dv, spill);
+    };
+    const int64_t chunk_jobs = H * ((total_tokens + 63) / 64 + n_seqs);
+    int64_t best = (chunk_jobs + 8 * slots - 1) / (8 * slots);
+    best = best < 4 ? 4 : (best > 255 ? 255 : best);
+    double least = 0.93 * cost(best, 0.0);
+    for (int64_t p = 4; p <= 32; ++p) {
+        const double c = cost(p, 0.12);
+        if (c < least) {
+            best = p;
+            least = c;
+        }
+    }
+    return (int)best;
 }
 
 bool prefill_shape_ok(int Dk, int Dv) { return prefill_shape_supported(Dk, Dv); }
@@ -147,8 +194,7 @@ PrefillPlan plan_dense(int64_t B, int64_t T, int64_t H, int Dk, int Dv, int flag
 
 PrefillPlan plan_varlen(int64_t n_seqs, int64_t total_tokens, int64_t H, int Dk, int Dv, int flags) {
     PrefillPlan p{};
-    const int64_t nchunks = (total_tokens + 63) / 64 + n_seqs;
-    p.P = varlen_seg_chunks(H * nchunks, Dk, Dv, flags);
+    p.P = varlen_seg_chunks(n_seqs, total_tokens, H, Dk, Dv, flags);
     p.n_work = (total_tokens + 64 * (int64_t)p.P - 1) / (64 * (int64_t)p.P) + n_seqs;
     p.nseg = 0;
     p.off_segoff = 0;
