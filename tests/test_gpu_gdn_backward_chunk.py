@@ -103,6 +103,22 @@ def test_only_the_final_state(dev):
     _check(got, ref, torch.bfloat16, NAMES)
 
 
+@pytest.mark.parametrize("D", [64, 128])
+def test_gate_and_beta_repeated_over_tokens(dev, D):
+    """One decay and one beta per head, expanded over the tokens (stride 0), with a partial last chunk
+    and a gradient of the final state: the gates past the last token count as none."""
+    q, k, v, _, _, do, ds = _inputs(2, 100, 3, D, "head", True, torch.bfloat16, seed=D)
+    g = torch.tensor([-0.25, -0.03125, -0.5]).bfloat16().expand(2, 100, 3)
+    b = torch.tensor([0.5, 0.25, 0.75]).bfloat16().expand(2, 100, 3)
+    kind = _lib.BETA_HEAD
+    dg, db = (x[0, 0].to(dev).expand(2, 100, 3) for x in (g, b))
+    got = FG._gdn_bwd(*(x.to(dev) for x in (q, k, v)), dg, db, None, kind, do.to(dev), ds.to(dev))
+    torch.cuda.synchronize()
+    ref = list(O.gdn_bwd(q, k, v, g.unsqueeze(-1).expand(2, 100, 3, D).contiguous(), b.contiguous(), None, do, ds))
+    ref[3] = ref[3].sum(-1)
+    _check(got, ref, torch.bfloat16, NAMES)
+
+
 @pytest.mark.parametrize("gate", ["key", "head"])
 def test_operator_views_and_padding(dev, gate, monkeypatch):
     """The operator's autograd with strided q, k, v views, a non-contiguous beta and gate, and head

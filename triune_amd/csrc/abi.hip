@@ -1164,6 +1164,9 @@ int triune_hip_gdn_bwd_chunked(const void* q, const void* k, const void* v, cons
     for (int i = 0; i < 6; ++i) {
         const int64_t ts = i == 4 && beta_kind == TRIUNE_BETA_NONE ? 0 : (i == 5 && !dout ? 0 : strides[3 * i + 1]);
         if (ts < 0 || ts > 0x7fffffff / 160) return TRIUNE_ERR_LAYOUT;
+        // rows are read up to the last token's end: rows of D elements must not overlap
+        const bool wide = i < 3 || (i == 3 && !g_head) || (i == 5 && dout);
+        if (wide && T > 1 && ts < D) return TRIUNE_ERR_LAYOUT;
     }
     if (H > 0x7fffffff / (160 * D)) return TRIUNE_ERR_LAYOUT;
     if (B == 0) return TRIUNE_OK;

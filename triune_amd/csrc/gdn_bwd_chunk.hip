@@ -323,6 +323,12 @@ __device__ __forceinline__ void load_gate(const GdnChunkBwdParams& p, const Chun
                                           f32x4 (&x)[4]) {
     const int64_t off = k.b * p.f.g_sb + k.c * GC * p.f.g_st + k.h * p.f.g_sh;
     load_rows<T>(rows_at<T>(p.f.g, off, p.f.g_st, p.g_head ? 1 : D, p.g_head ? 0 : col, k.nv, L), x);
+    // a head gate that repeats one value over the tokens (stride 0) is in range past the last row too
+    if (k.nv < GC) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+            if (16 * (e >> 2) + 4 * L.g4 + (e & 3) >= k.nv) x[e >> 2][e & 3] = 0.f;
+    }
 }
 template <typename T>
 __device__ __forceinline__ void load_beta(const GdnChunkBwdParams& p, const Chunk& k, const Lane& L, f32x4 (&x)[4]) {
