@@ -215,9 +215,10 @@ int triune_hip_gla_prefill_onepass(const void* q, const void* k, const void* v, 
 /* triune_hip_gla_prefill without a workspace argument, for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
  * No counterpart in the reference.  The workspace is a static device array of
- * TRIUNE_GLA_PREFILL_SCRATCH_BYTES (32 MiB) per GPU, held until the process ends; a call whose
- * workspace (triune_hip_gla_prefill_workspace_size) exceeds it returns TRIUNE_ERR_SCRATCH and
- * launches nothing.  Config 1 (B = 4, T = 16384, H = 6, D = 64) needs about 8 MB; at D = 128 the
+ * TRIUNE_GLA_PREFILL_SCRATCH_BYTES (32 MiB) per GPU, held until the process ends.  Where
+ * triune_hip_gla_prefill's segments (triune_hip_gla_prefill_workspace_size) exceed it, the call
+ * runs on fewer and longer ones (other roundings at their borders); if not even one round of
+ * workgroups fits it returns TRIUNE_ERR_SCRATCH and launches nothing.  Config 1 (B = 4, T = 16384, H = 6, D = 64) needs about 8 MB; at D = 128 the
  * bound is reached near B * H = 500 (head, sequence) pairs.  Every call on a GPU shares that
  * GPU's array (each call writes what it reads, so nothing needs clearing): calls that overlap on
  * one GPU (other streams or host threads) race and must be serialised by the caller.  stream must

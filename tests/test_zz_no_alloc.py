@@ -84,3 +84,20 @@ def test_noalloc_python_wrapper_and_limits(dev):
         gla_prefill_noalloc(q, k, v, g[:, :1].expand_as(g), s0, out, fin)
     # a call needing more than the scratch (TRIUNE_ERR_SCRATCH, nothing launched) is checked on the
     # host only (tests/test_abi_host.py::test_noalloc_prefill_validation)
+
+
+def test_noalloc_takes_calls_whose_several_rounds_exceed_the_scratch(dev):
+    """170 (sequence, head) pairs at D = 128 leave a third of the slots empty, so the workspace entry
+    takes two rounds of workgroups (three segments, more than the scratch holds); here one segment each."""
+    q, k, v, g, _ = _dev(gla_inputs(17, 960, 10, 128, seed=9, dtype=torch.bfloat16), dev)
+    L, st = lib(), stream_of(q)
+    assert int(L.triune_hip_gla_prefill_workspace_size(17, 960, 10, 128, 128, 0)) > 32 << 20
+    o, s = _noalloc(q, k, v, g, None, torch.float32)
+    o_ref, s_ref = torch.empty_like(o), torch.empty_like(s)
+    head = _args(q, k, v, g, None, o_ref, s_ref)[:-1]
+    one = 15 << 8  # all 15 chunks in one segment
+    wsb = int(L.triune_hip_gla_prefill_workspace_size(17, 960, 10, 128, 128, one))
+    ws = torch.empty(wsb, device=dev, dtype=torch.uint8)
+    check(L.triune_hip_gla_prefill(*head, one, ptr(ws), wsb, st), "prefill")
+    torch.cuda.synchronize()
+    assert torch.equal(o, o_ref) and torch.equal(s, s_ref)

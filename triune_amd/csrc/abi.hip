@@ -103,11 +103,17 @@ int64_t fewest_segments(int64_t nchunks, int64_t nseg) {
     return 20 * fewest <= 17 * nseg ? fewest : nseg;
 }
 
+// Workspace of a dense plan: every segment's states and log-decay sums.
+size_t dense_bytes(int64_t n_work, int64_t H, int Dk, int Dv) {
+    return align_up((size_t)n_work * H * Dk * Dv * sizeof(float)) + align_up((size_t)n_work * H * Dk * sizeof(float));
+}
+
 // Segments per sequence (dense): near-equal segments that fill the resident workgroup slots once, or
 // two to four times where one round leaves enough slots empty for that to cost 5 % less (B = 8,
 // H = 12, T = 8192, D = 128: 96 (sequence, head) pairs on 256 slots, 2 segments 618 us, 8 segments
-// 510 us); never more segments than chunks.  flags bits 8..15 force a chunk count instead.
-int64_t dense_segments(int64_t B, int64_t H, int64_t nchunks, int Dk, int Dv, int flags, bool ck) {
+// 510 us) and their states and decays fit in `limit` bytes; never more segments than chunks.  flags bits
+// 8..15 force a chunk count instead.
+int64_t dense_segments(int64_t B, int64_t H, int64_t nchunks, int Dk, int Dv, int flags, bool ck, size_t limit) {
     const int forced = (flags >> TRIUNE_FLAG_SEG_SHIFT) & 0xff;
     if (forced > 0) return (nchunks + forced - 1) / forced;
     if (B * H <= 0 || nchunks <= 1) return 1;
@@ -117,6 +123,7 @@ int64_t dense_segments(int64_t B, int64_t H, int64_t nchunks, int Dk, int Dv, in
     for (int rounds = 1; rounds <= 4; ++rounds) {
         int64_t nseg = rounds * slots / (B * H);
         nseg = fewest_segments(nchunks, nseg < 1 ? 1 : (nseg > nchunks ? nchunks : nseg));
+        if (rounds > 1 && dense_bytes(B * nseg, H, Dk, Dv) > limit) break;
         const double c = seg_cost((double)(B * H * nseg), (nchunks + nseg - 1) / nseg, slots, Dk, Dv);
         if (rounds == 1 || c < 0.95 * least) {
             best = nseg;
@@ -179,16 +186,17 @@ struct PrefillPlan {
     size_t off_segoff, off_state, off_gamma, total;
 };
 
-PrefillPlan plan_dense(int64_t B, int64_t T, int64_t H, int Dk, int Dv, int flags) {
+// limit: bytes that a plan of more than one round has to fit in (a plan of one round may exceed it).
+PrefillPlan plan_dense(int64_t B, int64_t T, int64_t H, int Dk, int Dv, int flags, size_t limit = SIZE_MAX) {
     PrefillPlan p{};
     const int64_t nchunks = (T + 63) / 64;
-    p.nseg = dense_segments(B, H, nchunks, Dk, Dv, flags, T % 4 != 0);
+    p.nseg = dense_segments(B, H, nchunks, Dk, Dv, flags, T % 4 != 0, limit);
     p.P = (int)((nchunks + p.nseg - 1) / p.nseg);
     p.n_work = B * p.nseg;
     p.off_segoff = 0;
     p.off_state = 0;
     p.off_gamma = align_up((size_t)p.n_work * H * Dk * Dv * sizeof(float));
-    p.total = p.off_gamma + align_up((size_t)p.n_work * H * Dk * sizeof(float));
+    p.total = dense_bytes(p.n_work, H, Dk, Dv);
     return p;
 }
 
@@ -407,10 +415,10 @@ static void fill_tok(TokTensor& t, const void* p, const int64_t* st3, int64_t nb
     t.extent = ((nb - 1) * t.sb + (nt - 1) * t.st + (H - 1) * t.sh + D) * es;
 }
 
-int triune_hip_gla_prefill(const void* q, const void* k, const void* v, const void* g, int io_dtype, int g_dtype,
-                           const int64_t* strides, const float* s0, void* o, int o_dtype, float* s_final,
-                           int64_t B, int64_t T, int64_t H, int Dk, int Dv, int flags, void* workspace,
-                           size_t workspace_bytes, void* stream) {
+static int prefill_dense(const void* q, const void* k, const void* v, const void* g, int io_dtype, int g_dtype,
+                         const int64_t* strides, const float* s0, void* o, int o_dtype, float* s_final, int64_t B,
+                         int64_t T, int64_t H, int Dk, int Dv, int flags, size_t limit, void* workspace,
+                         size_t workspace_bytes, void* stream) {
     if (!q || !k || !v || !g || !o || !strides) return TRIUNE_ERR_NULL;
     if (!dtype_ok(io_dtype) || !dtype_ok(g_dtype) || !dtype_ok(o_dtype)) return TRIUNE_ERR_DTYPE;
     if (!gate_dtype_ok(io_dtype, g_dtype)) return TRIUNE_ERR_DTYPE;
@@ -431,7 +439,7 @@ int triune_hip_gla_prefill(const void* q, const void* k, const void* v, const vo
         sc.n_outer = B; sc.H = H; sc.Dk = Dk; sc.Dv = Dv; sc.N = 0;
         return launch_status(launch_recurrent_scan(sc, st));
     }
-    const PrefillPlan pl = plan_dense(B, T, H, Dk, Dv, flags);
+    const PrefillPlan pl = plan_dense(B, T, H, Dk, Dv, flags, limit);
     if (!workspace || workspace_bytes < pl.total) return TRIUNE_ERR_WORKSPACE;
     char* ws = reinterpret_cast<char*>(workspace);
     if (reinterpret_cast<uintptr_t>(ws) % 16) return TRIUNE_ERR_LAYOUT;
@@ -449,6 +457,14 @@ int triune_hip_gla_prefill(const void* q, const void* k, const void* v, const vo
     a.n_seqs = B; a.H = H; a.T = T; a.Dk = Dk; a.Dv = Dv;
     a.P = pl.P; a.nseg_dense = (int)pl.nseg; a.varlen = 0; a.flags = flags & 0xff;
     return dense_launch(a, pl, s0, s_final, io_dtype, false, st);
+}
+
+int triune_hip_gla_prefill(const void* q, const void* k, const void* v, const void* g, int io_dtype, int g_dtype,
+                           const int64_t* strides, const float* s0, void* o, int o_dtype, float* s_final,
+                           int64_t B, int64_t T, int64_t H, int Dk, int Dv, int flags, void* workspace,
+                           size_t workspace_bytes, void* stream) {
+    return prefill_dense(q, k, v, g, io_dtype, g_dtype, strides, s0, o, o_dtype, s_final, B, T, H, Dk, Dv, flags,
+                         SIZE_MAX, workspace, workspace_bytes, stream);
 }
 
 }  // extern "C"
@@ -700,13 +716,13 @@ int triune_hip_gla_prefill_noalloc(const void* q, const void* k, const void* v, 
     if (B < 0 || T < 0 || H <= 0 || !prefill_shape_ok(Dk, Dv)) return TRIUNE_ERR_SHAPE;
     size_t need = 0;
     if (B > 0 && T > 0) {
-        need = plan_dense(B, T, H, Dk, Dv, flags).total;
+        need = plan_dense(B, T, H, Dk, Dv, flags, kScratchBytes).total;
         if (need > kScratchBytes) return TRIUNE_ERR_SCRATCH;
     }
     void* ws = need ? scratch_for(stream) : nullptr;
     if (need && !ws) return TRIUNE_ERR_LAUNCH;
-    return triune_hip_gla_prefill(q, k, v, g, io_dtype, g_dtype, strides, s0, o, o_dtype, s_final, B, T, H, Dk, Dv,
-                                  flags, ws, need ? kScratchBytes : 0, stream);
+    return prefill_dense(q, k, v, g, io_dtype, g_dtype, strides, s0, o, o_dtype, s_final, B, T, H, Dk, Dv, flags,
+                         kScratchBytes, ws, need ? kScratchBytes : 0, stream);
 }
 
 size_t triune_hip_gla_prefill_bwd_workspace_size(int64_t B, int64_t T, int64_t H, int Dk, int Dv, int flags) {
