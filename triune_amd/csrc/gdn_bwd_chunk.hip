@@ -32,9 +32,10 @@
 // of the four diagonal blocks.
 //
 // Measured, forward and backward together (bf16): B=4, H=6, T=8192, D=64, gate and beta per head
-// 3059 -> 483 us; B=4, H=12, T=2048, D=128, gate per key dim 5932 -> 752 us, against the token-serial
-// kernels.  Of that the map kernel 118 / 156 us, the scan 89 / 158, the gradients 176 / 216.  On the
-// fp32 MFMA (a quarter of the K per pass, no splitting) they took 156 / 220, 106 / 211, 253 / 319.
+// 3054 -> 494 us; B=4, H=12, T=2048, D=128, gate per key dim 5923 -> 737 us, against the token-serial
+// kernels.  Of that, when the split products came in, the map kernel 118 / 156 us, the scan 89 / 158,
+// the gradients 176 / 216; on the fp32 MFMA (a quarter of the K per pass, no splitting) they took
+// 156 / 220, 106 / 211, 253 / 319.
 // What bounds them now is the traffic of M, N, K, S and D: 16 D^2 bytes per chunk written and read
 // by the scan, 300 / 600 MB of it at 3.4-3.8 TB/s.
 //
