@@ -680,7 +680,8 @@ def _gdn(q, k, v, g, beta, initial_state, beta_kind, out_dtype=None):
 def _gdn_bwd(q, k, v, g, beta, initial_state, beta_kind, do, ds):
     """Gradients (dq, dk, dv, dg, dbeta, ds0) of _gdn_fwd for upstream do (of o) and ds (of the
     fp32 final state), either of which may be None, on triune_hip_gdn_bwd_chunked (16-bit throughout,
-    beta none or per head, no initial state) or triune_hip_gdn_bwd.  Head dims are zero-padded to the kernels' 64 or 128 (padded rows and columns of the state stay zero)."""
+    beta none or per head, no initial state) or triune_hip_gdn_bwd.  Head dims are zero-padded to the
+    kernels' 64 or 128 (padded rows and columns of the state stay zero)."""
     B, T, H, Dk0 = q.shape
     Dv0 = v.shape[-1]
     D = 64 if max(Dk0, Dv0) <= 64 else 128
