@@ -376,7 +376,7 @@ int triune_hip_gdn_bwd(const void* q, const void* k, const void* v, const void* 
                        void* dg, void* dbeta, float* ds0, int64_t B, int64_t T, int64_t H, int Dk, int Dv,
                        void* workspace, size_t workspace_bytes, void* stream);
 
-/* triune_hip_gdn_bwd for 16-bit I/O in chunk form on the matrix cores: io_dtype bf16 or fp16, g,
+/* triune_hip_gdn_bwd for 16-bit I/O in chunk form on the fp32 matrix cores: io_dtype bf16 or fp16, g,
  * beta and dout in io_dtype, beta none or per (token, head).  With g_head != 0 the gate is one value per
  * (token, head) (strides[9..11] of a [B, T, H] tensor) and dg is [B, T, H], the sum over the key
  * dims; otherwise g and dg are [B, T, H, D].  Other arguments as triune_hip_gdn_bwd; rows need unit

@@ -119,6 +119,22 @@ def test_gate_and_beta_repeated_over_tokens(dev, D):
     _check(got, ref, torch.bfloat16, NAMES)
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("gate,beta", [("key", False), ("head", True)])
+def test_small_gate_gradients(dev, D, gate, beta):
+    """dg is a difference of sums: fp32 products (2^-24 of each term, exponents up to 26 nats on either
+    side of the midpoint: about 60 * 2^-24 = 4e-6) leave its elements below a thousandth of the rms
+    (2^-12 of which, 2.4e-7, is fp16's own rounding) within 2e-6 of the rms, root mean square."""
+    q, k, v, g, b, do, ds = _inputs(2, 600, 3, D, gate, beta, torch.float16, seed=D + 5)
+    got, ref = _run(dev, q, k, v, g, b, do, ds)
+    r = torch.as_tensor(np.asarray(ref[3], dtype=np.float64))
+    rms = float(r.square().mean().sqrt())
+    small = (r != 0) & (r.abs() < (1e-3 if gate == "key" else 2e-2) * rms)
+    assert int(small.sum()) >= 20
+    err = (got[3].double().cpu() - r)[small].square().mean().sqrt()
+    assert float(err) <= (2e-6 if gate == "key" else 6e-6) * rms, float(err) / rms
+
+
 @pytest.mark.parametrize("gate", ["key", "head"])
 def test_operator_views_and_padding(dev, gate, monkeypatch):
     """The operator's autograd with strided q, k, v views, a non-contiguous beta and gate, and head

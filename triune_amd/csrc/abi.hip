@@ -1148,9 +1148,9 @@ int triune_hip_gdn_bwd(const void* q, const void* k, const void* v, const void* 
     return TRIUNE_OK;
 }
 
-// Chunk-form backward: per (b, h, chunk) the block-triangular tiles and four D x D matrices.
+// Chunk-form backward: per (b, h, chunk) the block-triangular tiles and three D x D matrices.
 static size_t gdn_bwd_chunked_bytes(int64_t B, int64_t T, int64_t H, int D) {
-    return (size_t)(B * H * ((T + 63) / 64)) * (4 * D * D + 20 * 256) * sizeof(float);
+    return (size_t)(B * H * ((T + 63) / 64)) * (3 * D * D + 20 * 256) * sizeof(float);
 }
 
 size_t triune_hip_gdn_bwd_chunked_workspace_size(int64_t B, int64_t T, int64_t H, int Dk, int Dv) {
@@ -1210,7 +1210,7 @@ int triune_hip_gdn_bwd_chunked(const void* q, const void* k, const void* v, cons
     p.nc = (T + 63) / 64;
     const int64_t n = B * H * p.nc;
     p.ws_m = reinterpret_cast<float*>(workspace);
-    p.ws_s = p.ws_m + 2 * n * D * D;
+    p.ws_s = p.ws_m + n * D * D;
     p.ws_d = p.ws_s + n * D * D;
     p.ws_t = p.ws_d + n * D * D;
     return launch_status(launch_gdn_bwd_chunk(p, D, st));

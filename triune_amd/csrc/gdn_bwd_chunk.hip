@@ -1,5 +1,5 @@
 // gdn_bwd_chunk.hip -- gradients of the Gated DeltaNet reference variant in chunk (WY/UT) form on the
-// matrix cores.
+// fp32 matrix cores.
 //
 // Same arithmetic as gdn_bwd.hip (the reference differentiates fast_recurrent_gated_deltanet,
 // triune/kernels/fast_gla.py:781-836, with autograd).  Per 64-token chunk, with G the inclusive and
@@ -24,20 +24,25 @@
 //   gdn_bwd_grad_kernel  one workgroup per (b, h, chunk): the gradients
 // so only the scan is serial, and its step is one product.
 //
-// Products run on v_mfma_f32_16x16x32_bf16 with both operands split into two bf16 parts (three MFMAs
-// per product, bf16 rows of dO as they are), as in the forward kernels: every gradient is rounded to
-// 16 bits, 2^-9 or 2^-12, far above the split's 2^-17.  A tile held in accumulator layout (lane 16 g4
-// + r16: rows 4 g4 + r of column r16) is half of a B operand, and half of the A operand of its
-// transpose, without moving lanes.  The solves with I + L are block substitutions with the inverses
-// of the four diagonal blocks.
+// Products run on v_mfma_f32_16x16x4_f32: its operands are fp32 as they come out of the accumulators
+// (nothing is rounded on the way), and a tile held in accumulator layout (lane 16 g4 + r16: rows
+// 4 g4 + r of column r16) is a B operand as it stands when product r contracts rows 4 g4 + r.  With
+// two bf16 parts per operand on v_mfma_f32_16x16x32_bf16 the kernels were a fifth faster (403 against
+// 480 us at D = 64, 520 against 730 at D = 128, the shapes below) but carried 2^-17 into dg, which is
+// a difference of sums: against 64 bits its error rose from the token-serial kernels' 2.08e-4 to
+// 2.14e-4 (fp16, B = 2, T = 600, H = 4, D = 64, gate per key dim) and elements below 1 % of its rms
+// lost up to eight bits (at 1e-3 to 1e-2 of it 1.6e-4 -> 4.4e-3 of their value).  In fp32 those are
+// 2.08e-4 and 2.1e-4.  Solves with I + L are block substitutions with the inverses of the four diagonal
+// blocks; dependent products issue back to back (32 cycles each), so the substitutions cost no more
+// than products with an explicit inverse would.
 //
-// Measured, forward and backward together (bf16): B=4, H=6, T=8192, D=64, gate and beta per head
-// 3054 -> 494 us; B=4, H=12, T=2048, D=128, gate per key dim 5923 -> 737 us, against the token-serial
-// kernels.  Of that, when the split products came in, the map kernel 118 / 156 us, the scan 89 / 158,
-// the gradients 176 / 216; on the fp32 MFMA (a quarter of the K per pass, no splitting) they took
-// 156 / 220, 106 / 211, 253 / 319.
-// What bounds them now is the traffic of M, N, K, S and D: 16 D^2 bytes per chunk written and read
-// by the scan, 300 / 600 MB of it at 3.4-3.8 TB/s.
+// Measured, backward alone (bf16): B=4, H=6, T=8192, D=64, gate and beta per head 2884 us on the
+// token-serial kernels, 480 here (map 165, scan 90, gradients 258); B=4, H=12, T=2048, D=128, gate per
+// key dim 5834 and 729 (232, 229, 332).  The map and gradient kernels are bound by the fp32 MFMA and by
+// the chain of a chunk beside it (416 and 680 products of 32 cycles per wave and chunk at D = 64: 67
+// and 109 us of the times above on two workgroups per CU, a third of each kernel at one per CU for
+// D = 128); the scan by the traffic of M, N, K, S and D (20 D^2 bytes per chunk: 2.8 TB/s at D = 64)
+// and the latency of its steps.
 //
 // A chunk in which some key dim decays by more than GB_SPAN nats forms its pair sums from running
 // products of the decays instead (L and A in the map kernel, [.] in the gradient kernel); the
@@ -51,12 +56,18 @@ namespace {
 constexpr int GC = 64;            // tokens per chunk
 constexpr float GB_SPAN = 128.f;  // factors within e^(+-64)
 constexpr float GB_GMIN = -104.f; // e^-104 is 0 in fp32: gates below it (-inf resets) act alike
-constexpr int TSR = 20;           // row stride of a 16 x 16 tile in LDS (elements)
-constexpr int TSZ = 16 * TSR;     // a tile's fp32 elements, or its two bf16 parts' TSZ each
-constexpr int TLB = TSZ * 4;      // bytes of a tile, either way
+constexpr int TSR = 20;           // row stride of a 16 x 16 tile in LDS (floats): rows and columns conflict-free
+constexpr int TSZ = 16 * TSR;
 constexpr int NTL = 10;           // lower-triangular 16 x 16 tiles of a 64 x 64 matrix
 
 __host__ __device__ constexpr int tl(int i, int j) { return i * (i + 1) / 2 + j; }
+
+// c + a b over 16 contracted indices: product r contracts index 4 g4 + r.
+__device__ __forceinline__ f32x4 mma(const f32x4& a, const f32x4& b, f32x4 c) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r], b[r], c, 0, 0, 0);
+    return c;
+}
 
 struct Lane {
     int w, g4, r16;
@@ -68,7 +79,7 @@ struct Lane {
     }
 };
 
-// N, K, S and D in memory: 16 x 16 tiles, row tile major, each in accumulator order (lane's four
+// M, N, K, S and D in memory: 16 x 16 tiles, row tile major, each in accumulator order (lane's four
 // rows of its column contiguous).  As an accumulator tile or B operand, and transposed.
 __device__ __forceinline__ f32x4 mem_col(const float* m, int t, const Lane& L) {
     return *reinterpret_cast<const f32x4*>(m + t * 256 + (uint32_t)(L.g4 * 64 + L.r16 * 4));
@@ -82,22 +93,25 @@ __device__ __forceinline__ void mem_put(float* m, int t, const Lane& L, const f3
     *reinterpret_cast<f32x4*>(m + t * 256 + (uint32_t)(L.g4 * 64 + L.r16 * 4)) = x;
 }
 
-// M and M^T in memory as the scan's A operands: operand f = row tile * NKS + K step, its two bf16
-// parts of 64 lanes x 8 slots each.  The four values x of a tile go to slots 4 half .. 4 half + 3.
-__device__ __forceinline__ void mem_put_half(float* m, int f, int half, const f32x4& x) {
-    float r[4] = {x[0], x[1], x[2], x[3]};
-    uint32_t w[2][2];
-    split_pairs<2, 2>(r, w);
-    uint2* p = reinterpret_cast<uint2*>(m) + (uint32_t)(f * 256 + (threadIdx.x & 63) * 2 + half);
-    p[0] = uint2{w[0][0], w[0][1]};
-    p[128] = uint2{w[1][0], w[1][1]};
+// Operand whose free index is the row of a row-major plane or tile (contracted index along the row).
+__device__ __forceinline__ f32x4 row_frag(const float* p, int ld, const Lane& L) {
+    return *reinterpret_cast<const f32x4*>(p + L.r16 * ld + 4 * L.g4);
 }
-__device__ __forceinline__ Split8<2> mem_operand(const float* m, int f) {
-    const uint4* p = reinterpret_cast<const uint4*>(m) + (uint32_t)(f * 128 + (threadIdx.x & 63));
-    Split8<2> a;
-    a.p[0] = __builtin_bit_cast(bf16x8, p[0]);
-    a.p[1] = __builtin_bit_cast(bf16x8, p[64]);
-    return a;
+// Operand whose free index is the column (contracted index down the rows).
+__device__ __forceinline__ f32x4 col_frag(const float* p, int ld, const Lane& L) {
+    const float* q = p + 4 * L.g4 * ld + L.r16;
+    return f32x4{q[0], q[ld], q[2 * ld], q[3 * ld]};
+}
+__device__ __forceinline__ void put_tile(float* p, int ld, const Lane& L, const f32x4& x) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) p[(4 * L.g4 + r) * ld + L.r16] = x[r];
+}
+// Four consecutive 16-bit elements of an LDS row as an operand.
+template <typename T>
+__device__ __forceinline__ f32x4 row_frag16(const T* p, int ld, const Lane& L) {
+    typedef T v4 __attribute__((ext_vector_type(4)));
+    const v4 x = *reinterpret_cast<const v4*>(p + L.r16 * ld + 4 * L.g4);
+    return f32x4{(float)x[0], (float)x[1], (float)x[2], (float)x[3]};
 }
 
 // A chunk's rows of one 16-bit tensor: records end at the last valid row, so rows past it read as
@@ -154,105 +168,6 @@ __device__ __forceinline__ void store_rows(const Rows& a, const f32x4 (&x)[4]) {
         for (int e = 0; e < 16; ++e)
             __builtin_amdgcn_raw_buffer_store_b16(u[e], a.r, a.lane + (16 * (e >> 2) + (e & 3)) * a.st, 0, 0);
     }
-}
-
-// ---- operands in bf16 parts ---------------------------------------------------------------
-// A K = 32 operand covers two 16-wide blocks: K slots 0..3 of a lane are rows 4 g4 + r of the first
-// block, 4..7 those of the second (as lds_frag and lds_frag_tr of chunk_common.h read them).
-__device__ __forceinline__ Split8<2> split_pair(const f32x4& lo, const f32x4& hi) {
-    const float x[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-    return split8<2>(x);
-}
-// Three products of two split operands (two where a is bf16 as it stands).
-template <int NA>
-__device__ __forceinline__ f32x4 mms(const Split8<NA>& a, const Split8<2>& b, const f32x4& c) {
-    return mfma_split<NA, 2, 2>(a, b, c);
-}
-
-// Column block x (accumulator layout) of rows row0 + [0, 16) and column col into NP planes.
-template <int NP, int D>
-__device__ __forceinline__ void put_col(char* base, int row0, int col, const Lane& L, const f32x4& x) {
-    using PL = Plane<D>;
-    float r[4] = {x[0], x[1], x[2], x[3]};
-    uint32_t w[NP][2];
-    split_pairs<NP, 2>(r, w);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int row = 4 * L.g4 + e;
-        uint16_t* p = reinterpret_cast<uint16_t*>(base) + (row0 + row) * PL::RS + PL::unit(col & ~3, PL::swz(row)) + (col & 3);
-#pragma unroll
-        for (int pl = 0; pl < NP; ++pl) p[pl * (PL::BYTES / 2)] = (uint16_t)(w[pl][e >> 1] >> (16 * (e & 1)));
-    }
-}
-
-// Lower-triangular tiles in two bf16 parts: part n of tile t at t * TLB + n * TLB / 2, rows TSR apart.
-__device__ __forceinline__ void put_ltile(char* tiles, int t, const Lane& L, const f32x4& x) {
-    float r[4] = {x[0], x[1], x[2], x[3]};
-    uint32_t w[2][2];
-    split_pairs<2, 2>(r, w);
-    uint16_t* p = reinterpret_cast<uint16_t*>(tiles + t * TLB) + 4 * L.g4 * TSR + L.r16;
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int pl = 0; pl < 2; ++pl) p[pl * TSZ + e * TSR] = (uint16_t)(w[pl][e >> 1] >> (16 * (e & 1)));
-}
-__device__ __forceinline__ bf16x4 tile_row(const char* tiles, int t, int part, const Lane& L) {
-    return *reinterpret_cast<const bf16x4*>(reinterpret_cast<const __bf16*>(tiles + t * TLB + part * (TLB / 2)) +
-                                            L.r16 * TSR + 4 * L.g4);
-}
-__device__ __forceinline__ bf16x4 tile_col(const char* tiles, int t, int part, const Lane& L) {
-    return lds_read_tr(reinterpret_cast<const __bf16*>(tiles + t * TLB + part * (TLB / 2)) +
-                       (4 * L.g4 + (L.r16 >> 2)) * TSR + 4 * (L.r16 & 3));
-}
-// Operand over tiles t0 (K slots 0..3) and t1 (4..7); a negative index stands for a zero tile.
-// TR: the tiles' transposes.
-template <bool TR>
-__device__ __forceinline__ Split8<2> tile_frag(const char* tiles, int t0, int t1, const Lane& L) {
-    Split8<2> f;
-#pragma unroll
-    for (int n = 0; n < 2; ++n) {
-        bf16x4 a = {}, b = {};
-        if (t0 >= 0) a = TR ? tile_col(tiles, t0, n, L) : tile_row(tiles, t0, n, L);
-        if (t1 >= 0) b = TR ? tile_col(tiles, t1, n, L) : tile_row(tiles, t1, n, L);
-        f.p[n] = bf16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
-    }
-    return f;
-}
-// Element (row, col) of the lower-triangular matrix.
-__device__ __forceinline__ float tile_at(const char* tiles, int row, int col) {
-    const __bf16* p = reinterpret_cast<const __bf16*>(tiles + tl(row >> 4, col >> 4) * TLB) + (row & 15) * TSR + (col & 15);
-    return (float)p[0] + (float)p[TSZ];
-}
-__device__ __forceinline__ int lower_index(int i, int j) { return i >= j ? tl(i, j) : -1; }
-
-// X <- Lt X (or Lt^T X) for a lower-triangular Lt in tiles and a 64-row column block X given as the
-// two K = 32 operands b: acc[i] += ...
-template <bool TR>
-__device__ __forceinline__ void mul_lower(const char* tiles, const Split8<2> (&b)[2], const Lane& L, f32x4 (&acc)[4]) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            if (TR ? ks < i / 2 : ks > i / 2) continue;
-            const int t0 = TR ? lower_index(2 * ks, i) : lower_index(i, 2 * ks);
-            const int t1 = TR ? lower_index(2 * ks + 1, i) : lower_index(i, 2 * ks + 1);
-            acc[i] = mms(tile_frag<TR>(tiles, t0, t1, L), b[ks], acc[i]);
-        }
-}
-// The same for rows of 16-bit elements known to fit NX bf16 parts.
-template <int NX>
-__device__ __forceinline__ void mul_lower_x(const char* tiles, const Split8<NX> (&b)[2], const Lane& L, f32x4 (&acc)[4]) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int ks = i / 2; ks < 2; ++ks)
-            acc[i] = mfma_split<2, NX, 2>(
-                tile_frag<true>(tiles, lower_index(2 * ks, i), lower_index(2 * ks + 1, i), L), b[ks], acc[i]);
-}
-template <int NX>
-__device__ __forceinline__ Split8<NX> split_pair_x(const f32x4& lo, const f32x4& hi) {
-    const float x[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-    return split8<NX>(x);
 }
 
 // Sum over the four row groups, in every lane.
@@ -356,26 +271,39 @@ __device__ __forceinline__ Rows out_rows(const GdnChunkBwdParams& p, void* o, co
     return rows_at<T>(o, ((k.b * p.f.T + k.c * GC) * p.f.H + k.h) * D, p.f.H * D, D, col, k.nv, L);
 }
 
-// X_i = T_ii (R_i - sum_{j<i} L_ij X_j), in place (TR: with the transpose, X_i = T_ii^T (R_i -
-// sum_{j>i} L_ji^T X_j)).  tiles: T_ii on the diagonal, -L_ij below it.
-template <bool TR>
-__device__ __forceinline__ void solve(const char* tiles, const Lane& L, f32x4 (&x)[4]) {
+// X_i = T_ii (R_i - sum_{j<i} L_ij X_j), in place.  tiles: T_ii on the diagonal, -L_ij below it.
+__device__ __forceinline__ void solve(const float* tiles, const Lane& L, f32x4 (&x)[4]) {
 #pragma unroll
-    for (int ii = 0; ii < 4; ++ii) {
-        const int i = TR ? 3 - ii : ii;
+    for (int i = 0; i < 4; ++i) {
         f32x4 a = x[i];
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            // blocks 2 ks and 2 ks + 1 that are already solved
-            const bool u0 = TR ? 2 * ks > i : 2 * ks < i, u1 = TR ? 2 * ks + 1 > i : 2 * ks + 1 < i;
-            if (!u0 && !u1) continue;
-            const int t0 = u0 ? (TR ? tl(2 * ks, i) : tl(i, 2 * ks)) : -1;
-            const int t1 = u1 ? (TR ? tl(2 * ks + 1, i) : tl(i, 2 * ks + 1)) : -1;
-            a = mms(tile_frag<TR>(tiles, t0, t1, L),
-                    split_pair(u0 ? x[2 * ks] : zero4(), u1 ? x[2 * ks + 1] : zero4()), a);
-        }
-        x[i] = mms(tile_frag<TR>(tiles, tl(i, i), -1, L), split_pair(a, zero4()), zero4());
+        for (int j = 0; j < i; ++j) a = mma(row_frag(tiles + tl(i, j) * TSZ, TSR, L), x[j], a);
+        x[i] = mma(row_frag(tiles + tl(i, i) * TSZ, TSR, L), a, zero4());
     }
+}
+// The same with the transpose: X_i = T_ii^T (Y_i - sum_{j>i} L_ji^T X_j).
+__device__ __forceinline__ void solve_t(const float* tiles, const Lane& L, f32x4 (&x)[4]) {
+#pragma unroll
+    for (int i = 3; i >= 0; --i) {
+        f32x4 a = x[i];
+#pragma unroll
+        for (int j = 3; j > i; --j) a = mma(col_frag(tiles + tl(j, i) * TSZ, TSR, L), x[j], a);
+        x[i] = mma(col_frag(tiles + tl(i, i) * TSZ, TSR, L), a, zero4());
+    }
+}
+// acc += Lt^T X for a lower-triangular Lt in tiles and a 64-row column block X.
+__device__ __forceinline__ void mul_lower_t(const float* tiles, const f32x4 (&x)[4], const Lane& L, f32x4 (&acc)[4]) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = j; i < 4; ++i) acc[j] = mma(col_frag(tiles + tl(i, j) * TSZ, TSR, L), x[i], acc[j]);
+}
+// acc += Lt X.
+__device__ __forceinline__ void mul_lower(const float* tiles, const f32x4 (&x)[4], const Lane& L, f32x4 (&acc)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j <= i; ++j) acc[i] = mma(row_frag(tiles + tl(i, j) * TSZ, TSR, L), x[j], acc[i]);
 }
 
 __device__ __forceinline__ void tile_ij(int n, int& i, int& j) {
@@ -395,20 +323,14 @@ __device__ __forceinline__ f32x4 lower(const f32x4& x, bool on_diag, bool with_d
     return y;
 }
 
-// The 2 NTL split tiles between LDS (padded rows) and memory (1 KB each).  NT: threads.
+// The 2 NTL tiles between LDS (padded rows) and memory (1 KB each).  NT: threads.
 template <bool OUT, int NT>
-__device__ __forceinline__ void copy_tiles(char* tiles, float* mem) {
+__device__ __forceinline__ void copy_tiles(float* tiles, float* mem) {
     for (int n = threadIdx.x; n < 2 * NTL * 64; n += NT) {
-        uint2* l = reinterpret_cast<uint2*>(tiles + (n >> 6) * TLB + ((n >> 5) & 1) * (TLB / 2) +
-                                            ((n >> 1) & 15) * (TSR * 2) + (n & 1) * 16);
-        uint4* m = reinterpret_cast<uint4*>(mem) + n;
-        if constexpr (OUT) {
-            *m = uint4{l[0].x, l[0].y, l[1].x, l[1].y};
-        } else {
-            const uint4 u = *m;
-            l[0] = uint2{u.x, u.y};
-            l[1] = uint2{u.z, u.w};
-        }
+        f32x4* l = reinterpret_cast<f32x4*>(tiles + (n >> 6) * TSZ + ((n >> 2) & 15) * TSR + (n & 3) * 4);
+        f32x4* m = reinterpret_cast<f32x4*>(mem) + n;
+        if constexpr (OUT) *m = *l;
+        else *l = *m;
     }
 }
 
@@ -418,29 +340,23 @@ __device__ __forceinline__ void copy_tiles(char* tiles, float* mem) {
 template <int D>
 struct MapLay {
     static constexpr int NW = D / 16;
-    static constexpr int ROWP = Plane<D>::BYTES;
-    static constexpr int BYTES = 3 * 2 * ROWP + 2 * NTL * TLB + GC * 4;
+    static constexpr int LD = D + 4;  // rows 4 banks apart for row reads, 4 rows 16 banks apart for column reads
+    static constexpr int PL = GC * LD;
+    static constexpr int BYTES = (3 * PL + 2 * NTL * TSZ + GC) * 4;
 };
 
-// Element (t, s) of a lower-triangular matrix into the split tiles (wide chunks).
-__device__ __forceinline__ void put_at(char* tiles, int t, int s, float x) {
-    __bf16* p = reinterpret_cast<__bf16*>(tiles + tl(t >> 4, s >> 4) * TLB) + (t & 15) * TSR + (s & 15);
-    p[0] = (__bf16)x;
-    p[TSZ] = (__bf16)(x - (float)p[0]);
-}
-
+// MFMA-bound: 416 products of 32 cycles per wave and chunk at D = 64 (2 workgroups per CU).
 template <typename T, int D>
 __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_map_kernel(GdnChunkBwdParams p) {
     using Y = MapLay<D>;
-    using PL = Plane<D>;
-    constexpr int NW = Y::NW, NKS = D / 32, NX = Prec<T>::NX;
+    constexpr int NW = Y::NW, LD = Y::LD;
     __shared__ __attribute__((aligned(16))) char smem[Y::BYTES];
-    char* P0 = smem;                   // Qt rows, then Q0
-    char* P1 = P0 + 2 * Y::ROWP;       // Bt rows, then B0
-    char* P2 = P1 + 2 * Y::ROWP;       // Wt rows, then Wc
-    char* sL = P2 + 2 * Y::ROWP;       // T_ii and -L_ij (L_ii in fp32 until it is inverted)
-    char* sA = sL + NTL * TLB;         // A
-    float* sB = reinterpret_cast<float*>(sA + NTL * TLB);  // beta (wide chunks)
+    float* P0 = reinterpret_cast<float*>(smem);  // Qt rows, then Q0
+    float* P1 = P0 + Y::PL;                      // Bt rows, then B0
+    float* P2 = P1 + Y::PL;                      // Wt rows, then Wc
+    float* sL = P2 + Y::PL;                      // T_ii and -L_ij
+    float* sA = sL + NTL * TSZ;                  // A
+    float* sB = sA + NTL * TSZ;                  // beta (wide chunks)
     const Lane L;
     const int w = L.w, g4 = L.g4, r16 = L.r16, col = 16 * w + r16;
     const Chunk k = chunk_of(p);
@@ -465,34 +381,23 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_map_kernel(GdnChunkBwdParams
     if (!wide) {
         const float m = 0.5f * gc, em = fast_exp(m);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                q[i][r] *= fast_exp(G[i][r] - m);
-                g[i][r] = kk[i][r] * be[i][r] * fast_exp(m - G[i][r]);  // g holds the W rows from here on
-                kk[i][r] *= fast_exp(Gp[i][r] - m);
+                const int a = (16 * i + 4 * g4 + r) * LD + col;
+                P0[a] = q[i][r] *= fast_exp(G[i][r] - m);
+                P2[a] = g[i][r] = kk[i][r] * be[i][r] * fast_exp(m - G[i][r]);  // g holds the W rows from here on
+                P1[a] = kk[i][r] *= fast_exp(Gp[i][r] - m);
             }
-            put_col<2, D>(P0, 16 * i, col, L, q[i]);
-            put_col<2, D>(P1, 16 * i, col, L, kk[i]);
-            put_col<2, D>(P2, 16 * i, col, L, g[i]);
-        }
         lds_sync();
         for (int n = w; n < NTL; n += NW) {
             int i, j;
             tile_ij(n, i, j);
             f32x4 a = zero4();
 #pragma unroll
-            for (int ks = 0; ks < NKS; ++ks)
-                a = mms(PL::template frag<2>(P1, 16 * i, r16, ks, g4),
-                        PL::template frag<2>(P2, 16 * j, r16, ks, g4), a);
-            if (i == j) {
-                a = lower(a, true, false, L);
-                float* t = reinterpret_cast<float*>(sL + n * TLB) + 4 * g4 * TSR + r16;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) t[r * TSR] = a[r];
-            } else {
-                put_ltile(sL, n, L, -a);
-            }
+            for (int kt = 0; kt < NW; ++kt)
+                a = mma(row_frag(P1 + 16 * i * LD + 16 * kt, LD, L), row_frag(P2 + 16 * j * LD + 16 * kt, LD, L), a);
+            put_tile(sL + n * TSZ, TSR, L, i == j ? lower(a, true, false, L) : -a);
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -501,13 +406,9 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_map_kernel(GdnChunkBwdParams
             g[i] *= em;
         }
     } else {
-        // rows of q, k and the decays in fp32; L and A from running products of the decays, a lane
-        // (pair of lanes' elements at D = 128) per key dim
-        constexpr int LD = D;
-        float* F0 = reinterpret_cast<float*>(P0);
-        float* F1 = reinterpret_cast<float*>(P1);
-        float* F2 = reinterpret_cast<float*>(P2);
-        for (int n = threadIdx.x; n < 2 * NTL * TSZ; n += 4 * D) reinterpret_cast<uint32_t*>(sL)[n] = 0u;
+        // rows of q, k and the decays; L and A from running products of the decays, a lane (pair of
+        // lanes' elements at D = 128) per key dim
+        for (int n = threadIdx.x; n < 2 * NTL * TSZ; n += 4 * D) sL[n] = 0.f;
         f32x4 S[4], Se[4];
         token_scan<true>(g, L, S, Se);
 #pragma unroll
@@ -515,9 +416,9 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_map_kernel(GdnChunkBwdParams
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int t = 16 * i + 4 * g4 + r;
-                F0[t * LD + col] = q[i][r];
-                F1[t * LD + col] = kk[i][r];
-                F2[t * LD + col] = fast_exp(g[i][r]);
+                P0[t * LD + col] = q[i][r];
+                P1[t * LD + col] = kk[i][r];
+                P2[t * LD + col] = fast_exp(g[i][r]);
                 if (w == 0 && r16 == 0) sB[t] = be[i][r];
                 q[i][r] *= fast_exp(G[i][r]);
                 g[i][r] = kk[i][r] * be[i][r] * fast_exp(Se[i][r]);
@@ -529,28 +430,26 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_map_kernel(GdnChunkBwdParams
             float run[D / 64], dot = 0.f;
 #pragma unroll
             for (int e = 0; e < D / 64; ++e) {
-                run[e] = sB[s] * F1[s * LD + lane + 64 * e];
-                dot += F0[s * LD + lane + 64 * e] * run[e];
+                run[e] = sB[s] * P1[s * LD + lane + 64 * e];
+                dot += P0[s * LD + lane + 64 * e] * run[e];
             }
             dot = g4_sum(dpp_sum16(dot));
-            if (lane == 0) put_at(sA, s, s, dot);
+            if (lane == 0) sA[tl(s >> 4, s >> 4) * TSZ + (s & 15) * (TSR + 1)] = dot;
             for (int t = s + 1; t < GC; ++t) {
                 float l = 0.f, a = 0.f;
 #pragma unroll
                 for (int e = 0; e < D / 64; ++e) {
                     const int o = t * LD + lane + 64 * e;
-                    l += F1[o] * run[e];
-                    run[e] *= F2[o];
-                    a += F0[o] * run[e];
+                    l += P1[o] * run[e];
+                    run[e] *= P2[o];
+                    a += P0[o] * run[e];
                 }
                 l = g4_sum(dpp_sum16(l));
                 a = g4_sum(dpp_sum16(a));
+                const int o = tl(t >> 4, s >> 4) * TSZ + (t & 15) * TSR + (s & 15);
                 if (lane == 0) {
-                    put_at(sA, t, s, a);
-                    if ((t >> 4) == (s >> 4))
-                        reinterpret_cast<float*>(sL + tl(t >> 4, s >> 4) * TLB)[(t & 15) * TSR + (s & 15)] = l;
-                    else
-                        put_at(sL, t, s, -l);
+                    sL[o] = (t >> 4) == (s >> 4) ? l : -l;
+                    sA[o] = a;
                 }
             }
         }
@@ -558,8 +457,7 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_map_kernel(GdnChunkBwdParams
     lds_sync();
     if (w == 0) {
         // T = (I + L_ii)^-1 of the four diagonal blocks, one column per lane: T[i] = 1[i = c] - sum L[i][k] T[k]
-        char* tile = sL + (g4 * (g4 + 3) / 2) * TLB;
-        const float* t = reinterpret_cast<const float*>(tile);
+        float* t = sL + (g4 * (g4 + 3) / 2) * TSZ;
         float x[16];
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
@@ -573,68 +471,53 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_map_kernel(GdnChunkBwdParams
             }
             x[i] = a;
         }
-        asm volatile("" ::: "memory");  // the parts take the place of the fp32 tile just read
-        __bf16* o = reinterpret_cast<__bf16*>(tile) + r16;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const __bf16 h = (__bf16)x[i];
-            o[i * TSR] = h;
-            o[TSZ + i * TSR] = (__bf16)(x[i] - (float)h);
-        }
+        for (int i = 0; i < 16; ++i) t[i * TSR + r16] = x[i];
     } else if (!wide) {
         for (int n = w - 1; n < NTL; n += NW - 1) {
             int i, j;
             tile_ij(n, i, j);
             f32x4 a = zero4();
 #pragma unroll
-            for (int ks = 0; ks < NKS; ++ks)
-                a = mms(PL::template frag<2>(P0, 16 * i, r16, ks, g4),
-                        PL::template frag<2>(P2, 16 * j, r16, ks, g4), a);
-            put_ltile(sA, n, L, lower(a, i == j, true, L));
+            for (int kt = 0; kt < NW; ++kt)
+                a = mma(row_frag(P0 + 16 * i * LD + 16 * kt, LD, L), row_frag(P2 + 16 * j * LD + 16 * kt, LD, L), a);
+            put_tile(sA + n * TSZ, TSR, L, lower(a, i == j, true, L));
         }
     }
     lds_sync();
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        put_col<2, D>(P0, 16 * i, col, L, q[i]);
-        put_col<2, D>(P1, 16 * i, col, L, kk[i]);
-        put_col<2, D>(P2, 16 * i, col, L, g[i]);
+        put_tile(P0 + 16 * i * LD + 16 * w, LD, L, q[i]);
+        put_tile(P1 + 16 * i * LD + 16 * w, LD, L, kk[i]);
+        put_tile(P2 + 16 * i * LD + 16 * w, LD, L, g[i]);
     }
     copy_tiles<true, 4 * D>(sL, p.ws_t + k.id * (2 * NTL * 256));
     lds_sync();
 
-    float* wm = p.ws_m + k.id * (2 * D * D);  // M, then M^T
+    float* wm = p.ws_m + k.id * (D * D);
     float* wn = p.ws_s + k.id * (D * D);
     float* wk = p.ws_d + k.id * (D * D);
-    solve<false>(sL, L, kk);
-    solve<false>(sL, L, v);
-    const Split8<NX> ds[2] = {split_pair_x<NX>(dO[0], dO[1]), split_pair_x<NX>(dO[2], dO[3])};
+    solve(sL, L, kk);
+    solve(sL, L, v);
     f32x4 z[4] = {zero4(), zero4(), zero4(), zero4()};  // -dR from A^T dO alone
-    mul_lower_x<NX>(sA, ds, L, z);
-    solve<true>(sL, L, z);
-    const Split8<2> xs[2] = {split_pair(kk[0], kk[1]), split_pair(kk[2], kk[3])};
-    const Split8<2> vs[2] = {split_pair(v[0], v[1]), split_pair(v[2], v[3])};
-    const Split8<2> zs[2] = {split_pair(-z[0], -z[1]), split_pair(-z[2], -z[3])};
+    mul_lower_t(sA, dO, L, z);
+    solve_t(sL, L, z);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) z[j] = -z[j];
 #pragma unroll 1
     for (int rt = 0; rt < NW; ++rt) {
-        f32x4 am = zero4(), at = zero4(), an = zero4(), ak = zero4();
+        f32x4 am = zero4(), an = zero4(), ak = zero4();
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            const Split8<2> a = PL::template frag_tr<2>(P2, 32 * ks, rt, g4, r16);
-            am = mms(a, xs[ks], am);
-            at = mms(xs[ks], a, at);  // the same tile transposed
-            an = mms(a, vs[ks], an);
-            ak = mfma_split<2, NX, 2>(PL::template frag_tr<2>(P0, 32 * ks, rt, g4, r16), ds[ks], ak);
-            ak = mms(PL::template frag_tr<2>(P1, 32 * ks, rt, g4, r16), zs[ks], ak);
+        for (int i = 0; i < 4; ++i) {
+            const f32x4 a = col_frag(P2 + 16 * i * LD + 16 * rt, LD, L);
+            am = mma(a, kk[i], am);
+            an = mma(a, v[i], an);
+            ak = mma(col_frag(P0 + 16 * i * LD + 16 * rt, LD, L), dO[i], ak);
+            ak = mma(col_frag(P1 + 16 * i * LD + 16 * rt, LD, L), z[i], ak);
         }
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const float e = (rt == w && r16 == 4 * g4 + r) ? ec : 0.f;
-            am[r] = e - am[r];
-            at[r] = e - at[r];
-        }
-        mem_put_half(wm, rt * NKS + w / 2, w & 1, at);
-        mem_put_half(wm + D * D, w * NKS + rt / 2, rt & 1, am);
+        for (int r = 0; r < 4; ++r) am[r] = ((rt == w && r16 == 4 * g4 + r) ? ec : 0.f) - am[r];
+        mem_put(wm, rt * NW + w, L, am);
         mem_put(wn, rt * NW + w, L, an);
         mem_put(wk, rt * NW + w, L, ak);
     }
@@ -643,78 +526,48 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_map_kernel(GdnChunkBwdParams
 // ---------------------------------------------------------------------------------------
 // Scan over the chunks: S_next = M S + N forwards, D_prev = M^T D + K backwards
 // ---------------------------------------------------------------------------------------
-// One workgroup per (b, h, direction, strip of CT * 16 columns), one wave per 16-row tile.  A step is
-// one chain: the strip's state, split into bf16 parts, crosses the waves through LDS (one barrier),
-// then 3 D / 32 MFMAs.  The operands of the next PF chunks are in flight.  The strips of a (b, h)
-// read the same maps, so its workgroups share an XCD (workgroup x runs on XCD x mod 8); at D = 128
-// two column tiles per wave halve what they read from its L2.
-template <int D, int CT, int PF, bool REV>
-__device__ __forceinline__ void scan_walk(const GdnChunkBwdParams& p, char* sX, int64_t bh, int strip) {
-    constexpr int NW = D / 16, NKS = D / 32, XB = NKS * 2048;  // bytes of a column tile's operands
+// One workgroup per (b, h, direction, strip of 16 columns), one wave per 16-row tile.  A step is one
+// chain: the strip's state crosses the waves through LDS (one barrier), then D / 4 MFMAs of 32 cycles
+// in two chains.  The operands of the next PF chunks are in flight.  The strips of a (b, h) read the
+// same maps, so its workgroups share an XCD (workgroup x runs on XCD x mod 8).
+// Two column tiles per wave at D = 128, which halve what its waves read from L2, ran 2 % slower (235
+// against 229 us at B = 4, H = 12, T = 2048), M stored a second time with its rows contiguous 10 %
+// faster, all of which the map kernel's added stores took back.
+template <int D, int PF, bool REV>
+__device__ __forceinline__ void scan_walk(const GdnChunkBwdParams& p, float* sX, int64_t bh, int strip) {
+    constexpr int NW = D / 16, XLD = D + 4;
     const Lane L;
-    const int w = L.w, lane = threadIdx.x & 63;
+    const int w = L.w;
     const int64_t DD = (int64_t)D * D, base = bh * p.nc;
     float* io = REV ? p.ws_d : p.ws_s;
-    const int own = w * NW + strip * CT;  // this wave's first tile of the state
+    const int own = w * NW + strip;  // this wave's tile of the state
     const float* x0 = REV ? p.dsf : p.f.s0;
-    const int64_t flat = bh * DD + (16 * w + 4 * L.g4) * D + 16 * strip * CT + L.r16;
-    f32x4 x[CT];
+    const int64_t flat = bh * DD + (16 * w + 4 * L.g4) * D + 16 * strip + L.r16;
+    f32x4 x = zero4();
+    if (x0)
 #pragma unroll
-    for (int c = 0; c < CT; ++c) {
-        x[c] = zero4();
-        if (x0)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) x[c][r] = x0[flat + r * D + 16 * c];
-    }
-    Split8<2> mf[PF][NKS];
-    f32x4 yf[PF][CT];
+        for (int r = 0; r < 4; ++r) x[r] = x0[flat + r * D];
+    f32x4 mf[PF][NW], yf[PF];
     auto slot = [&](int64_t n) { return base + (REV ? p.nc - 1 - n : n); };
-    auto fetch = [&](int64_t n, Split8<2>(&m)[NKS], f32x4(&y)[CT]) {
+    auto fetch = [&](int64_t n, f32x4(&m)[NW], f32x4& y) {
         const int64_t c = slot(n);
-        const float* M = p.ws_m + c * 2 * DD + (REV ? DD : 0);
+        const float* M = p.ws_m + c * DD;
 #pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) m[ks] = mem_operand(M, w * NKS + ks);
-#pragma unroll
-        for (int t = 0; t < CT; ++t) y[t] = mem_col(io + c * DD, own + t, L);
+        for (int kt = 0; kt < NW; ++kt) m[kt] = REV ? mem_col(M, kt * NW + w, L) : mem_row(M, w * NW + kt, L);
+        y = mem_col(io + c * DD, own, L);
     };
-    auto step = [&](int64_t n, const Split8<2>(&m)[NKS], const f32x4(&y)[CT]) {
-        char* X = sX + (n & 1) * CT * XB;
-#pragma unroll
-        for (int t = 0; t < CT; ++t) {
-            mem_put(io + slot(n) * DD, own + t, L, x[t]);
-            float r[4] = {x[t][0], x[t][1], x[t][2], x[t][3]};
-            uint32_t u[2][2];
-            split_pairs<2, 2>(r, u);
-#pragma unroll
-            for (int pl = 0; pl < 2; ++pl)
-                *reinterpret_cast<uint2*>(X + t * XB + ((w >> 1) * 2 + pl) * 1024 + lane * 16 + (w & 1) * 8) =
-                    uint2{u[pl][0], u[pl][1]};
-        }
+    auto step = [&](int64_t n, const f32x4(&m)[NW], const f32x4& y) {
+        mem_put(io + slot(n) * DD, own, L, x);
+        float* X = sX + (n & 1) * 16 * XLD;
+        *reinterpret_cast<f32x4*>(X + L.r16 * XLD + 16 * w + 4 * L.g4) = x;
         lds_sync();  // LDS only: the maps in flight need not land
-        f32x4 a[CT][NKS];
-        Split8<2> b[CT][NKS];
+        f32x4 a = y, b = zero4();
 #pragma unroll
-        for (int t = 0; t < CT; ++t)
-#pragma unroll
-            for (int ks = 0; ks < NKS; ++ks) {
-                a[t][ks] = ks ? zero4() : y[t];
-#pragma unroll
-                for (int pl = 0; pl < 2; ++pl)
-                    b[t][ks].p[pl] = *reinterpret_cast<const bf16x8*>(X + t * XB + (ks * 2 + pl) * 1024 + lane * 16);
-            }
-        // CT * NKS independent chains of three
-#pragma unroll
-        for (int e = 0; e < 3; ++e)
-#pragma unroll
-            for (int t = 0; t < CT; ++t)
-#pragma unroll
-                for (int ks = 0; ks < NKS; ++ks)
-                    a[t][ks] = mfma(m[ks].p[e == 2], b[t][ks].p[e == 1], a[t][ks]);
-#pragma unroll
-        for (int t = 0; t < CT; ++t) {
-            x[t] = a[t][0] + a[t][1];
-            if constexpr (NKS == 4) x[t] += a[t][2] + a[t][3];
+        for (int kt = 0; kt < NW; kt += 2) {
+            a = mma(m[kt], row_frag(X + 16 * kt, XLD, L), a);
+            b = mma(m[kt + 1], row_frag(X + 16 * (kt + 1), XLD, L), b);
         }
+        x = a + b;
     };
     // every step of the main loop issues the same loads and stores, so its waits count exactly
     // (steps past the end fetch the last chunk again)
@@ -735,44 +588,40 @@ __device__ __forceinline__ void scan_walk(const GdnChunkBwdParams& p, char* sX, 
     }
     if (REV && p.ds0)
 #pragma unroll
-        for (int c = 0; c < CT; ++c)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) p.ds0[flat + r * D + 16 * c] = x[c][r];
+        for (int r = 0; r < 4; ++r) p.ds0[flat + r * D] = x[r];
 }
 
 template <int D>
-struct ScanPlan {
-    static constexpr int CT = D == 128 ? 2 : 1, PF = D == 128 ? 2 : 4, NS = D / 16 / CT;  // NS: strips
-};
-template <int D>
 __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_scan_kernel(GdnChunkBwdParams p) {
-    using P = ScanPlan<D>;
-    __shared__ __attribute__((aligned(16))) char sX[2 * P::CT * (D / 32) * 2048];
+    constexpr int NS = D / 16, PF = D == 128 ? 2 : 4;  // NS: strips
+    __shared__ __attribute__((aligned(16))) float sX[2 * 16 * (D + 4)];
     const int64_t BH = p.f.B * p.f.H;
     const int64_t slot = blockIdx.x / 8;
-    const int64_t bh = slot / (2 * P::NS) * 8 + blockIdx.x % 8;
+    const int64_t bh = slot / (2 * NS) * 8 + blockIdx.x % 8;
     if (bh >= BH) return;
-    const int s = (int)(slot % (2 * P::NS));
-    if (s < P::NS) scan_walk<D, P::CT, P::PF, false>(p, sX, bh, s);
-    else scan_walk<D, P::CT, P::PF, true>(p, sX, bh, s - P::NS);
+    const int s = (int)(slot % (2 * NS));
+    if (s < NS) scan_walk<D, PF, false>(p, sX, bh, s);
+    else scan_walk<D, PF, true>(p, sX, bh, s - NS);
 }
 
 // ---------------------------------------------------------------------------------------
 // Gradients
 // ---------------------------------------------------------------------------------------
-template <int D, int NX>
+template <int D>
 struct GradLay {
     static constexpr int NW = D / 16;
-    static constexpr int ROWP = Plane<D>::BYTES;
-    static constexpr int BYTES = (2 * 2 + NX) * ROWP + 2 * NTL * TLB + 2 * NW * GC * 4;
+    static constexpr int LD = D + 4;
+    static constexpr int PL = GC * LD;
+    static constexpr int LO = D + 8;  // 16-bit row stride of the dO plane
+    static constexpr int BYTES = (2 * PL + 2 * NTL * TSZ + 2 * NW * GC) * 4 + GC * LO * 2;
 };
 
 // The pair sums of a wide chunk for the lane's key dim and its 16 tokens: running products of the
 // decays from each token outwards, with the other tokens' rows read again from memory.  pq and pb
 // go to rows of two LDS planes, pw to rows of D floats in memory (the lane's own elements).
 template <typename T, int D, int LD>
-__device__ __forceinline__ void wide_pairs(const GdnChunkBwdParams& p, const Chunk& k, int col, const char* sdA,
-                                        const char* sdL, float* pq, float* pb, float* pw) {
+__device__ __forceinline__ void wide_pairs(const GdnChunkBwdParams& p, const Chunk& k, int col, const float* sdA,
+                                        const float* sdL, float* pq, float* pb, float* pw) {
     const Lane L;
     auto row0 = [&](const void* x, int64_t sb, int64_t st, int64_t sh, int c) {
         return reinterpret_cast<const T*>(x) + k.b * sb + k.c * GC * st + k.h * sh + c;
@@ -794,21 +643,23 @@ __device__ __forceinline__ void wide_pairs(const GdnChunkBwdParams& p, const Chu
             float rq = 1.f, rb = 1.f;  // products of the decays over (s, t] and (s, t - 1]
 #pragma unroll 1
             for (int s = t; s >= 0; --s) {
+                const int o = tl(t >> 4, s >> 4) * TSZ + (t & 15) * TSR + (s & 15);
                 const float ws = wrow(s), a = decay(s);
-                aq += tile_at(sdA, t, s) * ws * rq;
+                aq += sdA[o] * ws * rq;
                 if (s < t) {
-                    ab += tile_at(sdL, t, s) * ws * rb;
+                    ab += sdL[o] * ws * rb;
                     rb *= a;
                 }
                 rq *= a;
             }
             float rw = 1.f;
-            aw = tile_at(sdA, t, t) * (float)q[t * p.f.q_st];
+            aw = sdA[tl(t >> 4, t >> 4) * TSZ + (t & 15) * (TSR + 1)] * (float)q[t * p.f.q_st];
 #pragma unroll 1
             for (int s = t + 1; s < k.nv; ++s) {
-                aw += tile_at(sdL, s, t) * (float)kr[s * p.f.k_st] * rw;
+                const int o = tl(s >> 4, t >> 4) * TSZ + (s & 15) * TSR + (t & 15);
+                aw += sdL[o] * (float)kr[s * p.f.k_st] * rw;
                 rw *= decay(s);
-                aw += tile_at(sdA, s, t) * (float)q[s * p.f.q_st] * rw;
+                aw += sdA[o] * (float)q[s * p.f.q_st] * rw;
             }
         }
         pq[t * LD + col] = aq;
@@ -817,19 +668,18 @@ __device__ __forceinline__ void wide_pairs(const GdnChunkBwdParams& p, const Chu
     }
 }
 
+// MFMA-bound: 680 products of 32 cycles per wave and chunk at D = 64 (2 workgroups per CU).
 template <typename T, int D>
 __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_grad_kernel(GdnChunkBwdParams p) {
-    constexpr int NX = Prec<T>::NX;
-    using Y = GradLay<D, NX>;
-    using PL = Plane<D>;
-    constexpr int NW = Y::NW, NKS = D / 32;
+    using Y = GradLay<D>;
+    constexpr int NW = Y::NW, LD = Y::LD, LO = Y::LO;
     __shared__ __attribute__((aligned(16))) char smem[Y::BYTES];
-    char* P1 = smem;                  // B0 rows, then U
-    char* P2 = P1 + 2 * Y::ROWP;      // Wc rows, then dR
-    char* sO = P2 + 2 * Y::ROWP;      // dO rows
-    char* sL = sO + NX * Y::ROWP;     // T_ii and -L_ij, then dL
-    char* sA = sL + NTL * TLB;        // A, then dA
-    float* red = reinterpret_cast<float*>(sA + NTL * TLB);  // [2][NW][64] sums over each wave's key dims
+    float* P1 = reinterpret_cast<float*>(smem);  // B0 rows, then U
+    float* P2 = P1 + Y::PL;                      // Wc rows, then dR
+    float* sL = P2 + Y::PL;                      // T_ii and -L_ij, then dL
+    float* sA = sL + NTL * TSZ;                  // A, then dA
+    float* red = sA + NTL * TSZ;                 // [2][NW][64] sums over each wave's key dims
+    T* sO = reinterpret_cast<T*>(red + 2 * NW * GC);  // dO rows
     const Lane L;
     const int w = L.w, g4 = L.g4, r16 = L.r16, col = 16 * w + r16;
     const Chunk k = chunk_of(p);
@@ -868,17 +718,14 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_grad_kernel(GdnChunkBwdParam
             for (int r = 0; r < 4; ++r) ew[i][r] = fast_exp(gc - G[i][r]);
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        f32x4 b0, wc;
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            b0[r] = kk[i][r] * fast_exp(Gp[i][r]);
-            wc[r] = kk[i][r] * be[i][r] * ew[i][r];
+            const int t = 16 * i + 4 * g4 + r;
+            P1[t * LD + col] = kk[i][r] * fast_exp(Gp[i][r]);
+            P2[t * LD + col] = kk[i][r] * be[i][r] * ew[i][r];
+            sO[t * LO + col] = (T)dO[i][r];
         }
-        put_col<2, D>(P1, 16 * i, col, L, b0);
-        put_col<2, D>(P2, 16 * i, col, L, wc);
-        put_col<NX, D>(sO, 16 * i, col, L, dO[i]);
-    }
     copy_tiles<false, 4 * D>(sL, p.ws_t + k.id * (2 * NTL * 256));
     lds_sync();
 
@@ -886,29 +733,24 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_grad_kernel(GdnChunkBwdParam
     const float* Dn = p.ws_d + k.id * (D * D);
     // value columns [16 w, 16 w + 16): U in v, dR in z
     f32x4 z[4] = {zero4(), zero4(), zero4(), zero4()};
-    {
-        const Split8<NX> ds[2] = {split_pair_x<NX>(dO[0], dO[1]), split_pair_x<NX>(dO[2], dO[3])};
-        mul_lower_x<NX>(sA, ds, L, z);
-    }
-#pragma unroll 1
-    for (int ks = 0; ks < NKS; ++ks) {
-        const int o = 2 * ks * NW + w;
-        const Split8<2> s = split_pair(-mem_col(S, o, L), -mem_col(S, o + NW, L));
-        const Split8<2> d = split_pair(mem_col(Dn, o, L), mem_col(Dn, o + NW, L));
+    mul_lower_t(sA, dO, L, z);
+#pragma unroll 2
+    for (int kt = 0; kt < NW; ++kt) {
+        const f32x4 s = -mem_col(S, kt * NW + w, L), d = mem_col(Dn, kt * NW + w, L);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            v[i] = mms(PL::template frag<2>(P1, 16 * i, r16, ks, g4), s, v[i]);
-            z[i] = mms(PL::template frag<2>(P2, 16 * i, r16, ks, g4), d, z[i]);
+            v[i] = mma(row_frag(P1 + 16 * i * LD + 16 * kt, LD, L), s, v[i]);
+            z[i] = mma(row_frag(P2 + 16 * i * LD + 16 * kt, LD, L), d, z[i]);
         }
     }
-    solve<false>(sL, L, v);
-    solve<true>(sL, L, z);
+    solve(sL, L, v);
+    solve_t(sL, L, z);
     store_rows<T>(out_rows<T, D>(p, p.dv, k, col, L), z);
     lds_sync();
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        put_col<2, D>(P1, 16 * i, col, L, v[i]);
-        put_col<2, D>(P2, 16 * i, col, L, z[i]);
+        put_tile(P1 + 16 * i * LD + 16 * w, LD, L, v[i]);
+        put_tile(P2 + 16 * i * LD + 16 * w, LD, L, z[i]);
     }
     lds_sync();
     for (int n = w; n < 2 * NTL; n += NW) {
@@ -916,14 +758,17 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_grad_kernel(GdnChunkBwdParam
         int i, j;
         tile_ij(isA ? n : n - NTL, i, j);
         f32x4 a = zero4();
+        if (isA) {
 #pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) {
-            const Split8<2> u = PL::template frag<2>(P1, 16 * j, r16, ks, g4);
-            if (isA) a = mms(PL::template frag<NX>(sO, 16 * i, r16, ks, g4), u, a);
-            else a = mms(PL::template frag<2>(P2, 16 * i, r16, ks, g4), u, a);
+            for (int kt = 0; kt < NW; ++kt)
+                a = mma(row_frag16(sO + 16 * i * LO + 16 * kt, LO, L), row_frag(P1 + 16 * j * LD + 16 * kt, LD, L), a);
+            put_tile(sA + n * TSZ, TSR, L, lower(a, i == j, true, L));
+        } else {
+#pragma unroll
+            for (int kt = 0; kt < NW; ++kt)
+                a = mma(row_frag(P2 + 16 * i * LD + 16 * kt, LD, L), row_frag(P1 + 16 * j * LD + 16 * kt, LD, L), a);
+            put_tile(sL + (n - NTL) * TSZ, TSR, L, -lower(a, i == j, false, L));
         }
-        if (isA) put_ltile(sA, n, L, lower(a, i == j, true, L));
-        else put_ltile(sL, n - NTL, L, -lower(a, i == j, false, L));
     }
     lds_sync();
 
@@ -932,19 +777,16 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_grad_kernel(GdnChunkBwdParam
     float es = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) aq[i] = ab[i] = aw[i] = zero4();
-#pragma unroll 1
-    for (int ks = 0; ks < NKS; ++ks) {
-        const int o = w * NW + 2 * ks;
-        const f32x4 s0 = mem_row(S, o, L), s1 = mem_row(S, o + 1, L);
-        const f32x4 d0 = mem_row(Dn, o, L), d1 = mem_row(Dn, o + 1, L);
+#pragma unroll 2
+    for (int kt = 0; kt < NW; ++kt) {
+        const f32x4 s = mem_row(S, w * NW + kt, L), d = mem_row(Dn, w * NW + kt, L);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) es = fmaf(s0[r], d0[r], fmaf(s1[r], d1[r], es));
-        const Split8<2> s = split_pair(s0, s1), d = split_pair(d0, d1);
+        for (int r = 0; r < 4; ++r) es = fmaf(s[r], d[r], es);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            aq[i] = mms(PL::template frag<NX>(sO, 16 * i, r16, ks, g4), s, aq[i]);
-            ab[i] = mms(PL::template frag<2>(P2, 16 * i, r16, ks, g4), s, ab[i]);
-            aw[i] = mms(PL::template frag<2>(P1, 16 * i, r16, ks, g4), d, aw[i]);
+            aq[i] = mma(row_frag16(sO + 16 * i * LO + 16 * kt, LO, L), s, aq[i]);
+            ab[i] = mma(row_frag(P2 + 16 * i * LD + 16 * kt, LD, L), s, ab[i]);
+            aw[i] = mma(row_frag(P1 + 16 * i * LD + 16 * kt, LD, L), d, aw[i]);
         }
     }
     es = g4_sum(es) * fast_exp(gc);
@@ -968,11 +810,8 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_grad_kernel(GdnChunkBwdParam
             for (int r = 0; r < 4; ++r) x[i][r] = kk[i][r] * be[i][r] * fast_exp(m - G[i][r]);
             a[i] = b[i] = zero4();
         }
-        {
-            const Split8<2> xs[2] = {split_pair(x[0], x[1]), split_pair(x[2], x[3])};
-            mul_lower<false>(sA, xs, L, a);
-            mul_lower<false>(sL, xs, L, b);
-        }
+        mul_lower(sA, x, L, a);
+        mul_lower(sL, x, L, b);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
 #pragma unroll
@@ -985,12 +824,8 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_grad_kernel(GdnChunkBwdParam
             }
             a[i] = zero4();
         }
-        {
-            const Split8<2> xs[2] = {split_pair(x[0], x[1]), split_pair(x[2], x[3])};
-            const Split8<2> ys[2] = {split_pair(y[0], y[1]), split_pair(y[2], y[3])};
-            mul_lower<true>(sA, xs, L, a);
-            mul_lower<true>(sL, ys, L, a);
-        }
+        mul_lower_t(sA, x, L, a);
+        mul_lower_t(sL, y, L, a);
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -998,19 +833,16 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_grad_kernel(GdnChunkBwdParam
     } else {
         // once every wave is past its reads of U, dR and D, their places take the three sums
         __syncthreads();
-        constexpr int LD = D;  // an fp32 row takes the place of the two parts' rows
-        float* F1 = reinterpret_cast<float*>(P1);
-        float* F2 = reinterpret_cast<float*>(P2);
-        float* F3 = p.ws_d + k.id * (D * D);
-        wide_pairs<T, D, LD>(p, k, col, sA, sL, F1, F2, F3);
+        float* P3 = p.ws_d + k.id * (D * D);
+        wide_pairs<T, D, LD>(p, k, col, sA, sL, P1, P2, P3);
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int a = (16 * i + 4 * g4 + r) * LD + col;
-                aq[i][r] += F1[a];
-                ab[i][r] += F2[a];
-                aw[i][r] += F3[(16 * i + 4 * g4 + r) * D + col];
+                aq[i][r] += P1[a];
+                ab[i][r] += P2[a];
+                aw[i][r] += P3[(16 * i + 4 * g4 + r) * D + col];
             }
     }
     store_rows<T>(out_rows<T, D>(p, p.dq, k, col, L), aq);
@@ -1065,7 +897,7 @@ hipError_t launch_t(const GdnChunkBwdParams& p, hipStream_t stream) {
     hipLaunchKernelGGL((gdn_bwd_map_kernel<T, D>), dim3(chunks), dim3(4 * D), 0, stream, p);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     const unsigned pairs8 = (unsigned)((p.f.B * p.f.H + 7) / 8 * 8);
-    hipLaunchKernelGGL((gdn_bwd_scan_kernel<D>), dim3(pairs8 * 2 * ScanPlan<D>::NS), dim3(4 * D), 0, stream, p);
+    hipLaunchKernelGGL((gdn_bwd_scan_kernel<D>), dim3(pairs8 * 2 * (D / 16)), dim3(4 * D), 0, stream, p);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     hipLaunchKernelGGL((gdn_bwd_grad_kernel<T, D>), dim3(chunks), dim3(4 * D), 0, stream, p);
     return hipGetLastError();

@@ -176,8 +176,8 @@ struct GdnChunkBwdParams {
     float* ds0;              // [B, H, D, D] or null
     int64_t nc;              // chunks per sequence
     // per (b, h, chunk), in the orders gdn_bwd_chunk.hip reads them
-    float* ws_t;             // ten tiles of (I + L)'s blocks, ten of A, in two bf16 parts
-    float* ws_m;             // M and M^T in two bf16 parts
+    float* ws_t;             // ten tiles of (I + L)'s blocks, ten of A
+    float* ws_m;             // M
     float* ws_s;             // N, then the state entering the chunk
     float* ws_d;             // K, then the gradient reaching the state that leaves it
 };
