@@ -37,7 +37,7 @@ def _check(got, ref, dtype, names):
         assert bool((err <= _ulp(r, dtype) + slack).all()), (name, float((err - _ulp(r, dtype)).max()), slack)
 
 
-def _inputs(B, T, H, D, gate, beta, dtype, seed, steep=None):
+def _inputs(B, T, H, D, gate, beta, dtype, seed, steep=None, resets=False):
     gen = torch.Generator().manual_seed(seed)
     q, k = (F.normalize(torch.randn(B, T, H, D, generator=gen), dim=-1).to(dtype) for _ in range(2))
     v, do = (torch.randn(B, T, H, D, generator=gen).to(dtype) for _ in range(2))
@@ -47,7 +47,8 @@ def _inputs(B, T, H, D, gate, beta, dtype, seed, steep=None):
     g[:, 1::7] = 0.05  # clamped: no gradient
     if steep is not None:
         g[:, : T // 2] = g[:, : T // 2] * steep  # some chunks steep, some not
-        g[:, 5::31] = -float("inf")  # resets
+        if resets:
+            g[:, 5::31] = -float("inf")
     b = torch.sigmoid(torch.randn(B, T, H, generator=gen)).to(dtype) if beta else None
     ds = torch.randn(B, H, D, D, generator=gen)
     return q, k, v, g.to(dtype), b, do, ds
@@ -86,14 +87,16 @@ def test_many_chunks_fp16(dev, D, gate, beta):
     _check(got, ref, torch.float16, NAMES)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("D", [64, 128])
-@pytest.mark.parametrize("gate,beta", [("key", True), ("head", True)])
-def test_steep_and_reset_gates(dev, D, gate, beta):
-    """Chunks that decay by more than 128 nats, with -inf gates that reset the state, beside ordinary
-    ones."""
-    x = _inputs(1, 230, 2, D, gate, beta, torch.bfloat16, seed=D + 9, steep=12.0)
+@pytest.mark.parametrize("gate,beta", [("key", True), ("head", True), ("key", False)])
+@pytest.mark.parametrize("steep,resets", [(1.0, True), (4.0, False), (12.0, True), (40.0, False)])
+def test_steep_and_reset_gates(dev, D, gate, beta, steep, resets, dtype):
+    """Chunks that decay by more than 128 nats beside ordinary ones: by tiles of at most 64 nats, by
+    steeper tiles, and with -inf gates that reset the state."""
+    x = _inputs(1, 230, 2, D, gate, beta, dtype, seed=D + 9, steep=steep * (1 if gate == "key" else 4), resets=resets)
     got, ref = _run(dev, *x)
-    _check(got, ref, torch.bfloat16, NAMES)
+    _check(got, ref, dtype, NAMES)
 
 
 def test_only_the_final_state(dev):

@@ -32,7 +32,7 @@
 // a difference of sums: against 64 bits its error rose from the token-serial kernels' 2.08e-4 to
 // 2.14e-4 (fp16, B = 2, T = 600, H = 4, D = 64, gate per key dim) and elements below 1 % of its rms
 // lost up to eight bits (at 1e-3 to 1e-2 of it 1.6e-4 -> 4.4e-3 of their value).  In fp32 those are
-// 2.08e-4 and 2.1e-4.  Solves with I + L are block substitutions with the inverses of the four diagonal
+// 2.08e-4 and 1.9e-4.  Solves with I + L are block substitutions with the inverses of the four diagonal
 // blocks; dependent products issue back to back (32 cycles each), so the substitutions cost no more
 // than products with an explicit inverse would.
 //
@@ -44,9 +44,15 @@
 // D = 128); the scan by the traffic of M, N, K, S and D (20 D^2 bytes per chunk: 2.8 TB/s at D = 64)
 // and the latency of its steps.
 //
-// A chunk in which some key dim decays by more than GB_SPAN nats forms its pair sums from running
-// products of the decays instead (L and A in the map kernel, [.] in the gradient kernel); the
-// products with S and D use factors of at most 1 everywhere.
+// A chunk in which some key dim decays by more than GB_SPAN nats takes its pair sums ([.], L and A) in
+// two levels.  Between two 16-token tiles the decay from s to t is the rest of s's tile, the tiles
+// between and t's tile up to t, all factors of at most 1.  Within a tile whose dims decay by at most
+// GB_TILE the factors are e^(sum up to t) and e^-(sum up to s); a steeper tile (a reset, -inf) takes
+// running products of its decays token by token.  The products with S and D use factors of at most 1
+// everywhere.  With gates three times as steep, all chunks past GB_SPAN: B=4, H=12, T=8192, D=64 1010 us
+// (ordinary gates 920, token-serial kernels 5036, all pair sums token by token 4320), T=1000 155 (125,
+// 694, 674), B=1, H=4, T=200 50 (45, 123, 297); every tile past GB_TILE (B=4, H=6, T=8192) 770 (2881
+// token-serial).
 #include "chunk_common.h"
 
 namespace triune {
@@ -55,6 +61,7 @@ namespace {
 
 constexpr int GC = 64;            // tokens per chunk
 constexpr float GB_SPAN = 128.f;  // factors within e^(+-64)
+constexpr float GB_TILE = 64.f;   // the same for a tile of a steeper chunk, all on one side
 constexpr float GB_GMIN = -104.f; // e^-104 is 0 in fp32: gates below it (-inf resets) act alike
 constexpr int TSR = 20;           // row stride of a 16 x 16 tile in LDS (floats): rows and columns conflict-free
 constexpr int TSZ = 16 * TSR;
@@ -134,14 +141,14 @@ __device__ __forceinline__ Rows rows_at(const void* base, int64_t off, int64_t s
     return x;
 }
 template <typename T>
-__device__ __forceinline__ float from16(uint16_t u) {
-    if constexpr (std::is_same<T, __bf16>::value) return __uint_as_float((uint32_t)u << 16);
-    else return (float)__builtin_bit_cast(_Float16, u);
+__device__ __forceinline__ float from16(uint32_t u) {
+    if constexpr (std::is_same<T, __bf16>::value) return __uint_as_float(u << 16);
+    else return (float)__builtin_bit_cast(_Float16, (uint16_t)u);
 }
 // x[i][r] = row 16 i + 4 g4 + r of the lane's column.
 template <typename T>
 __device__ __forceinline__ void load_rows(const Rows& a, f32x4 (&x)[4]) {
-    uint16_t u[16];
+    uint32_t u[16];  // one per register: packed pairs would have to land before the next tensor's loads
     if (a.whole) {
 #pragma unroll
         for (int e = 0; e < 16; ++e)
@@ -173,35 +180,41 @@ __device__ __forceinline__ void store_rows(const Rows& a, const f32x4 (&x)[4]) {
 // Sum over the four row groups, in every lane.
 __device__ __forceinline__ float g4_sum(float x) { return xor_sum<32>(xor_sum<16>(x)); }
 
-// Sums over the chunk's tokens of the lane's column in accumulator layout: inc[i][r] over tokens up
-// to and with 16 i + 4 g4 + r, exc[i][r] without it; the total is returned.  REV: from the end.
+// Sums of the lane's column in accumulator layout over the 16 tokens of a tile, on top of run: inc[r]
+// over tokens up to and with 4 g4 + r, exc[r] without it; the tile's total is returned.  REV: from
+// the end.
+template <bool REV>
+__device__ __forceinline__ float scan16(const f32x4& x, float run, const Lane& L, f32x4& inc, f32x4& exc) {
+    float s = 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) s += x[r];
+    const RowPair a = swap16(s);
+    const RowPair b = swap32(a.lo + a.hi);
+    float e = run;
+    if constexpr (REV) {
+        e += (L.g4 & 2) ? 0.f : b.hi;
+        e += (L.g4 & 1) ? 0.f : a.hi;
+    } else {
+        e += (L.g4 & 2) ? b.lo : 0.f;
+        e += (L.g4 & 1) ? a.lo : 0.f;
+    }
+#pragma unroll
+    for (int rr = 0; rr < 4; ++rr) {
+        const int r = REV ? 3 - rr : rr;
+        exc[r] = e;
+        e += x[r];
+        inc[r] = e;
+    }
+    return b.lo + b.hi;
+}
+// The same over the chunk's four tiles: token 16 i + 4 g4 + r in [i][r].
 template <bool REV>
 __device__ __forceinline__ float token_scan(const f32x4 (&x)[4], const Lane& L, f32x4 (&inc)[4], f32x4 (&exc)[4]) {
     float run = 0.f;
 #pragma unroll
     for (int ii = 0; ii < 4; ++ii) {
         const int i = REV ? 3 - ii : ii;
-        float s = 0.f;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) s += x[i][r];
-        const RowPair a = swap16(s);
-        const RowPair b = swap32(a.lo + a.hi);
-        float e = run;
-        if constexpr (REV) {
-            e += (L.g4 & 2) ? 0.f : b.hi;
-            e += (L.g4 & 1) ? 0.f : a.hi;
-        } else {
-            e += (L.g4 & 2) ? b.lo : 0.f;
-            e += (L.g4 & 1) ? a.lo : 0.f;
-        }
-#pragma unroll
-        for (int rr = 0; rr < 4; ++rr) {
-            const int r = REV ? 3 - rr : rr;
-            exc[i][r] = e;
-            e += x[i][r];
-            inc[i][r] = e;
-        }
-        run += b.lo + b.hi;
+        run += scan16<REV>(x[i], run, L, inc[i], exc[i]);
     }
     return run;
 }
@@ -342,7 +355,7 @@ struct MapLay {
     static constexpr int NW = D / 16;
     static constexpr int LD = D + 4;  // rows 4 banks apart for row reads, 4 rows 16 banks apart for column reads
     static constexpr int PL = GC * LD;
-    static constexpr int BYTES = (3 * PL + 2 * NTL * TSZ + GC) * 4;
+    static constexpr int BYTES = (3 * PL + 2 * NTL * TSZ + GC + 7 * D) * 4;
 };
 
 // MFMA-bound: 416 products of 32 cycles per wave and chunk at D = 64 (2 workgroups per CU).
@@ -356,7 +369,8 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_map_kernel(GdnChunkBwdParams
     float* P2 = P1 + Y::PL;                      // Wt rows, then Wc
     float* sL = P2 + Y::PL;                      // T_ii and -L_ij
     float* sA = sL + NTL * TSZ;                  // A
-    float* sB = sA + NTL * TSZ;                  // beta (wide chunks)
+    float* sB = sA + NTL * TSZ;                  // beta (steep tiles)
+    float* sC = sB + GC;                         // wide chunks: decays of tiles (see below)
     const Lane L;
     const int w = L.w, g4 = L.g4, r16 = L.r16, col = 16 * w + r16;
     const Chunk k = chunk_of(p);
@@ -406,52 +420,108 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_map_kernel(GdnChunkBwdParams
             g[i] *= em;
         }
     } else {
-        // rows of q, k and the decays; L and A from running products of the decays, a lane (pair of
-        // lanes' elements at D = 128) per key dim
-        for (int n = threadIdx.x; n < 2 * NTL * TSZ; n += 4 * D) sL[n] = 0.f;
-        f32x4 S[4], Se[4];
-        token_scan<true>(g, L, S, Se);
+        f32x4 inc[4], exc[4];
+        float tot[4];
+        bool steep[4], any = false;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            tot[i] = scan16<false>(g[i], 0.f, L, inc[i], exc[i]);
+            steep[i] = __syncthreads_or(tot[i] < -GB_TILE);
+            any |= steep[i];
+        }
+        if (any) {  // rows of q, k and the decays; a lane (two dims per lane at D = 128) per key dim
+            for (int n = threadIdx.x; n < 2 * NTL * TSZ; n += 4 * D) sL[n] = 0.f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int t = 16 * i + 4 * g4 + r;
+                    P0[t * LD + col] = q[i][r];
+                    P1[t * LD + col] = kk[i][r];
+                    P2[t * LD + col] = fast_exp(g[i][r]);
+                    if (w == 0 && r16 == 0) sB[t] = be[i][r];
+                }
+            lds_sync();
+            const int lane = threadIdx.x & 63;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (!steep[i]) continue;
+                for (int s = w; s < 16; s += NW) {
+                    const int rs = (16 * i + s) * LD + lane;
+                    float run[D / 64], dot = 0.f;
+#pragma unroll
+                    for (int e = 0; e < D / 64; ++e) {
+                        run[e] = sB[16 * i + s] * P1[rs + 64 * e];
+                        dot += P0[rs + 64 * e] * run[e];
+                    }
+                    dot = g4_sum(dpp_sum16(dot));
+                    if (lane == 0) sA[tl(i, i) * TSZ + s * (TSR + 1)] = dot;
+                    for (int t = s + 1; t < 16; ++t) {
+                        float l = 0.f, a = 0.f;
+#pragma unroll
+                        for (int e = 0; e < D / 64; ++e) {
+                            const int o = (16 * i + t) * LD + lane + 64 * e;
+                            l += P1[o] * run[e];
+                            run[e] *= P2[o];
+                            a += P0[o] * run[e];
+                        }
+                        l = g4_sum(dpp_sum16(l));
+                        a = g4_sum(dpp_sum16(a));
+                        if (lane == 0) {
+                            sL[tl(i, i) * TSZ + t * TSR + s] = l;
+                            sA[tl(i, i) * TSZ + t * TSR + s] = a;
+                        }
+                    }
+                }
+            }
+            lds_sync();
+        }
+        // rows decayed within their tile: q and k from its start, w to its end
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int a = (16 * i + 4 * g4 + r) * LD + col;
+                P0[a] = q[i][r] * fast_exp(inc[i][r]);
+                P1[a] = kk[i][r] * fast_exp(exc[i][r]);
+            }
+            scan16<true>(g[i], 0.f, L, inc[i], exc[i]);
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                P2[(16 * i + 4 * g4 + r) * LD + col] = kk[i][r] * be[i][r] * fast_exp(exc[i][r]);
+        }
+        if (g4 == 0) {  // what takes w's rows from their tile's end to the reference of the other row
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sC[i * D + col] = steep[i] ? 0.f : fast_exp(-tot[i]);  // own tile: its start
+            sC[4 * D + col] = fast_exp(tot[1]);  // tiles (2, 0)
+            sC[5 * D + col] = fast_exp(tot[2]);  // (3, 1)
+            sC[6 * D + col] = fast_exp(tot[1] + tot[2]);  // (3, 0)
+        }
+        token_scan<true>(g, L, inc, exc);
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int t = 16 * i + 4 * g4 + r;
-                P0[t * LD + col] = q[i][r];
-                P1[t * LD + col] = kk[i][r];
-                P2[t * LD + col] = fast_exp(g[i][r]);
-                if (w == 0 && r16 == 0) sB[t] = be[i][r];
                 q[i][r] *= fast_exp(G[i][r]);
-                g[i][r] = kk[i][r] * be[i][r] * fast_exp(Se[i][r]);
+                g[i][r] = kk[i][r] * be[i][r] * fast_exp(exc[i][r]);
                 kk[i][r] *= fast_exp(Gp[i][r]);
             }
-        __syncthreads();
-        const int lane = threadIdx.x & 63;
-        for (int s = w; s < GC; s += NW) {
-            float run[D / 64], dot = 0.f;
+        lds_sync();
+        for (int n = w; n < 2 * NTL; n += NW) {
+            const bool isA = n >= NTL;
+            int i, j;
+            tile_ij(isA ? n - NTL : n, i, j);
+            if (i == j && (i == 0 ? steep[0] : (i == 1 ? steep[1] : (i == 2 ? steep[2] : steep[3])))) continue;
+            const float* pr = (isA ? P0 : P1) + 16 * i * LD;
+            const float* pc = sC + (i == j ? i : (i - j == 3 ? 6 : 2 + i)) * D + 4 * g4;
+            f32x4 a = zero4();
 #pragma unroll
-            for (int e = 0; e < D / 64; ++e) {
-                run[e] = sB[s] * P1[s * LD + lane + 64 * e];
-                dot += P0[s * LD + lane + 64 * e] * run[e];
+            for (int kt = 0; kt < NW; ++kt) {
+                f32x4 b = row_frag(P2 + 16 * j * LD + 16 * kt, LD, L);
+                if (i - j != 1) b *= *reinterpret_cast<const f32x4*>(pc + 16 * kt);
+                a = mma(row_frag(pr + 16 * kt, LD, L), b, a);
             }
-            dot = g4_sum(dpp_sum16(dot));
-            if (lane == 0) sA[tl(s >> 4, s >> 4) * TSZ + (s & 15) * (TSR + 1)] = dot;
-            for (int t = s + 1; t < GC; ++t) {
-                float l = 0.f, a = 0.f;
-#pragma unroll
-                for (int e = 0; e < D / 64; ++e) {
-                    const int o = t * LD + lane + 64 * e;
-                    l += P1[o] * run[e];
-                    run[e] *= P2[o];
-                    a += P0[o] * run[e];
-                }
-                l = g4_sum(dpp_sum16(l));
-                a = g4_sum(dpp_sum16(a));
-                const int o = tl(t >> 4, s >> 4) * TSZ + (t & 15) * TSR + (s & 15);
-                if (lane == 0) {
-                    sL[o] = (t >> 4) == (s >> 4) ? l : -l;
-                    sA[o] = a;
-                }
-            }
+            put_tile(sL + n * TSZ, TSR, L, i == j ? lower(a, true, isA, L) : (isA ? a : -a));
         }
     }
     lds_sync();
@@ -616,95 +686,69 @@ struct GradLay {
     static constexpr int BYTES = (2 * PL + 2 * NTL * TSZ + 2 * NW * GC) * 4 + GC * LO * 2;
 };
 
-// The pair sums of a wide chunk for the lane's key dim and its 16 tokens: running products of the
-// decays from each token outwards, with the other tokens' rows read again from memory.  pq and pb
-// go to rows of two LDS planes, pw to rows of D floats in memory (the lane's own elements).
-template <typename T, int D, int LD>
-__device__ __forceinline__ void wide_pairs(const GdnChunkBwdParams& p, const Chunk& k, int col, const float* sdA,
-                                        const float* sdL, float* pq, float* pb, float* pw) {
-    const Lane L;
-    auto row0 = [&](const void* x, int64_t sb, int64_t st, int64_t sh, int c) {
-        return reinterpret_cast<const T*>(x) + k.b * sb + k.c * GC * st + k.h * sh + c;
-    };
-    const T* q = row0(p.f.q, p.f.q_sb, p.f.q_st, p.f.q_sh, col);
-    const T* kr = row0(p.f.k, p.f.k_sb, p.f.k_st, p.f.k_sh, col);
-    const T* gr = row0(p.f.g, p.f.g_sb, p.f.g_st, p.f.g_sh, p.g_head ? 0 : col);
-    const T* br = row0(p.f.beta, p.f.b_sb, p.f.b_st, p.f.b_sh, 0);
-    auto decay = [&](int t) { return fast_exp(gate_val((float)gr[t * p.f.g_st])); };
-    auto wrow = [&](int t) {
-        const float b = p.f.beta_kind == BETA_HEAD ? (float)br[t * p.f.b_st] : 1.f;
-        return b * (float)kr[t * p.f.k_st];
-    };
+// The pair sums inside the steep tiles (bits of mask) for the lane's key dim and its tokens, from
+// running products of the decays.  pq, pa, pk: the dim's column of q, decays and k in planes of 64
+// rows, pbe: beta per token; the lanes of the wave that share the column have filled them.  The sums
+// go to rows of D floats (oq, ob, ow: the dim's column).
+template <typename T, int D>
+__device__ __forceinline__ void steep_pairs(const float* pq, const float* pa, const T* pk, const float* pbe,
+                                            const float* sdA, const float* sdL, int mask, const Lane& L, float* oq,
+                                            float* ob, float* ow) {
+    constexpr int LD = GradLay<D>::LD, LO = GradLay<D>::LO;
 #pragma unroll 1
-    for (int e = 0; e < 16; ++e) {
-        const int t = 16 * (e >> 2) + 4 * L.g4 + (e & 3);
-        float aq = 0.f, ab = 0.f, aw = 0.f;
-        if (t < k.nv) {
-            float rq = 1.f, rb = 1.f;  // products of the decays over (s, t] and (s, t - 1]
-#pragma unroll 1
-            for (int s = t; s >= 0; --s) {
-                const int o = tl(t >> 4, s >> 4) * TSZ + (t & 15) * TSR + (s & 15);
-                const float ws = wrow(s), a = decay(s);
-                aq += sdA[o] * ws * rq;
-                if (s < t) {
-                    ab += sdL[o] * ws * rb;
-                    rb *= a;
-                }
-                rq *= a;
-            }
-            float rw = 1.f;
-            aw = sdA[tl(t >> 4, t >> 4) * TSZ + (t & 15) * (TSR + 1)] * (float)q[t * p.f.q_st];
-#pragma unroll 1
-            for (int s = t + 1; s < k.nv; ++s) {
-                const int o = tl(s >> 4, t >> 4) * TSZ + (s & 15) * TSR + (t & 15);
-                aw += sdL[o] * (float)kr[s * p.f.k_st] * rw;
-                rw *= decay(s);
-                aw += sdA[o] * (float)q[s * p.f.q_st] * rw;
-            }
+    for (int n = 0; n < 16; ++n) {
+        const int i = n >> 2, t = 4 * L.g4 + (n & 3);
+        if (!(mask >> i & 1)) continue;
+        const float *q = pq + 16 * i * LD, *a = pa + 16 * i * LD, *be = pbe + 16 * i;
+        const float *dA = sdA + tl(i, i) * TSZ, *dL = sdL + tl(i, i) * TSZ;
+        const T* k = pk + 16 * i * LO;
+        float rq = 1.f, rb = 1.f, sq = 0.f, sb = 0.f;  // decays over (s, t] and (s, t - 1]
+#pragma unroll 4
+        for (int e = 0; e < 16; ++e) {
+            const int s = (t - e) & 15;
+            const float w = t >= e ? be[s] * (float)k[s * LO] : 0.f, d = a[s * LD];
+            sq = fmaf(dA[t * TSR + s] * w, rq, sq);
+            sb = fmaf((e ? dL[t * TSR + s] : 0.f) * w, rb, sb);
+            rb = e ? rb * d : rb;
+            rq *= d;
         }
-        pq[t * LD + col] = aq;
-        pb[t * LD + col] = ab;
-        pw[t * D + col] = aw;
+        float rw = 1.f, sw = dA[t * (TSR + 1)] * q[t * LD];
+#pragma unroll 3
+        for (int e = 1; e < 16; ++e) {
+            const int s = (t + e) & 15;
+            const float in = t + e < 16 ? rw : 0.f;
+            sw = fmaf(dL[s * TSR + t] * (float)k[s * LO], in, sw);
+            rw *= a[s * LD];
+            sw = fmaf(dA[s * TSR + t] * q[s * LD], t + e < 16 ? rw : 0.f, sw);
+        }
+        const int o = (16 * i + t) * D;
+        oq[o] = sq;
+        ob[o] = sb;
+        ow[o] = sw;
     }
 }
 
-// MFMA-bound: 680 products of 32 cycles per wave and chunk at D = 64 (2 workgroups per CU).
-template <typename T, int D>
-__global__ __launch_bounds__(4 * D, 2) void gdn_bwd_grad_kernel(GdnChunkBwdParams p) {
+// The gradients of one chunk (WIDE: some key dim decays by more than GB_SPAN).  The two forms part at
+// the top of the kernel: one body with both branches spilled 300 registers.
+template <typename T, int D, bool WIDE>
+__device__ __forceinline__ void grad_chunk(const GdnChunkBwdParams& p, const Chunk& k, const Lane& L, char* smem,
+                                           f32x4 (&q)[4], f32x4 (&kk)[4], f32x4 (&g)[4], const f32x4 (&be)[4],
+                                           const f32x4 (&G)[4], const f32x4 (&Gp)[4], float gc, uint32_t pass) {
     using Y = GradLay<D>;
     constexpr int NW = Y::NW, LD = Y::LD, LO = Y::LO;
-    __shared__ __attribute__((aligned(16))) char smem[Y::BYTES];
     float* P1 = reinterpret_cast<float*>(smem);  // B0 rows, then U
     float* P2 = P1 + Y::PL;                      // Wc rows, then dR
     float* sL = P2 + Y::PL;                      // T_ii and -L_ij, then dL
     float* sA = sL + NTL * TSZ;                  // A, then dA
     float* red = sA + NTL * TSZ;                 // [2][NW][64] sums over each wave's key dims
     T* sO = reinterpret_cast<T*>(red + 2 * NW * GC);  // dO rows
-    const Lane L;
     const int w = L.w, g4 = L.g4, r16 = L.r16, col = 16 * w + r16;
-    const Chunk k = chunk_of(p);
-
-    f32x4 q[4], kk[4], g[4], be[4], G[4], Gp[4];
-    load_gate<T, D>(p, k, col, L, g);
-    load_in<T, D>(p.f.q, p.f.q_sb, p.f.q_st, p.f.q_sh, k, col, L, q);
-    load_in<T, D>(p.f.k, p.f.k_sb, p.f.k_st, p.f.k_sh, k, col, L, kk);
-    load_beta<T>(p, k, L, be);
     f32x4 v[4], dO[4];
     load_in<T, D>(p.f.v, p.f.v_sb, p.f.v_st, p.f.v_sh, k, col, L, v);
     load_dout<T, D>(p, k, col, L, dO);
-    uint32_t pass = 0;  // tokens whose gate takes a gradient: not clamped, and not reset to 0
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            if (!(g[i][r] > 0.f) && g[i][r] > GB_GMIN) pass |= 1u << (4 * i + r);
-            g[i][r] = gate_val(g[i][r]);
-        }
-    const float gc = token_scan<false>(g, L, G, Gp);
-    const bool wide = __syncthreads_or(gc < -GB_SPAN);
-    const float m = wide ? 0.f : 0.5f * gc;
+    const float m = 0.5f * gc;
     f32x4 ew[4];  // e^(G_C - G)
-    if (wide) {
+    if constexpr (WIDE) {
         f32x4 S[4], Se[4];
         token_scan<true>(g, L, S, Se);
 #pragma unroll
@@ -802,7 +846,7 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_grad_kernel(GdnChunkBwdParam
         }
     es += g4_sum(ew_sum);  // sum over the value columns of D * S_next
 
-    if (!wide) {
+    if constexpr (!WIDE) {
         f32x4 x[4], y[4], a[4], b[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -831,19 +875,105 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_grad_kernel(GdnChunkBwdParam
 #pragma unroll
             for (int r = 0; r < 4; ++r) aw[j][r] = fmaf(a[j][r], fast_exp(m - G[j][r]), aw[j][r]);
     } else {
-        // once every wave is past its reads of U, dR and D, their places take the three sums
-        __syncthreads();
-        float* P3 = p.ws_d + k.id * (D * D);
-        wide_pairs<T, D, LD>(p, k, col, sA, sL, P1, P2, P3);
+        __syncthreads();  // every wave is past its reads of U, dR and dO
+        // a lane's rows wait in its own places of the planes
+        float* X = P1 + 4 * g4 * LD + col;
+        float* Y = P2 + 4 * g4 * LD + col;
+        auto put = [&](float* p, int i, const f32x4& x) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+            for (int r = 0; r < 4; ++r) p[(16 * i + r) * LD] = x[r];
+        };
+        auto get = [&](const float* p, int i) {
+            const float* q = p + 16 * i * LD;
+            return f32x4{q[0], q[LD], q[2 * LD], q[3 * LD]};
+        };
+        float et[4], ei[4];  // decay of each tile and its inverse (0 where it is steep)
+        int steep = 0;
+        f32x4 inc, exc, x, y;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float t = scan16<true>(g[i], 0.f, L, inc, exc);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) x[r] = kk[i][r] * be[i][r] * fast_exp(exc[r]);
+            put(X, i, x);  // W to its tile's end
+            const bool st = __any(t < -GB_TILE);
+            steep |= st ? 1 << i : 0;
+            et[i] = fast_exp(t);
+            ei[i] = st ? 0.f : fast_exp(-t);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            f32x4 a = zero4(), b = zero4();
+#pragma unroll
+            for (int j = 0; j <= i; ++j) {
+                const f32x4 u = j == i ? get(X, i) * ei[i] : get(X, j);
+                a = mma(row_frag(sA + tl(i, j) * TSZ, TSR, L), u, j && j < i ? a * et[j] : a);
+                b = mma(row_frag(sL + tl(i, j) * TSZ, TSR, L), u, j && j < i ? b * et[j] : b);
+            }
+            scan16<false>(g[i], 0.f, L, inc, exc);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int a = (16 * i + 4 * g4 + r) * LD + col;
-                aq[i][r] += P1[a];
-                ab[i][r] += P2[a];
-                aw[i][r] += P3[(16 * i + 4 * g4 + r) * D + col];
+                aq[i][r] = fmaf(a[r], fast_exp(inc[r]), aq[i][r]);
+                ab[i][r] = fmaf(b[r], fast_exp(exc[r]), ab[i][r]);
             }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            scan16<false>(g[i], 0.f, L, inc, exc);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                x[r] = q[i][r] * fast_exp(inc[r]);
+                y[r] = kk[i][r] * fast_exp(exc[r]);
+            }
+            put(X, i, x);
+            put(Y, i, y);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            f32x4 a = zero4();
+#pragma unroll
+            for (int i = 3; i > j; --i) {
+                a = mma(col_frag(sA + tl(i, j) * TSZ, TSR, L), get(X, i), i < 3 ? a * et[i] : a);
+                a = mma(col_frag(sL + tl(i, j) * TSZ, TSR, L), get(Y, i), a);
+            }
+            // the later tiles' sums decay from this tile's end, its own from its start
+            f32x4 b = mma(col_frag(sA + tl(j, j) * TSZ, TSR, L), get(X, j), zero4());
+            b = mma(col_frag(sL + tl(j, j) * TSZ, TSR, L), get(Y, j), b);
+            scan16<true>(g[j], 0.f, L, inc, exc);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) aw[j][r] = fmaf(fmaf(b[r], ei[j], a[r]), fast_exp(exc[r]), aw[j][r]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (steep) {
+            float* be_w = red + w * GC;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int t = 16 * i + 4 * g4 + r;
+                    P1[t * LD + col] = q[i][r];
+                    P2[t * LD + col] = fast_exp(g[i][r]);
+                    sO[t * LO + col] = (T)kk[i][r];
+                    if (r16 == 0) be_w[t] = be[i][r];
+                }
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            // the chunk's M, S and D have been read: their places take the sums
+            float* o0 = p.ws_m + k.id * (D * D) + col;
+            float* o1 = p.ws_s + k.id * (D * D) + col;
+            float* o2 = p.ws_d + k.id * (D * D) + col;
+            steep_pairs<T, D>(P1 + col, P2 + col, sO + col, be_w, sA, sL, steep, L, o0, o1, o2);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (steep >> i & 1)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int o = (16 * i + 4 * g4 + r) * D;
+                        aq[i][r] += o0[o];
+                        ab[i][r] += o1[o];
+                        aw[i][r] += o2[o];
+                    }
+        }
     }
     store_rows<T>(out_rows<T, D>(p, p.dq, k, col, L), aq);
     // q dq - w dw (x) and k dkB (y): dg_t = D * S_next + sum_{r >= t} x_r + sum_{r > t} y_r
@@ -888,6 +1018,33 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_grad_kernel(GdnChunkBwdParam
         const int64_t at = (k.b * p.f.T + k.c * GC + t) * p.f.H + k.h;
         if (o && t < k.nv) reinterpret_cast<T*>(o)[at] = (T)s;
     }
+}
+
+// MFMA-bound: 680 products of 32 cycles per wave and chunk at D = 64 (2 workgroups per CU).
+template <typename T, int D>
+__global__ __launch_bounds__(4 * D, 2) void gdn_bwd_grad_kernel(GdnChunkBwdParams p) {
+    __shared__ __attribute__((aligned(16))) char smem[GradLay<D>::BYTES];
+    const Lane L;
+    const int col = 16 * L.w + L.r16;
+    const Chunk k = chunk_of(p);
+    f32x4 q[4], kk[4], g[4], be[4], G[4], Gp[4];
+    load_gate<T, D>(p, k, col, L, g);
+    load_in<T, D>(p.f.q, p.f.q_sb, p.f.q_st, p.f.q_sh, k, col, L, q);
+    load_in<T, D>(p.f.k, p.f.k_sb, p.f.k_st, p.f.k_sh, k, col, L, kk);
+    load_beta<T>(p, k, L, be);
+    uint32_t pass = 0;  // tokens whose gate takes a gradient: not clamped, and not reset to 0
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if (!(g[i][r] > 0.f) && g[i][r] > GB_GMIN) pass |= 1u << (4 * i + r);
+            g[i][r] = gate_val(g[i][r]);
+        }
+    asm volatile("" : "+v"(pass));  // the bits, not the sixteen gates, stay in registers
+    const float gc = token_scan<false>(g, L, G, Gp);
+    const bool wide = __syncthreads_or(gc < -GB_SPAN);
+    if (wide) grad_chunk<T, D, true>(p, k, L, smem, q, kk, g, be, G, Gp, gc, pass);
+    else grad_chunk<T, D, false>(p, k, L, smem, q, kk, g, be, G, Gp, gc, pass);
 }
 
 template <typename T, int D>
