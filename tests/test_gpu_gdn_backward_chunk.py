@@ -138,6 +138,23 @@ def test_small_gate_gradients(dev, D, gate, beta):
     assert float(err) <= (2e-6 if gate == "key" else 6e-6) * rms, float(err) / rms
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("gate", ["key", "head"])
+@pytest.mark.parametrize("rate", [1.5, 3.0, 12.0])
+def test_gate_gradients_of_steep_gates(dev, D, gate, rate):
+    """Every gate near -rate (chunks in one piece, by tiles, token by token): each gate's gradient is
+    about e^-rate of a token's products with itself and with the final state's gradient, which must
+    cancel without leaving their rounding behind.  What is left is off by fp32's 2^-24 of up to 64 terms
+    of its own size, with exponents up to 48 nats: 2^-24 (64 + 2 * 48 * log2 e) = 1.2e-5."""
+    q, k, v, g, b, do, ds = _inputs(2, 130, 2, D, gate, gate == "head", torch.bfloat16, seed=D)
+    g = (-rate * (1 + 0.1 * torch.rand(g.shape, generator=torch.Generator().manual_seed(D)))).bfloat16()
+    got, ref = _run(dev, q, k, v, g, b, do, ds)
+    r = torch.as_tensor(np.asarray(ref[3], dtype=np.float64))
+    err = (got[3].double().cpu() - r).abs()
+    assert bool((err <= _ulp(r, torch.bfloat16) + 1.2e-5 * float(r.abs().max())).all()), float(
+        ((err - _ulp(r, torch.bfloat16)) / r.abs().max()).max())
+
+
 @pytest.mark.parametrize("gate", ["key", "head"])
 def test_operator_views_and_padding(dev, gate, monkeypatch):
     """The operator's autograd with strided q, k, v views, a non-contiguous beta and gate, and head

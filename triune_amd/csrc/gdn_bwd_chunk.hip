@@ -13,6 +13,8 @@
 //   dq = e^G (dO S^T) + [dA W],   dkB = -e^Gp (dR S^T) + [dL W],   dw = e^(G_C - G) (U D^T) + [dA^T Q + dL^T B]
 //   dk = beta dw + dkB,   dbeta = sum_d k dw
 //   dg_t = sum_{r >= t} (q dq - w dw)_r + sum_{r > t} (k dkB)_r + sum_c (D * S_next), 0 where g_t > 0
+//        = sum_{r >= t} (q dq - w [.])_r + sum_{r > t} (k dkB)_r + sum_{s < t} w dw'_s + e^G_C sum_c (D * S),
+//          dw' the part of dw through D
 // where [.] are the in-chunk pair sums with their factors e^(G_t - G_s) (or Gp_t), formed as
 // e^(G - m) e^(m - G) around the midpoint m = G_C / 2 of each key dim.
 //
@@ -60,7 +62,7 @@ namespace triune {
 namespace {
 
 constexpr int GC = 64;            // tokens per chunk
-constexpr float GB_SPAN = 128.f;  // factors within e^(+-64)
+constexpr float GB_SPAN = 128.f;  // factors within e^(+-64); a chunk of fewer tokens counts as steep pro rata
 constexpr float GB_TILE = 64.f;   // the same for a tile of a steeper chunk, all on one side
 constexpr float GB_GMIN = -104.f; // e^-104 is 0 in fp32: gates below it (-inf resets) act alike
 constexpr int TSR = 20;           // row stride of a 16 x 16 tile in LDS (floats): rows and columns conflict-free
@@ -324,16 +326,19 @@ __device__ __forceinline__ void tile_ij(int n, int& i, int& j) {
     j = n - tl(i, 0);
 }
 
-// x where the tile entry lies below (or, with diag, on) the diagonal of tile (i, j), else 0.
-__device__ __forceinline__ f32x4 lower(const f32x4& x, bool on_diag, bool with_diag, const Lane& L) {
-    if (!on_diag) return x;
+// x where the entry of tile (i, j) lies at least `from` below the diagonal, else 0 (from at most 2).
+__device__ __forceinline__ f32x4 lower(const f32x4& x, int i, int j, int from, const Lane& L) {
+    if (i - j > 1 || (i != j && from < 2)) return x;
+    const int below = 16 * (i - j) + 4 * L.g4 - L.r16;
     f32x4 y;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int t = 4 * L.g4 + r;
-        y[r] = (t > L.r16 || (with_diag && t == L.r16)) ? x[r] : 0.f;
-    }
+    for (int r = 0; r < 4; ++r) y[r] = below + r >= from ? x[r] : 0.f;
     return y;
+}
+// The entries of tile (i, j) that lie `at` below the diagonal, to p[row].
+__device__ __forceinline__ void put_diag(float* p, const f32x4& x, int i, int j, int at, const Lane& L) {
+    const int u = L.r16 + at - 16 * (i - j);  // row of the lane's column
+    if (u >= 0 && u >> 2 == L.g4) p[16 * i + u] = (u & 2) ? ((u & 1) ? x[3] : x[2]) : ((u & 1) ? x[1] : x[0]);
 }
 
 // The 2 NTL tiles between LDS (padded rows) and memory (1 KB each).  NT: threads.
@@ -385,7 +390,7 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_map_kernel(GdnChunkBwdParams
 #pragma unroll
         for (int r = 0; r < 4; ++r) g[i][r] = gate_val(g[i][r]);
     const float gc = token_scan<false>(g, L, G, Gp);
-    const bool wide = __syncthreads_or(gc < -GB_SPAN);
+    const bool wide = __syncthreads_or(gc < -GB_SPAN / GC * k.nv);
     const float ec = fast_exp(gc);
     // V and dO fly until the products with them
     f32x4 v[4], dO[4];
@@ -411,7 +416,7 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_map_kernel(GdnChunkBwdParams
 #pragma unroll
             for (int kt = 0; kt < NW; ++kt)
                 a = mma(row_frag(P1 + 16 * i * LD + 16 * kt, LD, L), row_frag(P2 + 16 * j * LD + 16 * kt, LD, L), a);
-            put_tile(sL + n * TSZ, TSR, L, i == j ? lower(a, true, false, L) : -a);
+            put_tile(sL + n * TSZ, TSR, L, i == j ? lower(a, i, j, 1, L) : -a);
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -521,7 +526,7 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_map_kernel(GdnChunkBwdParams
                 if (i - j != 1) b *= *reinterpret_cast<const f32x4*>(pc + 16 * kt);
                 a = mma(row_frag(pr + 16 * kt, LD, L), b, a);
             }
-            put_tile(sL + n * TSZ, TSR, L, i == j ? lower(a, true, isA, L) : (isA ? a : -a));
+            put_tile(sL + n * TSZ, TSR, L, i == j ? lower(a, i, j, isA ? 0 : 1, L) : (isA ? a : -a));
         }
     }
     lds_sync();
@@ -551,7 +556,7 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_map_kernel(GdnChunkBwdParams
 #pragma unroll
             for (int kt = 0; kt < NW; ++kt)
                 a = mma(row_frag(P0 + 16 * i * LD + 16 * kt, LD, L), row_frag(P2 + 16 * j * LD + 16 * kt, LD, L), a);
-            put_tile(sA + n * TSZ, TSR, L, lower(a, i == j, true, L));
+            put_tile(sA + n * TSZ, TSR, L, lower(a, i, j, 0, L));
         }
     }
     lds_sync();
@@ -683,7 +688,7 @@ struct GradLay {
     static constexpr int LD = D + 4;
     static constexpr int PL = GC * LD;
     static constexpr int LO = D + 8;  // 16-bit row stride of the dO plane
-    static constexpr int BYTES = (2 * PL + 2 * NTL * TSZ + 2 * NW * GC) * 4 + GC * LO * 2;
+    static constexpr int BYTES = (2 * PL + 2 * NTL * TSZ + (2 * NW + 2) * GC + 4) * 4 + GC * LO * 2;
 };
 
 // The pair sums inside the steep tiles (bits of mask) for the lane's key dim and its tokens, from
@@ -708,11 +713,11 @@ __device__ __forceinline__ void steep_pairs(const float* pq, const float* pa, co
             const int s = (t - e) & 15;
             const float w = t >= e ? be[s] * (float)k[s * LO] : 0.f, d = a[s * LD];
             sq = fmaf(dA[t * TSR + s] * w, rq, sq);
-            sb = fmaf((e ? dL[t * TSR + s] : 0.f) * w, rb, sb);
+            sb = fmaf(dL[t * TSR + s] * w, rb, sb);
             rb = e ? rb * d : rb;
             rq *= d;
         }
-        float rw = 1.f, sw = dA[t * (TSR + 1)] * q[t * LD];
+        float rw = 1.f, sw = 0.f;
 #pragma unroll 3
         for (int e = 1; e < 16; ++e) {
             const int s = (t + e) & 15;
@@ -738,10 +743,12 @@ __device__ __forceinline__ void grad_chunk(const GdnChunkBwdParams& p, const Chu
     constexpr int NW = Y::NW, LD = Y::LD, LO = Y::LO;
     float* P1 = reinterpret_cast<float*>(smem);  // B0 rows, then U
     float* P2 = P1 + Y::PL;                      // Wc rows, then dR
-    float* sL = P2 + Y::PL;                      // T_ii and -L_ij, then dL
-    float* sA = sL + NTL * TSZ;                  // A, then dA
+    float* sL = P2 + Y::PL;                      // T_ii and -L_ij, then dL (WIDE: below its subdiagonal)
+    float* sA = sL + NTL * TSZ;                  // A, then dA below its diagonal
     float* red = sA + NTL * TSZ;                 // [2][NW][64] sums over each wave's key dims
-    T* sO = reinterpret_cast<T*>(red + 2 * NW * GC);  // dO rows
+    float* sD = red + 2 * NW * GC;               // dA's diagonal
+    float* sE = sD + GC;                         // WIDE: dL's subdiagonal, (t, t - 1) at t
+    T* sO = reinterpret_cast<T*>(sE + GC + 4);   // dO rows
     const int w = L.w, g4 = L.g4, r16 = L.r16, col = 16 * w + r16;
     f32x4 v[4], dO[4];
     load_in<T, D>(p.f.v, p.f.v_sb, p.f.v_st, p.f.v_sh, k, col, L, v);
@@ -770,6 +777,7 @@ __device__ __forceinline__ void grad_chunk(const GdnChunkBwdParams& p, const Chu
             P2[t * LD + col] = kk[i][r] * be[i][r] * ew[i][r];
             sO[t * LO + col] = (T)dO[i][r];
         }
+    if (WIDE && threadIdx.x == 0) sE[0] = sE[GC] = 0.f;
     copy_tiles<false, 4 * D>(sL, p.ws_t + k.id * (2 * NTL * 256));
     lds_sync();
 
@@ -806,12 +814,15 @@ __device__ __forceinline__ void grad_chunk(const GdnChunkBwdParams& p, const Chu
 #pragma unroll
             for (int kt = 0; kt < NW; ++kt)
                 a = mma(row_frag16(sO + 16 * i * LO + 16 * kt, LO, L), row_frag(P1 + 16 * j * LD + 16 * kt, LD, L), a);
-            put_tile(sA + n * TSZ, TSR, L, lower(a, i == j, true, L));
+            put_tile(sA + n * TSZ, TSR, L, lower(a, i, j, 1, L));
+            if (i == j) put_diag(sD, a, i, j, 0, L);
         } else {
 #pragma unroll
             for (int kt = 0; kt < NW; ++kt)
                 a = mma(row_frag(P2 + 16 * i * LD + 16 * kt, LD, L), row_frag(P1 + 16 * j * LD + 16 * kt, LD, L), a);
-            put_tile(sL + (n - NTL) * TSZ, TSR, L, -lower(a, i == j, false, L));
+            a = -a;
+            if (WIDE && i - j < 2) put_diag(sE, a, i, j, 1, L);
+            put_tile(sL + (n - NTL) * TSZ, TSR, L, lower(a, i, j, WIDE ? 2 : 1, L));
         }
     }
     lds_sync();
@@ -833,8 +844,9 @@ __device__ __forceinline__ void grad_chunk(const GdnChunkBwdParams& p, const Chu
             aw[i] = mma(row_frag(P1 + 16 * i * LD + 16 * kt, LD, L), d, aw[i]);
         }
     }
-    es = g4_sum(es) * fast_exp(gc);
-    float ew_sum = 0.f;
+    es = g4_sum(es) * fast_exp(gc);  // sum over the value columns of D * e^G_C S
+    f32x4 ad[4];                     // WIDE: dw through D, which joins dw at the end
+    float wd = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -842,9 +854,14 @@ __device__ __forceinline__ void grad_chunk(const GdnChunkBwdParams& p, const Chu
             aq[i][r] *= fast_exp(G[i][r]);
             ab[i][r] *= -fast_exp(Gp[i][r]);
             aw[i][r] *= ew[i][r];
-            ew_sum = fmaf(kk[i][r] * be[i][r], aw[i][r], ew_sum);
+            if constexpr (WIDE) {
+                ad[i][r] = aw[i][r];
+                aw[i][r] = 0.f;
+            } else {
+                wd = fmaf(kk[i][r] * be[i][r], aw[i][r], wd);
+            }
         }
-    es += g4_sum(ew_sum);  // sum over the value columns of D * S_next
+    if constexpr (!WIDE) es += g4_sum(wd);  // ... of D * S_next
 
     if constexpr (!WIDE) {
         f32x4 x[4], y[4], a[4], b[4];
@@ -975,25 +992,74 @@ __device__ __forceinline__ void grad_chunk(const GdnChunkBwdParams& p, const Chu
                     }
         }
     }
-    store_rows<T>(out_rows<T, D>(p, p.dq, k, col, L), aq);
-    // q dq - w dw (x) and k dkB (y): dg_t = D * S_next + sum_{r >= t} x_r + sum_{r > t} y_r
-    f32x4 y[4], inc[4], exc[4];
+    // dg_t takes what crosses t's decay: S to D, S to the tokens from t on (q dq and k dkB), the tokens
+    // before t to D (w dw), and in the pair sums x = q dq - w dw and k dkB over the tokens from t on, where
+    // the pairs on one side of t cancel.  A token's pair with itself (dA) is on one side of every t, and
+    // joins dq and dw afterwards.  In a steep chunk most of dg is far smaller than what cancels, so there
+    // a token's pair with the one before it (dL, no decay between them) joins afterwards too, and w dw
+    // through D is summed up to t instead of over all tokens less those from t on.
+    f32x4 y[4], inc[4], exc[4], pre[4];
+    if constexpr (!WIDE) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 4; ++i) {
+            const f32x4 d = *reinterpret_cast<const f32x4*>(sD + 16 * i + 4 * g4);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const float wdw = kk[i][r] * be[i][r] * aw[i][r];
-            q[i][r] = q[i][r] * aq[i][r] - wdw;
-            y[i][r] = q[i][r] + kk[i][r] * ab[i][r];
-            ab[i][r] = fmaf(be[i][r], aw[i][r], ab[i][r]);
-            aw[i][r] *= kk[i][r];
+            for (int r = 0; r < 4; ++r) {
+                const float wt = kk[i][r] * be[i][r], qt = q[i][r];
+                q[i][r] = qt * aq[i][r] - wt * aw[i][r];
+                y[i][r] = q[i][r] + kk[i][r] * ab[i][r];
+                aq[i][r] = fmaf(d[r], wt, aq[i][r]);
+                aw[i][r] = fmaf(d[r], qt, aw[i][r]);
+                ab[i][r] = fmaf(be[i][r], aw[i][r], ab[i][r]);
+                aw[i][r] *= kk[i][r];
+            }
+            pre[i] = zero4();
         }
+    } else {
+        float wv[4], kn[4];  // w of the token before the lane's four, k of the one behind them
+        float w3 = 0.f, k0 = 0.f;  // w of the last token of the tile before, k of the first one behind
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const RowPair a = swap16(kk[i][3] * be[i][3]), b = swap32(a.hi);
+            wv[i] = g4 == 2 ? b.lo : (g4 ? a.lo : w3);
+            w3 = b.hi;
+        }
+#pragma unroll
+        for (int i = 3; i >= 0; --i) {
+            const RowPair a = swap16(kk[i][0]), b = swap32(a.lo);
+            kn[i] = g4 == 1 ? b.hi : (g4 < 3 ? a.hi : k0);
+            k0 = b.lo;
+        }
+        f32x4 c[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int t = 16 * i + 4 * g4;
+            const f32x4 d = *reinterpret_cast<const f32x4*>(sD + t), e = *reinterpret_cast<const f32x4*>(sE + t);
+            const f32x4 en = {e[1], e[2], e[3], sE[t + 4]};
+            const f32x4 k1 = {kk[i][1], kk[i][2], kk[i][3], kn[i]};
+            float wp = wv[i];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float wt = kk[i][r] * be[i][r], qt = q[i][r];
+                c[i][r] = wt * ad[i][r];
+                q[i][r] = qt * aq[i][r] - wt * aw[i][r];
+                y[i][r] = q[i][r] + kk[i][r] * ab[i][r];
+                aq[i][r] = fmaf(d[r], wt, aq[i][r]);
+                aw[i][r] = fmaf(d[r], qt, fmaf(en[r], k1[r], aw[i][r])) + ad[i][r];
+                ab[i][r] = fmaf(be[i][r], aw[i][r], fmaf(e[r], wp, ab[i][r]));
+                aw[i][r] *= kk[i][r];
+                wp = wt;
+            }
+        }
+        token_scan<false>(c, L, inc, pre);
+    }
+    store_rows<T>(out_rows<T, D>(p, p.dq, k, col, L), aq);
     store_rows<T>(out_rows<T, D>(p, p.dk, k, col, L), ab);
     token_scan<true>(y, L, inc, exc);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) exc[i][r] = (pass >> (4 * i + r) & 1) ? exc[i][r] + q[i][r] + es : 0.f;
+        for (int r = 0; r < 4; ++r) exc[i][r] = (pass >> (4 * i + r) & 1) ? exc[i][r] + q[i][r] + (pre[i][r] + es) : 0.f;
     if (!p.g_head) store_rows<T>(out_rows<T, D>(p, p.dg, k, col, L), exc);
     const bool dbeta = p.f.beta_kind == BETA_HEAD;
     if (!p.g_head && !dbeta) return;
@@ -1042,7 +1108,7 @@ __global__ __launch_bounds__(4 * D, 2) void gdn_bwd_grad_kernel(GdnChunkBwdParam
         }
     asm volatile("" : "+v"(pass));  // the bits, not the sixteen gates, stay in registers
     const float gc = token_scan<false>(g, L, G, Gp);
-    const bool wide = __syncthreads_or(gc < -GB_SPAN);
+    const bool wide = __syncthreads_or(gc < -GB_SPAN / GC * k.nv);
     if (wide) grad_chunk<T, D, true>(p, k, L, smem, q, kk, g, be, G, Gp, gc, pass);
     else grad_chunk<T, D, false>(p, k, L, smem, q, kk, g, be, G, Gp, gc, pass);
 }
