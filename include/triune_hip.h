@@ -380,7 +380,7 @@ int triune_hip_gdn_bwd(const void* q, const void* k, const void* v, const void* 
  * beta and dout in io_dtype, beta none or per (token, head).  With g_head != 0 the gate is one value per
  * (token, head) (strides[9..11] of a [B, T, H] tensor) and dg is [B, T, H], the sum over the key
  * dims; otherwise g and dg are [B, T, H, D].  Other arguments as triune_hip_gdn_bwd; rows need unit
- * innermost stride and token strides of at least D (one value per token: any) and at most 2^31 / 160
+ * innermost stride and (T > 1) token strides of at least D (one value per token: any) and at most 2^31 / 160
  * elements (H D too).  workspace: at least triune_hip_gdn_bwd_chunked_workspace_size(B, T, H, Dk, Dv)
  * bytes, 16-byte aligned.
  * Replaces: autograd through fast_recurrent_gated_deltanet (fast_gla.py:781-836). */

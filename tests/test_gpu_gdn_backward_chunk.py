@@ -123,6 +123,31 @@ def test_gate_and_beta_repeated_over_tokens(dev, D):
 
 
 @pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("shared", ["heads", "cut"])
+def test_one_token_of_token_stride_zero(dev, D, shared):
+    """One token whose rows have token stride 0 (k, v and dO shared by the heads, or cut from a tensor
+    expanded over tokens), with a gradient of the final state: there are no tokens past it."""
+    B, H = 2, 3
+    q, k, v, g, _, do, ds = _inputs(B, 1, H, D, "key", False, torch.bfloat16, seed=D)
+
+    def zero_stride(x):
+        y = x.to(dev)
+        if shared == "heads":
+            y = y[:, :, :1].contiguous().view(B, D).as_strided((B, 1, H, D), (D, 0, 0, 1))
+        else:
+            y = y[:, :1].expand(B, 5, H, D)[:, :1]
+        assert y.stride(1) == 0
+        return y
+
+    x = [zero_stride(t) for t in (q, k, v, g, do)]
+    got = FG._gdn_bwd(x[0], x[1], x[2], x[3], None, None, _lib.BETA_NONE, x[4], ds.to(dev))
+    torch.cuda.synchronize()
+    c = [t.cpu().contiguous() for t in x]
+    ref = O.gdn_bwd(c[0], c[1], c[2], c[3], None, None, c[4], ds)
+    _check(got, ref, torch.bfloat16, NAMES)
+
+
+@pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("gate,beta", [("key", False), ("head", True)])
 def test_small_gate_gradients(dev, D, gate, beta):
     """dg is a difference of sums: fp32 products (2^-24 of each term, exponents up to 26 nats on either

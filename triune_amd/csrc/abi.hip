@@ -1176,9 +1176,12 @@ int triune_hip_gdn_bwd_chunked(const void* q, const void* k, const void* v, cons
     if (reinterpret_cast<uintptr_t>(s0) % 16 || reinterpret_cast<uintptr_t>(ds_final) % 16 ||
         reinterpret_cast<uintptr_t>(ds0) % 16 || reinterpret_cast<uintptr_t>(workspace) % 16)
         return TRIUNE_ERR_LAYOUT;
-    // 64 rows of a tensor are addressed in 32 bits
+    // 64 rows of a tensor are addressed in 32 bits; the one token of T == 1 has no next row, so its
+    // stride (0 in a tensor shared by the heads) is not the kernels' to read rows past it by
+    int64_t tstr[6];
     for (int i = 0; i < 6; ++i) {
-        const int64_t ts = i == 4 && beta_kind == TRIUNE_BETA_NONE ? 0 : (i == 5 && !dout ? 0 : strides[3 * i + 1]);
+        int64_t& ts = tstr[i];
+        ts = i == 4 && beta_kind == TRIUNE_BETA_NONE ? 0 : (i == 5 && !dout ? 0 : (T == 1 ? D : strides[3 * i + 1]));
         if (ts < 0 || ts > 0x7fffffff / 160) return TRIUNE_ERR_LAYOUT;
         // rows are read up to the last token's end: rows of D elements must not overlap
         const bool wide = i < 3 || (i == 3 && !g_head) || (i == 5 && dout);
@@ -1196,15 +1199,15 @@ int triune_hip_gdn_bwd_chunked(const void* q, const void* k, const void* v, cons
     GdnParams& a = p.f;
     a.q = q; a.k = k; a.v = v; a.g = g; a.beta = beta;
     a.io_dt = io_dtype; a.g_dt = g_dtype; a.beta_dt = beta_dtype; a.beta_kind = beta_kind;
-    a.q_sb = strides[0]; a.q_st = strides[1]; a.q_sh = strides[2];
-    a.k_sb = strides[3]; a.k_st = strides[4]; a.k_sh = strides[5];
-    a.v_sb = strides[6]; a.v_st = strides[7]; a.v_sh = strides[8];
-    a.g_sb = strides[9]; a.g_st = strides[10]; a.g_sh = strides[11];
-    a.b_sb = strides[12]; a.b_st = strides[13]; a.b_sh = strides[14];
+    a.q_sb = strides[0]; a.q_st = tstr[0]; a.q_sh = strides[2];
+    a.k_sb = strides[3]; a.k_st = tstr[1]; a.k_sh = strides[5];
+    a.v_sb = strides[6]; a.v_st = tstr[2]; a.v_sh = strides[8];
+    a.g_sb = strides[9]; a.g_st = tstr[3]; a.g_sh = strides[11];
+    a.b_sb = strides[12]; a.b_st = tstr[4]; a.b_sh = strides[14];
     a.s0 = s0;
     a.B = B; a.T = T; a.H = H;
     p.g_head = g_head != 0;
-    p.dout = dout; p.do_sb = strides[15]; p.do_st = strides[16]; p.do_sh = strides[17];
+    p.dout = dout; p.do_sb = strides[15]; p.do_st = tstr[5]; p.do_sh = strides[17];
     p.dsf = ds_final;
     p.dq = dq; p.dk = dk; p.dv = dv; p.dg = dg; p.dbeta = dbeta; p.ds0 = ds0;
     p.nc = (T + 63) / 64;
