@@ -76,15 +76,20 @@ struct Prec {
     static constexpr bool F32 = std::is_same<TIn, float>::value;
     static constexpr int NS = F32 ? 3 : 2;                                             // parts of derived operands
     static constexpr int NX = F32 ? 3 : (std::is_same<TIn, _Float16>::value ? 2 : 1);  // parts of V
-    // Largest chunk decay span (-G_C of a key dim, nats) of the GLA chunk kernels' factored form;
-    // chunks past it run token by token.  16-bit I/O: every factor lies in e^[-64, 64], where both
-    // bf16 parts are normal numbers; the non-causal products, up to e^128, overflow, but they lie
-    // in diagonal tiles, where a bit mask drops them.  fp32 I/O keeps half of that: the exponents'
-    // own rounding (about |x| 2^-24) would otherwise reach the third parts' size.  Gates of
-    // logsigmoid(N(0, 1)), the reference model's at initialisation, span 52 +- 5 nats: with a limit
-    // of 64 one chunk in five (4 heads of 64 dims) ran token by token and held up the whole launch
-    // (1024-token tile from raw projections 102 us against 20 us without such chunks).
-    static constexpr float SPAN_MAX = F32 ? 64.f : 128.f;
+    // Largest chunk decay span (-G_C of a key dim, nats) of the GLA chunk kernels' factored form; chunks
+    // past it run token by token.  The factors e^(G - m), e^(m - G) and the e^m that carried states and
+    // gradients are multiplied by before they are split lie in e^[-SPAN_MAX / 2, SPAN_MAX / 2].  A
+    // product's second bf16 part is a normal number while its operand is above 2^-117 e^(SPAN_MAX / 2):
+    // 5e-22 at 64 nats, 1.4e-18 at 80 (4e-8 at 128, where gradients of 1e-10 came out 0.3 % off and those
+    // of 1e-13 as zero).  Gates of logsigmoid(N(0, 1)), the reference model's at initialisation, span
+    // 52 +- 4 nats, 75 at most: with a limit of 64 one chunk in five (4 heads of 64 dims) ran token by
+    // token and held up the whole launch (1024-token tile from raw projections 102 us against 20 us
+    // without such chunks).  64 nats for fp32 I/O, where the exponents' own rounding (about |x| 2^-24)
+    // would otherwise reach the third parts' size, and for fp32 outputs of 16-bit inputs, which show the
+    // parts' 2^-17: a steeper chunk's stay exact to fp32, as they would be token by token.
+    static constexpr float SPAN_F32 = 64.f;
+    static constexpr float SPAN_MAX = F32 ? SPAN_F32 : 80.f;
+    __device__ __forceinline__ static float span_max(int o_dt) { return o_dt == DT_F32 ? SPAN_F32 : SPAN_MAX; }
 };
 // Log-decay limit of the scalar-gate Gated DeltaNet chunks (gdn_scalar.hip).
 constexpr float GDN_SG_SPAN_MAX = 64.f;

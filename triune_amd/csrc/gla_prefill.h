@@ -367,7 +367,7 @@ struct OutStep {
             chunk_cumsum<DL>(G, GC, lane);
             bool bad = tail_unclamped;
 #pragma unroll
-            for (int i = 0; i < DL; ++i) bad |= !(GC[i] >= -Prec<TIn>::SPAN_MAX);
+            for (int i = 0; i < DL; ++i) bad |= !(GC[i] >= -Prec<TIn>::span_max(oc.dt));
             float mh[DL];  // -m log2(e), m = GC / 2
 #pragma unroll
             for (int i = 0; i < DL; ++i) mh[i] = -0.5f * LOG2E * GC[i];
