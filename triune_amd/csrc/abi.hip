@@ -318,9 +318,8 @@ int triune_hip_gla_decode_step_count(const void* q, const void* k, const void* v
     a.g_sb = strides[6]; a.g_sh = strides[7];
     a.o_sb = strides[8]; a.o_sh = strides[9];
     a.state_in = state_in; a.state_out = state_out; a.slots = slots; a.n_state_rows = n_state_rows;
-    a.offsets = offsets;
     a.o = o; a.B = B; a.H = H;
-    return launch_status(launch_gla_decode(a, Dk, Dv, 4 * device_cus(), (hipStream_t)stream));
+    return launch_status(launch_gla_decode(a, offsets, Dk, Dv, 4 * device_cus(), (hipStream_t)stream));
 }
 
 // ---- the reference's own native decode signatures, on device pointers -----------------------
@@ -1434,7 +1433,7 @@ int triune_hip_gla_fused_decode_step(const void* qkvg, int io_dtype, const int64
     a.o = o; a.o_dt = o_dtype; a.o_sb = o_strides[0]; a.o_sh = o_strides[1];
     a.B = B; a.H = H; a.max_blocks = kFusedDecodeBlocksPerCU * device_cus();
     return launch_status(
-        launch_gla_fused_decode(a, HD, io_dtype, use_rope ? cs_dtype : TRIUNE_DT_F32, state_dtype, (hipStream_t)stream));
+        launch_gla_fused_decode(a, nullptr, HD, io_dtype, use_rope ? cs_dtype : TRIUNE_DT_F32, state_dtype, (hipStream_t)stream));
 }
 
 int triune_hip_gla_fused_decode_step_slots(const void* qkvg, int io_dtype, const int64_t* strides, const void* cos,
@@ -1474,11 +1473,10 @@ int triune_hip_gla_fused_decode_step_slots_count(const void* qkvg, int io_dtype,
     a.has_init = 1; a.save_final = 1;
     a.state_in = state_pool; a.state_out = state_pool;
     a.slots = slots; a.n_state_rows = n_slots;
-    a.offsets = offsets;
     a.o = o; a.o_dt = o_dtype; a.o_sb = o_strides[0]; a.o_sh = o_strides[1];
     a.B = B; a.H = H; a.max_blocks = kFusedDecodeBlocksPerCU * device_cus();
     return launch_status(
-        launch_gla_fused_decode(a, HD, io_dtype, use_rope ? cs_dtype : TRIUNE_DT_F32, state_dtype, (hipStream_t)stream));
+        launch_gla_fused_decode(a, offsets, HD, io_dtype, use_rope ? cs_dtype : TRIUNE_DT_F32, state_dtype, (hipStream_t)stream));
 }
 
 }  // extern "C"

@@ -24,8 +24,13 @@ using Vec4 = T __attribute__((ext_vector_type(4)));
 // next row's state loads are issued before this row's state is stored and its readout reduced,
 // so reads of one row overlap the writes of the previous one.  The row's small q/k/g/v loads are
 // issued at the top of its iteration (prefetching them as well measured 12% slower).
-template <int DK, int DV, int RPT, typename TIO, typename TG>
-__global__ __launch_bounds__(DK * DV / (4 * RPT)) void gla_decode_kernel(DecodeParams a, uint32_t rows) {
+// P: DecodeParams, or Counting<DecodeParams>, where head 0 of each slot of the pool adds one to its token
+// count.  An instance of its own: the pointer among every call's parameters and its test in every row
+// took 4 to 6 % of a step at small rows (32 steps in one graph, B = 1, H = 4, D = 64: 2.77 against 2.67
+// us each; B = 256, H = 6, D = 32: 5.19 against 4.90).
+template <int DK, int DV, int RPT, typename TIO, typename TG, typename P>
+__global__ __launch_bounds__(DK * DV / (4 * RPT)) void gla_decode_kernel(P a, uint32_t rows) {
+    constexpr bool COUNT = !std::is_same<P, DecodeParams>::value;
     constexpr int TPB = DK * DV / (4 * RPT);  // threads per block
     constexpr int CG = DV / 4;                // column groups (float4 columns)
     constexpr int WAVES = TPB / 64;
@@ -112,7 +117,9 @@ __global__ __launch_bounds__(DK * DV / (4 * RPT)) void gla_decode_kernel(DecodeP
 #pragma unroll
             for (int m = 0; m < RPT; ++m) __builtin_nontemporal_store(y[m], reinterpret_cast<f32x4*>(sout + m * DV));
         }
-        if (a.offsets && srow >= 0 && tid == 0 && row % H32 == 0) count_token(a.offsets, srow, a.H);
+        if constexpr (COUNT) {
+            if (srow >= 0 && tid == 0 && row % H32 == 0) count_token(a.offsets, srow, a.H);
+        }
         // reduce over the row groups of a wave (lanes tid ^ CG*2^k share a column group) ...
 #pragma unroll
         for (int c = 0; c < 4; ++c) o4[c] = xor_group_sum<CG>(o4[c]);
@@ -131,34 +138,32 @@ __global__ __launch_bounds__(DK * DV / (4 * RPT)) void gla_decode_kernel(DecodeP
     }
 }
 
-template <int DK, int DV, typename TIO, typename TG>
-static hipError_t launch_decode_t(const DecodeParams& a, int max_blocks, hipStream_t stream) {
+template <int DK, int DV, typename TIO, typename TG, typename P>
+static hipError_t launch_decode_t(const P& a, int max_blocks, hipStream_t stream) {
     constexpr int RPT = (DK * DV / (4 * 256)) > 4 ? (DK * DV / (4 * 256)) : 4;
     constexpr int TPB = DK * DV / (4 * RPT);
     const uint32_t rows = (uint32_t)(a.B * a.H);
     const uint32_t blocks = rows < (uint32_t)max_blocks ? rows : (uint32_t)max_blocks;
-    hipLaunchKernelGGL((gla_decode_kernel<DK, DV, RPT, TIO, TG>), dim3(blocks), dim3(TPB), 0, stream, a, rows);
+    hipLaunchKernelGGL((gla_decode_kernel<DK, DV, RPT, TIO, TG, P>), dim3(blocks), dim3(TPB), 0, stream, a, rows);
     return hipGetLastError();
 }
 
-template <int DK, int DV, typename TIO>
-static hipError_t launch_decode_g(const DecodeParams& a, int mb, hipStream_t stream) {
+template <int DK, int DV, typename TIO, typename P>
+static hipError_t launch_decode_g(const P& a, int mb, hipStream_t stream) {
     if (a.g_dt == DT_F32) return launch_decode_t<DK, DV, TIO, float>(a, mb, stream);
     if (a.g_dt == DT_BF16) return launch_decode_t<DK, DV, TIO, __bf16>(a, mb, stream);
     return launch_decode_t<DK, DV, TIO, _Float16>(a, mb, stream);
 }
 
-template <int DK, int DV>
-static hipError_t launch_decode_io(const DecodeParams& a, int mb, hipStream_t stream) {
+template <int DK, int DV, typename P>
+static hipError_t launch_decode_io(const P& a, int mb, hipStream_t stream) {
     if (a.io_dt == DT_F32) return launch_decode_g<DK, DV, float>(a, mb, stream);
     if (a.io_dt == DT_BF16) return launch_decode_g<DK, DV, __bf16>(a, mb, stream);
     return launch_decode_g<DK, DV, _Float16>(a, mb, stream);
 }
 
-// Supported (Dk, Dv): (32,32), (64,64), (128,128), (64,128), (128,64).  Returns
-// hipErrorInvalidValue for other shapes.  max_blocks caps the grid (blocks then walk several
-// rows); four blocks per CU measured best for the 16 KB rows of (64, 64).
-hipError_t launch_gla_decode(const DecodeParams& a, int Dk, int Dv, int max_blocks, hipStream_t stream) {
+template <typename P>
+static hipError_t launch_decode(const P& a, int Dk, int Dv, int max_blocks, hipStream_t stream) {
     const int mb = max_blocks > 0 ? max_blocks : 1;
     if (Dk == 64 && Dv == 64) return launch_decode_io<64, 64>(a, mb, stream);
     if (Dk == 128 && Dv == 128) return launch_decode_io<128, 128>(a, mb, stream);
@@ -166,6 +171,16 @@ hipError_t launch_gla_decode(const DecodeParams& a, int Dk, int Dv, int max_bloc
     if (Dk == 64 && Dv == 128) return launch_decode_io<64, 128>(a, mb, stream);
     if (Dk == 128 && Dv == 64) return launch_decode_io<128, 64>(a, mb, stream);
     return hipErrorInvalidValue;
+}
+
+// Supported (Dk, Dv): (32,32), (64,64), (128,128), (64,128), (128,64).  Returns
+// hipErrorInvalidValue for other shapes.  max_blocks caps the grid (blocks then walk several
+// rows); four blocks per CU measured best for the 16 KB rows of (64, 64).  offsets: the pool's token
+// counts or null.
+hipError_t launch_gla_decode(const DecodeParams& a, int64_t* offsets, int Dk, int Dv, int max_blocks,
+                             hipStream_t stream) {
+    if (offsets) return launch_decode(Counting<DecodeParams>(a, offsets), Dk, Dv, max_blocks, stream);
+    return launch_decode(a, Dk, Dv, max_blocks, stream);
 }
 
 }  // namespace triune

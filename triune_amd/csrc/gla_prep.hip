@@ -138,8 +138,11 @@ struct FusedDecodeTiling {
     static constexpr int EPL = HD / 64 > 0 ? HD / 64 : 1;  // norm elements per lane
 };
 
-template <int HD, typename TIO, typename TCS, typename TS>
-__global__ __launch_bounds__(FusedDecodeTiling<HD>::TPB) void gla_fused_decode_kernel(FusedDecodeParams a, uint32_t rows) {
+// P: FusedDecodeParams, or Counting<FusedDecodeParams>, where head 0 of each slot of the pool adds one to
+// its token count.
+template <int HD, typename TIO, typename TCS, typename TS, typename P>
+__global__ __launch_bounds__(FusedDecodeTiling<HD>::TPB) void gla_fused_decode_kernel(P a, uint32_t rows) {
+    constexpr bool COUNT = !std::is_same<P, FusedDecodeParams>::value;
     using Tl = FusedDecodeTiling<HD>;
     constexpr int RPT = Tl::RPT, CG = Tl::CG, WAVES = Tl::WAVES, EPL = Tl::EPL;
     constexpr int SB = (int)sizeof(TS);
@@ -355,7 +358,9 @@ __global__ __launch_bounds__(FusedDecodeTiling<HD>::TPB) void gla_fused_decode_k
                 __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), ro, voff + m * HD * SB, 0, 2);
             }
         }
-        if (a.offsets && h == 0 && sr >= 0 && tid == 0) count_token(a.offsets, sr, a.H);
+        if constexpr (COUNT) {
+            if (h == 0 && sr >= 0 && tid == 0) count_token(a.offsets, sr, a.H);
+        }
 #pragma unroll
         for (int c = 0; c < 4; ++c) o4[c] = xor_group_sum<CG>(o4[c]);
         if (lane < CG) red[buf][wave][cg] = f32x4{o4[0], o4[1], o4[2], o4[3]};
@@ -422,40 +427,46 @@ hipError_t launch_gla_prep(const PrepParams& a, int HD, int io_dt, int cs_dt, hi
     return launch_prep_cs<_Float16>(a, HD, cs_dt, stream);
 }
 
-template <int HD, typename TIO, typename TCS, typename TS>
-static hipError_t launch_fdec_t(const FusedDecodeParams& a, hipStream_t stream) {
+template <int HD, typename TIO, typename TCS, typename TS, typename P>
+static hipError_t launch_fdec_t(const P& a, hipStream_t stream) {
     const uint32_t rows = (uint32_t)(a.B * a.H);
     const uint32_t blocks = rows < (uint32_t)a.max_blocks ? rows : (uint32_t)a.max_blocks;
-    hipLaunchKernelGGL((gla_fused_decode_kernel<HD, TIO, TCS, TS>), dim3(blocks), dim3(FusedDecodeTiling<HD>::TPB), 0,
-                       stream, a, rows);
+    hipLaunchKernelGGL((gla_fused_decode_kernel<HD, TIO, TCS, TS, P>), dim3(blocks), dim3(FusedDecodeTiling<HD>::TPB),
+                       0, stream, a, rows);
     return hipGetLastError();
 }
 
-template <int HD, typename TIO, typename TCS>
-static hipError_t launch_fdec_s(const FusedDecodeParams& a, int s_dt, hipStream_t stream) {
+template <int HD, typename TIO, typename TCS, typename P>
+static hipError_t launch_fdec_s(const P& a, int s_dt, hipStream_t stream) {
     if (s_dt == DT_F32) return launch_fdec_t<HD, TIO, TCS, float>(a, stream);
     return launch_fdec_t<HD, TIO, TCS, TIO>(a, stream);  // state in the I/O type (checked by the caller)
 }
 
-template <int HD, typename TIO>
-static hipError_t launch_fdec_cs(const FusedDecodeParams& a, int cs_dt, int s_dt, hipStream_t stream) {
+template <int HD, typename TIO, typename P>
+static hipError_t launch_fdec_cs(const P& a, int cs_dt, int s_dt, hipStream_t stream) {
     if (cs_dt == DT_F32) return launch_fdec_s<HD, TIO, float>(a, s_dt, stream);
     return launch_fdec_s<HD, TIO, TIO>(a, s_dt, stream);  // tables in the I/O type (checked by the caller)
 }
 
-template <typename TIO>
-static hipError_t launch_fdec_hd(const FusedDecodeParams& a, int HD, int cs_dt, int s_dt, hipStream_t stream) {
+template <typename TIO, typename P>
+static hipError_t launch_fdec_hd(const P& a, int HD, int cs_dt, int s_dt, hipStream_t stream) {
     if (HD == 64) return launch_fdec_cs<64, TIO>(a, cs_dt, s_dt, stream);
     if (HD == 128) return launch_fdec_cs<128, TIO>(a, cs_dt, s_dt, stream);
     return launch_fdec_cs<32, TIO>(a, cs_dt, s_dt, stream);
 }
 
-hipError_t launch_gla_fused_decode(const FusedDecodeParams& a, int HD, int io_dt, int cs_dt, int s_dt,
-                                   hipStream_t stream) {
+template <typename P>
+static hipError_t launch_fdec(const P& a, int HD, int io_dt, int cs_dt, int s_dt, hipStream_t stream) {
     if (HD != 32 && HD != 64 && HD != 128) return hipErrorInvalidValue;
     if (io_dt == DT_F32) return launch_fdec_hd<float>(a, HD, cs_dt, s_dt, stream);
     if (io_dt == DT_BF16) return launch_fdec_hd<__bf16>(a, HD, cs_dt, s_dt, stream);
     return launch_fdec_hd<_Float16>(a, HD, cs_dt, s_dt, stream);
+}
+
+hipError_t launch_gla_fused_decode(const FusedDecodeParams& a, int64_t* offsets, int HD, int io_dt, int cs_dt, int s_dt,
+                                   hipStream_t stream) {
+    if (offsets) return launch_fdec(Counting<FusedDecodeParams>(a, offsets), HD, io_dt, cs_dt, s_dt, stream);
+    return launch_fdec(a, HD, io_dt, cs_dt, s_dt, stream);
 }
 
 }  // namespace triune

@@ -118,7 +118,6 @@ struct DecodeParams {
     float* state_out;       // may equal state_in
     const int32_t* slots;   // optional: state row of batch b is slots[b] (state pool), or null
     int64_t n_state_rows;   // rows of state_in / state_out; a slot outside [0, n_state_rows) is skipped
-    int64_t* offsets;       // optional, with slots: offsets[slots[b]] += 1 for slots of the pool
     void* o;
     int64_t B, H;
 };
@@ -215,7 +214,6 @@ struct FusedDecodeParams {
     // state_out; a slot outside [0, n_state_rows) reads no state, stores none and outputs zeros.
     const int32_t* slots;
     int64_t n_state_rows;
-    int64_t* offsets;  // optional, with slots: offsets[slots[b]] += 1 for slots of the pool
 };
 
 // Control block of the single-launch prefill (gla_onepass.hip): hdr[0] epoch, hdr[1] workgroups of
@@ -231,6 +229,12 @@ struct OnePassCtl {
     int64_t nh8;    // (sequence, head) pairs per XCD: ceil(B * H / 8)
 };
 
+// Parameters of a decode step that counts tokens: offsets[slots[b]] += 1 for slots of the pool.
+template <typename P>
+struct Counting : P {
+    int64_t* offsets;
+    Counting(const P& p, int64_t* o) : P(p), offsets(o) {}
+};
 // Head 0 of a decode step counts its session's token: srow = slot * H.
 __device__ __forceinline__ void count_token(int64_t* offsets, int64_t srow, int64_t H) {
     __hip_atomic_fetch_add(reinterpret_cast<unsigned long long*>(offsets) + srow / H, 1ull, __ATOMIC_RELAXED,
@@ -243,9 +247,9 @@ bool gla_bwd_supported(int D, int io_dt);
 hipError_t launch_gla_bwd_state(const BwdParams& a, int64_t n_work, int io_dt, hipStream_t stream);
 hipError_t launch_gla_bwd_chunk(const BwdParams& a, int64_t n_work, int io_dt, hipStream_t stream);
 hipError_t launch_gla_prep(const PrepParams& a, int HD, int io_dt, int cs_dt, hipStream_t stream);
-hipError_t launch_gla_fused_decode(const FusedDecodeParams& a, int HD, int io_dt, int cs_dt, int s_dt,
+hipError_t launch_gla_fused_decode(const FusedDecodeParams& a, int64_t* offsets, int HD, int io_dt, int cs_dt, int s_dt,
                                    hipStream_t stream);
-hipError_t launch_gla_decode(const DecodeParams& a, int Dk, int Dv, int max_blocks, hipStream_t stream);
+hipError_t launch_gla_decode(const DecodeParams& a, int64_t* offsets, int Dk, int Dv, int max_blocks, hipStream_t stream);
 hipError_t launch_gdn_tokenwise(const GdnParams& a, int Dk, int Dv, hipStream_t stream);
 // T == 1 of many rows (Dk = Dv = D in {64, 128}; q, k, g, v rows and beta vector-aligned, beta fp32)
 hipError_t launch_gdn_decode(const GdnParams& a, int D, int max_blocks, hipStream_t stream);
