@@ -58,7 +58,7 @@
 extern "C" {
 #endif
 
-#define TRIUNE_HIP_ABI_VERSION 3
+#define TRIUNE_HIP_ABI_VERSION 4
 
 enum {
     TRIUNE_DT_F32 = 0,
@@ -269,13 +269,15 @@ int triune_hip_gla_prefill_bwd(const void* q, const void* k, const void* v, cons
                                size_t workspace_bytes, void* stream);
 /* The same with the forward's segment states at hand: fwd_workspace is the workspace that
  * triune_hip_gla_prefill used for these inputs (same q, k, v, g, s0, shapes and flags; not written
- * here), or NULL to recompute them (two launches). */
+ * here) and fwd_workspace_bytes its size, at least triune_hip_gla_prefill_workspace_size(B, T, H, Dk,
+ * Dv, flags) (TRIUNE_ERR_WORKSPACE otherwise), or NULL to recompute them (two launches).  A workspace
+ * of another plan, or triune_hip_gla_prefill_noalloc's, will not do. */
 int triune_hip_gla_prefill_bwd_after(const void* q, const void* k, const void* v, const void* g, int io_dtype,
                                      int g_dtype, const void* dout, const int64_t* strides, const float* s0,
                                      const float* ds_final, void* dq, void* dk, void* dv, int d_dtype, void* dg,
                                      int dg_dtype, float* ds0, int64_t B, int64_t T, int64_t H, int Dk, int Dv,
-                                     int flags, const void* fwd_workspace, void* workspace, size_t workspace_bytes,
-                                     void* stream);
+                                     int flags, const void* fwd_workspace, size_t fwd_workspace_bytes, void* workspace,
+                                     size_t workspace_bytes, void* stream);
 
 /* triune_hip_gla_prefill_varlen over a device-resident state pool: sequence i starts from
  * pool[slots[i]] and its final state is written back to pool[slots[i]] (in place).  pool: fp32

@@ -278,6 +278,26 @@ def test_gdn_bwd_validation():
     assert lib.triune_hip_gdn_bwd_workspace_size(4, 8192, 6, 48, 48, 0) == 0
 
 
+def test_gla_bwd_after_checks_the_forward_workspace():
+    """The forward's workspace comes with its size: one of another plan is refused, not read past."""
+    lib = L.lib()
+    f = lib.triune_hip_gla_prefill_bwd_after
+    st = (ctypes.c_int64 * 27)(*([64 * 128 * 64, 64 * 128, 128] * 9))
+    need = int(lib.triune_hip_gla_prefill_workspace_size(1, 4096, 1, 64, 64, 0))
+    assert int(lib.triune_hip_gla_prefill_workspace_size(1, 4096, 1, 64, 64, 64 << L.FLAG_SEG_SHIFT)) < need
+
+    def call(fws, fws_bytes, ws=_FAKE, ws_bytes=1 << 40):
+        return f(_FAKE, _FAKE, _FAKE, _FAKE, 1, 1, _FAKE, st, None, None, _FAKE, _FAKE, _FAKE, 1, _FAKE, 1, None, 1,
+                 4096, 1, 64, 64, 0, fws, fws_bytes, ws, ws_bytes, None)
+
+    assert call(_FAKE, need - 1) == -5
+    assert call(_FAKE, 0) == -5
+    assert call(ctypes.c_void_p(0x1008), need) == -4
+    assert call(_FAKE, need, ws=ctypes.c_void_p(0x1008)) == -4
+    assert call(_FAKE, need, ws=None) == -5
+    assert call(_FAKE, need, ws_bytes=need) == -5  # the backward's own workspace is larger
+
+
 def test_workspace_sizes():
     lib = L.lib()
     w1 = lib.triune_hip_gla_prefill_workspace_size(4, 16384, 6, 64, 64, 0)

@@ -15,7 +15,7 @@ from pathlib import Path
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "libtriune_hip.so"
-ABI_VERSION = 3
+ABI_VERSION = 4
 
 DT_F32, DT_BF16, DT_F16 = 0, 1, 2
 FLAG_TAIL_UNCLAMPED = 0x1
@@ -97,7 +97,7 @@ def _bind(lib):
         ),
         "triune_hip_gla_prefill_bwd_after": (
             [_vp, _vp, _vp, _vp, _i, _i, _vp, _i64p, _vp, _vp, _vp, _vp, _vp, _i, _vp, _i, _vp,
-             _i64, _i64, _i64, _i, _i, _i, _vp, _vp, _sz, _vp],
+             _i64, _i64, _i64, _i, _i, _i, _vp, _sz, _vp, _sz, _vp],
             _i,
         ),
         "triune_hip_recurrent_scan_bwd": (

@@ -735,7 +735,7 @@ int triune_hip_gla_prefill_bwd(const void* q, const void* k, const void* v, cons
                                int64_t B, int64_t T, int64_t H, int Dk, int Dv, int flags, void* workspace,
                                size_t workspace_bytes, void* stream) {
     return triune_hip_gla_prefill_bwd_after(q, k, v, g, io_dtype, g_dtype, dout, strides, s0, ds_final, dq, dk, dv,
-                                            d_dtype, dg, dg_dtype, ds0, B, T, H, Dk, Dv, flags, nullptr, workspace,
+                                            d_dtype, dg, dg_dtype, ds0, B, T, H, Dk, Dv, flags, nullptr, 0, workspace,
                                             workspace_bytes, stream);
 }
 
@@ -743,8 +743,8 @@ int triune_hip_gla_prefill_bwd_after(const void* q, const void* k, const void* v
                                      int g_dtype, const void* dout, const int64_t* strides, const float* s0,
                                      const float* ds_final, void* dq, void* dk, void* dv, int d_dtype, void* dg,
                                      int dg_dtype, float* ds0, int64_t B, int64_t T, int64_t H, int Dk, int Dv,
-                                     int flags, const void* fwd_workspace, void* workspace, size_t workspace_bytes,
-                                     void* stream) {
+                                     int flags, const void* fwd_workspace, size_t fwd_workspace_bytes, void* workspace,
+                                     size_t workspace_bytes, void* stream) {
     if (!q || !k || !v || !g || !dout || !strides || !dq || !dk || !dv || !dg) return TRIUNE_ERR_NULL;
     if (!dtype_ok(io_dtype) || !dtype_ok(g_dtype) || !dtype_ok(d_dtype) || !dtype_ok(dg_dtype)) return TRIUNE_ERR_DTYPE;
     if (!gate_dtype_ok(io_dtype, g_dtype)) return TRIUNE_ERR_DTYPE;
@@ -781,6 +781,7 @@ int triune_hip_gla_prefill_bwd_after(const void* q, const void* k, const void* v
     }
     const BwdPlan pl = plan_bwd(B, T, H, Dk, flags);
     if (!workspace || workspace_bytes < pl.total) return TRIUNE_ERR_WORKSPACE;
+    if (fwd_workspace && fwd_workspace_bytes < pl.f.total) return TRIUNE_ERR_WORKSPACE;
     char* ws = reinterpret_cast<char*>(workspace);
     if (reinterpret_cast<uintptr_t>(ws) % 16 || reinterpret_cast<uintptr_t>(fwd_workspace) % 16) return TRIUNE_ERR_LAYOUT;
     // the forward's segment states and decays: its own workspace (read only), or recomputed here

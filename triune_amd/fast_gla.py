@@ -312,7 +312,7 @@ def _prefill_bwd(q, k, v, g, s0, do, ds, flags, grad_dtype=None, outs=None, acc=
     rc = L.triune_hip_gla_prefill_bwd_after(
         ptr(qp), ptr(kp), ptr(vp), ptr(gp), dtype_code(qp), dtype_code(gp), ptr(dop), st, ptr(s0p), ptr(dsf),
         ptr(dq), ptr(dk), ptr(dv), dtype_code(dq), ptr(dg), dtype_code(dg), ptr(ds0), B, T, H, D, D, flags | acc,
-        ptr(fwd_ws), ptr(ws), ws.numel(), stream_of(q),
+        ptr(fwd_ws), 0 if fwd_ws is None else fwd_ws.numel(), ptr(ws), ws.numel(), stream_of(q),
     )
     check(rc, "triune_hip_gla_prefill_bwd")
     if outs is not None:
