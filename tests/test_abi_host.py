@@ -278,6 +278,70 @@ def test_gdn_bwd_validation():
     assert lib.triune_hip_gdn_bwd_workspace_size(4, 8192, 6, 48, 48, 0) == 0
 
 
+def test_gdn_bwd_chunked_validation():
+    """The chunk-form Gated DeltaNet backward: 16-bit throughout, beta none or per head with its
+    gradient, rows of D elements that do not overlap (T > 1) and lie within 32-bit reach."""
+    lib = L.lib()
+    f = lib.triune_hip_gdn_bwd_chunked
+    rows = [4 * 64 * 64, 4 * 64, 64]
+
+    def call(io=1, gdt=1, head=0, beta=None, bdt=1, bk=0, db=None, dq=_FAKE, do=_FAKE, T=64, H=1, dk=64, dv=64, st=None,
+             ws=None, wsb=0, s0=None, dsf=None, ds0=None):
+        sts = (ctypes.c_int64 * 18)(*(rows * 6))
+        for i, v in (st or {}).items():
+            sts[i] = v
+        return f(_FAKE, _FAKE, _FAKE, _FAKE, io, gdt, head, beta, bdt, bk, sts, s0, do, dsf, dq, _FAKE, _FAKE, _FAKE, db,
+                 ds0, 1, T, H, dk, dv, ws, wsb, None)
+
+    odd = ctypes.c_void_p(0x1008)
+    assert call() == -5 and call(io=2, gdt=2) == -5  # valid, no workspace
+    assert call(ws=_FAKE, wsb=16) == -5
+    assert call(dq=None) == -1
+    assert call(io=0, gdt=0) == -3  # fp32 I/O stays with triune_hip_gdn_bwd, and so do mixed types
+    assert call(gdt=0) == -3
+    assert call(bk=1, beta=_FAKE, bdt=0, db=_FAKE) == -3
+    assert call(bk=1, beta=_FAKE) == -1  # beta without its gradient buffer
+    assert call(bk=1, beta=_FAKE, db=_FAKE) == -5
+    assert call(bk=2, beta=_FAKE, db=_FAKE) == -2  # beta per key dim
+    assert call(dk=32, dv=32) == -2 and call(dk=128, dv=64) == -2 and call(H=0) == -2
+    for i in (1, 4, 7, 10, 16):  # token strides of q, k, v, g, dO below the row width
+        assert call(st={i: 32}) == -4 and call(st={i: 0}) == -4
+        assert call(st={i: -256}) == -4 and call(st={i: 0x7fffffff // 160 + 1}) == -4
+        assert call(T=1, st={i: 0}) == -5  # one token has no next row
+    assert call(head=1, st={10: 0}) == -5  # one gate for every token
+    assert call(do=None, st={16: 0}) == -5
+    assert call(bk=1, beta=_FAKE, db=_FAKE, st={13: 0}) == -5
+    assert call(H=0x7fffffff // (160 * 64) + 1) == -4  # rows of the outputs out of reach
+    assert call(s0=odd) == -4 and call(dsf=odd) == -4 and call(ds0=odd) == -4 and call(ws=odd, wsb=1 << 40) == -4
+    assert call(T=0) == 0  # nothing to do
+    assert lib.triune_hip_gdn_bwd_chunked_workspace_size(1, 65, 1, 64, 64) == 2 * (3 * 64 * 64 + 20 * 256) * 4
+    assert lib.triune_hip_gdn_bwd_chunked_workspace_size(1, 65, 1, 64, 128) == 0
+
+
+def test_decode_steps_that_count_tokens_validation():
+    """offsets of the counting decode steps: 8-byte aligned, and in the plain step only with slots."""
+    lib = L.lib()
+    odd = ctypes.c_void_p(0x1004)
+    d = lib.triune_hip_gla_decode_step_count
+
+    def plain(slots, offsets, dv=64):
+        return d(_FAKE, _FAKE, _FAKE, _FAKE, 1, 1, _st(10), _FAKE, _FAKE, slots, 1, offsets, _FAKE, 1, 1, 1, 64, dv, None)
+
+    assert plain(None, _FAKE) == -1
+    assert plain(_FAKE, odd) == -4
+    assert plain(_FAKE, _FAKE, dv=32) == -2
+    f = lib.triune_hip_gla_fused_decode_step_slots_count
+    st = (ctypes.c_int64 * 3)(4 * 3 * 64, 3 * 64, 64)
+    ost = (ctypes.c_int64 * 2)(3 * 64, 64)
+
+    def fused(offsets, slots=_FAKE, hd=64):
+        return f(_FAKE, 1, st, None, None, 0, 0, _FAKE, 0, slots, 4, offsets, _FAKE, 1, ost, 2, 3, hd, None)
+
+    assert fused(odd) == -4
+    assert fused(_FAKE, slots=None) == -1
+    assert fused(_FAKE, hd=48) == -2
+
+
 def test_gla_bwd_after_checks_the_forward_workspace():
     """The forward's workspace comes with its size: one of another plan is refused, not read past."""
     lib = L.lib()

@@ -8,6 +8,8 @@ fp32, and a pair factor e^(G - m) e^(m - G') with exponents up to 64 carries up 
 2 * 64 * 2^-24 * (1 + log2 e) = 2e-5 of relative error.
 """
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -178,6 +180,38 @@ def test_gate_gradients_of_steep_gates(dev, D, gate, rate):
     err = (got[3].double().cpu() - r).abs()
     assert bool((err <= _ulp(r, torch.bfloat16) + 1.2e-5 * float(r.abs().max())).all()), float(
         ((err - _ulp(r, torch.bfloat16)) / r.abs().max()).max())
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("T", [0, 1, 64, 150])
+@pytest.mark.parametrize("ds", [True, False])
+def test_entry_with_an_initial_state(dev, D, T, ds):
+    """The entry itself with an initial state and its gradient (fp32: a chain of fp32 products over the
+    chunks, 4e-5 of the largest as for the others), which the Python layer leaves to the other entry."""
+    B, H = 2, 3
+    q, k, v, g, b, do, dsf = _inputs(B, max(T, 1), H, D, "key", True, torch.bfloat16, seed=T + D)
+    q, k, v, g, b, do = (x[:, :T].contiguous().to(dev) for x in (q, k, v, g, b, do))
+    s0 = (0.3 * torch.randn(B, H, D, D, generator=torch.Generator().manual_seed(T))).to(dev)
+    dsf = dsf.to(dev) if ds else None
+    L = _lib.lib()
+    dq, dk, dv, dg, db = (torch.empty_like(x) for x in (q, k, v, g, b))
+    ds0 = torch.empty_like(s0)
+    ws = torch.empty(int(L.triune_hip_gdn_bwd_chunked_workspace_size(B, T, H, D, D)), device=dev, dtype=torch.uint8)
+    st = (ctypes.c_int64 * 18)(*([T * H * D, H * D, D] * 4), T * H, H, 1, T * H * D, H * D, D)
+    # an empty tensor has no address: the entry wants one
+    ptr = [x.data_ptr() or ws.data_ptr() for x in (q, k, v, g, b, do, dq, dk, dv, dg, db)]
+    rc = L.triune_hip_gdn_bwd_chunked(*ptr[:4], 1, 1, 0, ptr[4], 1, _lib.BETA_HEAD, st, s0.data_ptr(), ptr[5],
+                                      dsf.data_ptr() if ds else None, *ptr[6:], ds0.data_ptr(), B, T, H, D, D,
+                                      ws.data_ptr(), ws.numel(), _lib.stream_of(q))
+    _lib.check(rc, "gdn_bwd_chunked")
+    torch.cuda.synchronize()
+    if T == 0:
+        assert torch.equal(ds0, dsf if ds else torch.zeros_like(s0))
+        return
+    ref = O.gdn_bwd(*(x.cpu() for x in (q, k, v, g, b, s0, do)), dsf.cpu() if ds else None)
+    _check((dq, dk, dv, dg, db), ref[:5], torch.bfloat16, NAMES)
+    r = torch.as_tensor(np.asarray(ref[5], dtype=np.float64))
+    assert float((ds0.double().cpu() - r).abs().max()) <= 4e-5 * max(1.0, float(r.abs().max()))
 
 
 @pytest.mark.parametrize("gate", ["key", "head"])
