@@ -1,7 +1,7 @@
 """The prefill's segment plans (rounds of segments, dropped segments, packed segment lengths) against the
 fp64 oracle and the forced plans, at shapes on both sides of each rule: fewer (sequence, head) pairs than
-slots, more than half of them, more than all of them, one chunk, and packed batches whose estimate leaves
-the eight-round length."""
+slots, so many that two rounds of segments pay, more than all of them, one chunk, and packed batches whose
+estimate leaves the eight-round length."""
 
 import numpy as np
 import pytest
@@ -19,8 +19,13 @@ def _err(a, b):
     return float((torch.as_tensor(a).double().cpu() - torch.as_tensor(np.asarray(b))).abs().max())
 
 
-@pytest.mark.parametrize("B,T,H,D", [(1, 64, 1, 64), (3, 3001, 8, 64), (8, 520, 12, 128), (6, 300, 100, 64)])
-def test_dense_plans(dev, B, T, H, D):
+# The last figure: rounds of resident workgroups (two per CU at D = 64, one at D = 128) the plan takes.
+@pytest.mark.parametrize("B,T,H,D,rounds", [(1, 64, 1, 64, 1), (3, 3001, 8, 64, 1), (8, 520, 12, 128, 1),
+                                            (6, 300, 100, 64, 2), (17, 960, 10, 128, 2), (17, 1984, 20, 64, 2)])
+def test_dense_plans(dev, B, T, H, D, rounds):
+    segments = int(_lib.lib().triune_hip_gla_prefill_workspace_size(B, T, H, D, D, 0)) // (B * H * (D * D + D) * 4)
+    slots = torch.cuda.get_device_properties(dev).multi_processor_count * (2 if D == 64 else 1)
+    assert -(-B * H * segments // slots) == rounds and (segments > 1) == (T > 64 and B * H < slots)
     q, k, v, g, s0 = gla_inputs(B, T, H, D, seed=T, dtype=torch.bfloat16, init_std=0.1)
     g = g.float()  # the three-launch form whatever the size
     x = [t.to(dev) for t in (q, k, v, g, s0)]

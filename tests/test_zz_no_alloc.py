@@ -101,3 +101,8 @@ def test_noalloc_takes_calls_whose_several_rounds_exceed_the_scratch(dev):
     check(L.triune_hip_gla_prefill(*head, one, ptr(ws), wsb, st), "prefill")
     torch.cuda.synchronize()
     assert torch.equal(o, o_ref) and torch.equal(s, s_ref)
+    wsb = int(L.triune_hip_gla_prefill_workspace_size(17, 960, 10, 128, 128, 0))  # the three segments
+    ws = torch.empty(wsb, device=dev, dtype=torch.uint8)
+    check(L.triune_hip_gla_prefill(*head, 0, ptr(ws), wsb, st), "prefill")
+    torch.cuda.synchronize()
+    assert float((o - o_ref).abs().max()) <= 2e-3 and float((s - s_ref).abs().max()) <= 2e-3
