@@ -78,18 +78,21 @@ struct Prec {
     static constexpr int NX = F32 ? 3 : (std::is_same<TIn, _Float16>::value ? 2 : 1);  // parts of V
     // Largest chunk decay span (-G_C of a key dim, nats) of the GLA chunk kernels' factored form; chunks
     // past it run token by token.  The factors e^(G - m), e^(m - G) and the e^m that carried states and
-    // gradients are multiplied by before they are split lie in e^[-SPAN_MAX / 2, SPAN_MAX / 2].  A
-    // product's second bf16 part is a normal number while its operand is above 2^-117 e^(SPAN_MAX / 2):
-    // 5e-22 at 64 nats, 1.4e-18 at 80 (4e-8 at 128, where gradients of 1e-10 came out 0.3 % off and those
-    // of 1e-13 as zero).  Gates of logsigmoid(N(0, 1)), the reference model's at initialisation, span
-    // 52 +- 4 nats, 75 at most: with a limit of 64 one chunk in five (4 heads of 64 dims) ran token by
-    // token and held up the whole launch (1024-token tile from raw projections 102 us against 20 us
-    // without such chunks).  64 nats for fp32 I/O, where the exponents' own rounding (about |x| 2^-24)
-    // would otherwise reach the third parts' size, and for fp32 outputs of 16-bit inputs, which show the
-    // parts' 2^-17: a steeper chunk's stay exact to fp32, as they would be token by token.
+    // gradients are multiplied by before they are split lie in e^[-span / 2, span / 2].  A product's second
+    // bf16 part is a normal number while its operand is above 2^-117 e^(span / 2): 5e-22 at 64 nats, 1.4e-18
+    // at 80, 2.3e-13 at 104, 4e-8 at 128.
+    // Gates of logsigmoid(N(0, 1)), the reference model's at initialisation, span 52 +- 4 nats, 75 at most,
+    // and its outputs taken as gates 53 +- 8, 96 at most (16384 tokens, 32 heads).  With a limit of 64 one
+    // chunk in five (4 heads of 64 dims) ran token by token and held up the whole launch: 1024-token tile
+    // from raw projections 97 us against 19.
+    //   forward   104: activations and their states lie far above 2.3e-13
+    //   backward   80: gradients of a mean over many tokens do not (at 128 those of 1e-11 came out 3 % off)
+    //   64 for fp32 I/O, where the exponents' own rounding (about |x| 2^-24) would otherwise reach the third
+    //   parts' size, and for fp32 outputs of 16-bit inputs, which show the parts' 2^-17 that a steeper chunk
+    //   taken token by token does not have
     static constexpr float SPAN_F32 = 64.f;
-    static constexpr float SPAN_MAX = F32 ? SPAN_F32 : 80.f;
-    __device__ __forceinline__ static float span_max(int o_dt) { return o_dt == DT_F32 ? SPAN_F32 : SPAN_MAX; }
+    static constexpr float SPAN_BWD = F32 ? SPAN_F32 : 80.f;
+    __device__ __forceinline__ static float span_fwd(int o_dt) { return F32 || o_dt == DT_F32 ? SPAN_F32 : 104.f; }
 };
 // Log-decay limit of the scalar-gate Gated DeltaNet chunks (gdn_scalar.hip).
 constexpr float GDN_SG_SPAN_MAX = 64.f;

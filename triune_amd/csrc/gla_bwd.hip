@@ -26,7 +26,7 @@
 //   dv = A^T dO + Kt (e^m dH)                   dH <- e^{G_C} dH + e^m (Qt^T dO)
 // and dg from the in-chunk suffix sums of q.dq - k.dk plus the sum carried from the later
 // chunks (started at sum_j dH S over the segment's end state).  Chunks whose decay span exceeds
-// SPAN_MAX, or that hold the reference's unclamped 1-token tail, run token by token.
+// SPAN_BWD, or that hold the reference's unclamped 1-token tail, run token by token.
 //
 // Wave w of a workgroup (NW = D / 16 waves) owns key dims [16w, 16w+16) of dq and dk and value
 // columns [16w, 16w+16) of dv and of the carried dH.  Products run on v_mfma_f32_16x16x32_bf16
@@ -492,7 +492,7 @@ struct BwdStep {
             chunk_cumsum<DL>(G, GC, lane);
             bool bad = tail_chunk;
 #pragma unroll
-            for (int i = 0; i < DL; ++i) bad |= !(GC[i] >= -Prec<TIn>::SPAN_MAX);
+            for (int i = 0; i < DL; ++i) bad |= !(GC[i] >= -Prec<TIn>::SPAN_BWD);
 #pragma unroll
             for (int j = 0; j < 4; ++j)
 #pragma unroll

@@ -282,7 +282,7 @@ __global__ __launch_bounds__(OP_THREADS, 1) void gla_onepass_kernel(PrefillParam
     {
         bool bad = tail_unclamped;
 #pragma unroll
-        for (int i = 0; i < DL; ++i) bad |= !(GC[i] >= -Prec<TIn>::span_max(a.o_dt));
+        for (int i = 0; i < DL; ++i) bad |= !(GC[i] >= -Prec<TIn>::span_fwd(a.o_dt));
         const bool any_bad = __any(bad);
         if (lane == 0) sFLAG[wave] = any_bad ? 1 : 0;
         if (tg == 0) {

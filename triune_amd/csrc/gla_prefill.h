@@ -32,7 +32,7 @@
 //            transposed LDS read
 // The next chunk's inputs are loaded while the current chunk is processed: into registers, or
 // (2-byte inputs at 64 x 64) q, k, g / k, g, v straight into LDS tiles of whole 128-byte rows.
-// Chunks whose key-dim decay span exceeds SPAN_MAX (or that hold the reference's unclamped
+// Chunks whose key-dim decay span exceeds span_fwd (or that hold the reference's unclamped
 // 1-token tail) run token by token on the same state registers.
 #pragma once
 
@@ -367,7 +367,7 @@ struct OutStep {
             chunk_cumsum<DL>(G, GC, lane);
             bool bad = tail_unclamped;
 #pragma unroll
-            for (int i = 0; i < DL; ++i) bad |= !(GC[i] >= -Prec<TIn>::span_max(oc.dt));
+            for (int i = 0; i < DL; ++i) bad |= !(GC[i] >= -Prec<TIn>::span_fwd(oc.dt));
             float mh[DL];  // -m log2(e), m = GC / 2
 #pragma unroll
             for (int i = 0; i < DL; ++i) mh[i] = -0.5f * LOG2E * GC[i];
