@@ -591,7 +591,7 @@ def bench_gdn_bwd(dev, reps=3):
     return {"workload": "Gated DeltaNet backward, config 3 (B=4, H=6, T=8192, D=64, bf16, per-head beta)",
             "ms": round(ms, 3), "tok_s": round(B * T / (ms * 1e-3), 1), "alg_bytes": alg,
             "kernels": "gdn_bwd_map + gdn_bwd_scan + gdn_bwd_grad (chunk form: per-chunk maps, one scan, per-chunk gradients)",
-            "roofline": {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS,
+            "roofline": {"bound": "fp32 mfma", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS,
                          "unit": "GB/s", "frac": round(gbs / HBM_PEAK_GBS, 4)}}
 
 
@@ -619,7 +619,7 @@ def bench_gdn_bwd128(dev, reps=3):
     return {"workload": "Gated DeltaNet backward at head dim 128 (B=4, H=12, T=8192, D=128, bf16, "
                         "per-key-dim logsigmoid gate, no beta)",
             "ms": round(ms, 3), "tok_s": round(B * T / (ms * 1e-3), 1), "alg_bytes": alg,
-            "roofline": {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS,
+            "roofline": {"bound": "fp32 mfma", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS,
                          "unit": "GB/s", "frac": round(gbs / HBM_PEAK_GBS, 4)}}
 
 

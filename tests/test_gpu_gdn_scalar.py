@@ -86,7 +86,7 @@ def test_scalar_gdn_positive_gates_clamped(dev):
 
 
 def test_scalar_gdn_tokenwise_chunks(dev):
-    """Chunks whose total log-decay is below -SPAN_MAX, or that hold a -inf gate (a state reset),
+    """Chunks whose total log-decay is below -GDN_SG_SPAN_MAX, or that hold a -inf gate (a state reset),
     run token by token inside the chunked kernels; the other chunks stay on the MFMA path."""
     q, k, v, la, beta, s0 = _case(2, 320, 2, 64, "head", seed=11)
     la = la.clone()

@@ -29,31 +29,31 @@
 // Products run on v_mfma_f32_16x16x4_f32: its operands are fp32 as they come out of the accumulators
 // (nothing is rounded on the way), and a tile held in accumulator layout (lane 16 g4 + r16: rows
 // 4 g4 + r of column r16) is a B operand as it stands when product r contracts rows 4 g4 + r.  With
-// two bf16 parts per operand on v_mfma_f32_16x16x32_bf16 the kernels were a fifth faster (403 against
+// two bf16 parts per operand on v_mfma_f32_16x16x32_bf16 they were a fifth to a third faster (403 against
 // 480 us at D = 64, 520 against 730 at D = 128, the shapes below) but carried 2^-17 into dg, which is
-// a difference of sums: against 64 bits its error rose from the token-serial kernels' 2.08e-4 to
-// 2.14e-4 (fp16, B = 2, T = 600, H = 4, D = 64, gate per key dim) and elements below 1 % of its rms
+// a difference of sums: against 64 bits its error rose from the token-serial kernels' 2.087e-4 to
+// 2.141e-4 (fp16, B = 2, T = 600, H = 4, D = 64, gate per key dim) and elements below 1 % of its rms
 // lost up to eight bits (at 1e-3 to 1e-2 of it 1.6e-4 -> 4.4e-3 of their value).  In fp32 those are
-// 2.08e-4 and 1.9e-4.  Solves with I + L are block substitutions with the inverses of the four diagonal
+// 2.087e-4 and 1.9e-4.  Solves with I + L are block substitutions with the inverses of the four diagonal
 // blocks; dependent products issue back to back (32 cycles each), so the substitutions cost no more
 // than products with an explicit inverse would.
 //
 // Measured, backward alone (bf16): B=4, H=6, T=8192, D=64, gate and beta per head 2884 us on the
 // token-serial kernels, 480 here (map 165, scan 90, gradients 258); B=4, H=12, T=2048, D=128, gate per
-// key dim 5834 and 729 (232, 229, 332).  The map and gradient kernels are bound by the fp32 MFMA and by
-// the chain of a chunk beside it (416 and 680 products of 32 cycles per wave and chunk at D = 64: 67
-// and 109 us of the times above on two workgroups per CU, a third of each kernel at one per CU for
-// D = 128); the scan by the traffic of M, N, K, S and D (20 D^2 bytes per chunk: 2.8 TB/s at D = 64)
-// and the latency of its steps.
+// key dim 5834 and 727 (232, 229, 332).  The map and gradient kernels are bound by the fp32 matrix pipe
+// and the chain of a chunk between its products: by counters the pipe is busy 58 and 49 % of the cycles
+// at D = 64 (two workgroups per CU), 62 and 55 % at D = 128 (one), HBM moves 254 and 319 MB (1.5 and 1.2
+// TB/s) and LDS is active in 15-20 %.  The scan is bound by the latency of its steps: pipe 41-42 %, 188
+// and 371 MB (2.1 and 1.6 TB/s).
 //
 // A chunk in which some key dim decays by more than GB_SPAN nats takes its pair sums ([.], L and A) in
 // two levels.  Between two 16-token tiles the decay from s to t is the rest of s's tile, the tiles
 // between and t's tile up to t, all factors of at most 1.  Within a tile whose dims decay by at most
 // GB_TILE the factors are e^(sum up to t) and e^-(sum up to s); a steeper tile (a reset, -inf) takes
 // running products of its decays token by token.  The products with S and D use factors of at most 1
-// everywhere.  With gates three times as steep, all chunks past GB_SPAN: B=4, H=12, T=8192, D=64 1010 us
-// (ordinary gates 920, token-serial kernels 5036, all pair sums token by token 4320), T=1000 155 (125,
-// 694, 674), B=1, H=4, T=200 50 (45, 123, 297); every tile past GB_TILE (B=4, H=6, T=8192) 770 (2881
+// everywhere.  With gates three times as steep, all chunks past GB_SPAN: B=4, H=12, T=8192, D=64 1019 us
+// (ordinary gates 901, token-serial kernels 5036, all pair sums token by token 4320), T=1000 154 (122,
+// 694, 674), B=1, H=4, T=200 50 (44, 123, 297); every tile past GB_TILE (B=4, H=6, T=8192) 771 (2881
 // token-serial).
 #include "chunk_common.h"
 

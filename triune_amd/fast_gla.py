@@ -372,9 +372,13 @@ class _ChunkGLA(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, v, g, initial_state, flags):
-        # The segment states stay for the backward (16 KB per segment and head at D = 64, 8 MB for
-        # 512 segment-heads: recomputing them took 16 of its 98 us there); heads wider than the
-        # gradient kernels hold run in blocks, which recompute theirs.
+        # The segment states stay for the backward (recomputing them took 16 of its 98 us at 512
+        # segment-heads, D = 64); heads wider than the gradient kernels hold run in blocks, which
+        # recompute theirs.  Held with the graph per call: 16 KB per segment and head at D = 64, against
+        # 32 KB and more of 16-bit q, k, v, g in a segment; measured 8.1 MiB beside 32 of inputs and 16.5
+        # of outputs at B = 8, T = 2048, H = 4, and 8.0 beside 192 at B = 4, T = 16384, H = 6.  A plan of
+        # several rounds of workgroups holds as many times 8 MiB (16.2 at B = 17, H = 20).  It is a saved
+        # tensor like the inputs: torch.autograd.graph's hooks move it off the device with them.
         keep = []
         o, s = _prefill(q, k, v, g, initial_state, None, flags, keep=keep)
         whole = max(q.shape[-1], v.shape[-1]) <= (32 if q.dtype == torch.float32 else 64)
@@ -868,7 +872,8 @@ def fast_recurrent_gated_deltanet(q, k, v, g, beta=None, initial_state=None, *, 
     beta None, [B, T, H] or [B, T, H, D]; a 4-D beta scales rows (key dim), as this reference
     function does.  out_dtype: dtype of the output (default v.dtype; float32 keeps the fp32
     accumulators unrounded).  Differentiable in q, k, v, g, beta and initial_state, as the
-    reference's autograd through this loop (backward: triune_hip_gdn_bwd).  Returns (out,
+    reference's autograd through this loop (backward: triune_hip_gdn_bwd_chunked where everything is
+    16-bit, beta none or [B, T, H] and no initial state given, else triune_hip_gdn_bwd).  Returns (out,
     final_state fp32)."""
     return _gdn(q, k, v, g, beta, initial_state, _beta_kind(beta, "key"), out_dtype)
 
@@ -878,8 +883,8 @@ def fast_chunk_gated_deltanet(q, k, v, g, beta=None, initial_state=None, chunk_s
     A 4-D beta scales columns (value dim) as the reference's GPU kernel does for T > 1
     (fast_gla.py:464-465), and rows at T == 1 (fast_gla.py:880) and whenever a gradient is needed
     (the reference then runs its PyTorch recurrence, fast_gla.py:885-904, which scales rows).
-    Differentiable in q, k, v, g, beta and initial_state (backward: triune_hip_gdn_bwd).
-    chunk_size is accepted for signature parity.  out_dtype as for
+    Differentiable in q, k, v, g, beta and initial_state (backward as for
+    fast_recurrent_gated_deltanet's).  chunk_size is accepted for signature parity.  out_dtype as for
     fast_recurrent_gated_deltanet.  Returns (out, final_state fp32)."""
     T = q.shape[1]
     grad = _needs_grad(q, k, v, g, beta, initial_state)
