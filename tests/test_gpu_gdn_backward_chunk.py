@@ -214,6 +214,28 @@ def test_entry_with_an_initial_state(dev, D, T, ds):
     assert float((ds0.double().cpu() - r).abs().max()) <= 4e-5 * max(1.0, float(r.abs().max()))
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("steep", [1.0, 12.0])
+def test_captured_backward_replays(dev, D, steep):
+    """The backward captured in a graph gives the eager call's bits on every replay, with eager work in
+    between and new inputs in the captured buffers."""
+    q, k, v, g, b, do, ds = (x.to(dev) for x in _inputs(2, 200, 2, D, "key", True, torch.bfloat16, seed=D, steep=steep,
+                                                        resets=steep > 1))
+    kind = _lib.BETA_HEAD
+    call = lambda: FG._gdn_bwd(q, k, v, g, b, None, kind, do, ds)  # noqa: E731
+    call()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call()
+    for n in range(3):
+        do.copy_(torch.randn(do.shape, generator=torch.Generator().manual_seed(n)))
+        graph.replay()
+        torch.cuda.synchronize()
+        got = [x.clone() for x in out[:5]]
+        for x, y in zip(got, call()[:5]):
+            assert torch.equal(x, y)
+
+
 @pytest.mark.parametrize("gate", ["key", "head"])
 def test_operator_views_and_padding(dev, gate, monkeypatch):
     """The operator's autograd with strided q, k, v views, a non-contiguous beta and gate, and head
